@@ -79,6 +79,7 @@ struct bsattn_cache {
   int32_t* idx_ws = nullptr;  // [rows][hkv][nsel_max]
   float* partials = nullptr;  // [rows][hq][nsplit][D + 2]
   float* err_ws = nullptr;    // [rows][hkv][2][mfma_err_stride]: MFMA score bounds, chunk floors
+  float* prefill_ws = nullptr;  // split prefill partials (allocated by the first call that splits)
   std::vector<int32_t> len;
   // set by bsattn_append_step: the device-side lengths may be ahead of `len`
   // until bsattn_sync
@@ -397,6 +398,7 @@ int bsattn_cache_destroy(bsattn_cache* c) try {
   (void)hipFree(c->idx_ws);
   (void)hipFree(c->partials);
   (void)hipFree(c->err_ws);
+  (void)hipFree(c->prefill_ws);
   delete c;
   return BSATTN_OK;
 } catch (...) {
@@ -927,6 +929,24 @@ int bsattn_decode_multi(bsattn_cache* c, const void* q, const int32_t* seq_ids, 
   return on_exception();
 }
 
+// The split prefill's workspace, or null when it cannot be had (the call then
+// runs unsplit).  Allocated once per cache and kept until it is destroyed (a
+// captured graph may hold its address); the relaxed capture mode keeps the
+// allocation from invalidating a capture that is under way on any thread.
+static float* prefill_workspace(bsattn_cache* c) {
+  if (c->prefill_ws) return c->prefill_ws;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+  float* p = nullptr;
+  const hipError_t e = hipMalloc((void**)&p, (size_t)kPrefillRows * (kHeadDim + 2) * sizeof(float));
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return c->prefill_ws = p;
+}
+
 int bsattn_prefill(bsattn_cache* c, const void* q, const int32_t* seq_ids, int32_t n_seqs,
                    int32_t n_query, float scale, void* out, void* stream) try {
   if (!c || !q || !out) return fail(BSATTN_ERR_INVALID, "null argument");
@@ -950,15 +970,20 @@ int bsattn_prefill(bsattn_cache* c, const void* q, const int32_t* seq_ids, int32
     SeqBatch b{};
     b.n = std::min(step, n - i0);
     b.qhs = n_query * kHeadDim;
+    int tokens = 0;
     for (int i = 0; i < b.n; ++i) {
       b.ids[i] = seqs[i0 + i];
       b.len[i] = -1;
       b.qoff[i] = (int32_t)(i * per_seq);
+      tokens = std::max(tokens, c->len[seqs[i0 + i]]);
     }
+    int nsplit = prefill_splits(c->geo, b.n, n_query, tokens);
+    float* ws = nsplit > 1 ? prefill_workspace(c) : nullptr;
+    if (!ws) nsplit = 1;
     Timing tm[kProfKinds];
     Timing* prof = prof_slots(c, s, tm);
-    hipError_t e = launch_prefill(c->geo, b, n_query, (const uint16_t*)q + i0 * per_seq, scale,
-                                  (uint16_t*)out + i0 * per_seq, s, prof);
+    hipError_t e = launch_prefill(c->geo, b, n_query, nsplit, (const uint16_t*)q + i0 * per_seq, scale,
+                                  (uint16_t*)out + i0 * per_seq, ws, s, prof);
     prof_collect(c, prof);
     if (e != hipSuccess) return hip_fail(e, "prefill launch");
   }

@@ -25,6 +25,8 @@ constexpr int kWavesWide = 9;
 constexpr int kMaxSplits = 512;       // attention splits per (sequence, kv head)
 // device scratch of the no-allocation decode (bsattn_noalloc.hip), per GPU
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
+// rows of prefill partials (query rows times parts) a cache's workspace holds
+constexpr int64_t kPrefillRows = 131072;
 // floats after the last block-score row: the workgroup selection reads a
 // thread's candidates as whole vectors, up to 12 x 1024 entries from a row
 // start, and the entries past the row are never candidates
@@ -207,9 +209,14 @@ hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, cons
                                       const PatchBatch& pb, const void* k, const void* v, const void* q,
                                       int32_t* idx_out, float scale, void* out, float* partials,
                                       hipStream_t s, Timing* prof);
-// dense causal attention of the last L tokens of each sequence
-hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, const void* q, float scale,
-                          void* out, hipStream_t s, Timing* prof);
+// dense causal attention of the last L tokens of each sequence.  nsplit > 1:
+// every query's tokens are split into that many parts, whose partials (ws:
+// nsplit * n * hq * L rows of kHeadDim + 2 floats, at most kPrefillRows rows)
+// a second launch merges.
+hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, int nsplit, const void* q, float scale,
+                          void* out, float* ws, hipStream_t s, Timing* prof);
+// parts for a launch of n sequences of up to `tokens` tokens
+int prefill_splits(const Geometry& g, int n, int L, int tokens);
 hipError_t launch_export(const Geometry& g, const SeqBatch& b, int T, void* k_out,
                          void* v_out, hipStream_t s);
 hipError_t launch_export_quantized(const Geometry& g, const SeqBatch& b, int T,

@@ -1,6 +1,5 @@
 // bsattn_prefill.hip -- gfx950 (CDNA4) dense causal attention of a prefill
-// chunk over a 16-bit block-sparse cache (the quantized caches' version is
-// in bsattn_quant.hip).
+// chunk over a block-sparse cache (16-bit or affine-quantized).
 //
 // Built with -fno-honor-nans -mno-amdgpu-ieee: the scores are MFMA results
 // (never signalling NaNs), so max trees compile to v_max3_f32 without the
@@ -8,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 // (the shared header's NaN-aware helpers are not used here)
@@ -18,447 +18,541 @@
 
 namespace bsattn {
 
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int DT>
+__device__ __forceinline__ f32x16 mfma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
+  if constexpr (DT == 0)
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+// a workgroup barrier that orders LDS only: the global loads of later units
+// stay in flight across it
+__device__ __forceinline__ void unit_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// x of the lane 32 places away (the other half of a column's tokens)
+__device__ __forceinline__ float pair_max(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+}
+__device__ __forceinline__ float pair_sum(float x) {
+  const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(a[0]) + __uint_as_float(a[1]);
+}
+
+constexpr int kPfWaves = 8;           // waves per workgroup
+constexpr int kPfCols = 32;           // MFMA columns per wave
+constexpr int kPfSplits = 16;         // most parts a tile's tokens are split into
+constexpr float kNoMax = -3.0e38f;    // running maximum of a column that has seen nothing
+
+// one wave's share of a 32-token unit, as loaded: K fragment `wave` and V
+// fragment `wave` (16 bytes a lane), or their codes and one token's scales
+template <int KB>
+struct Staged {
+  uint32_t k[KB / 4], v[KB / 4];
+  u32x4 e;
+};
+template <>
+struct Staged<0> {
+  u32x4 k, v;
+};
+
 // ---------------------------------------------------------------------------
 // dense causal attention for the last L tokens of each sequence (a prefill
 // chunk whose keys / values were appended): query token i of a sequence
 // holding T tokens sits at position T - L + i and attends to tokens
 // [0, T - L + i] (the causal mask BaseKVCache.makeMask gives for n > 1).
-// A wave owns R column sets of 16 MFMA columns, each column a (query token,
-// q head) pair (16 / G tokens x the G heads of kv head h); the workgroup's
-// W waves take consecutive tokens of one (sequence, kv head) and stream its
-// K / V blocks from block 0 to the last one any of them sees, with an online
-// softmax per column:
+// A wave owns 32 MFMA columns, each a (query token, q head) pair (32 / G
+// tokens x the G heads of kv head h); the workgroup's 8 waves take
+// consecutive tokens of one (sequence, kv head) and walk its tokens in units
+// of 32, with an online softmax per column:
 //   S^T[token][col] = K[token] . Q[col]        (A = K rows, B = Q^T)
 //   O^T[dim][col]  += V^T[dim] . P^T[col]      (A = V^T, B = P^T)
-// An MFMA's A and B operands take the same lane layout, so the
-// fragment-major K / V tiles and the P registers of the decode kernel serve
-// both products unchanged, and each lane holds the running max, sum and
-// O^T entries of its own column.
-// The K / V blocks are streamed in units of 32 tokens (a block of 32, or
-// half of a block of 64: 8 K and 8 V fragments of 1 KiB), each loaded from
-// memory once per workgroup into one of two 16 KiB LDS buffers (every wave
-// fetches 16 / W fragments): the loads of unit u + 1 are in flight while the
-// workgroup computes unit u from the other buffer.  A wave reads each
-// fragment from LDS once and applies it to all R column sets.
-// Affine-quantized caches (KB = 4 / 8 bits, fp16 q / out): a unit's codes
-// and scales / biases are loaded raw into LDS (4.5 / 8.5 KiB) and
-// dequantized once per workgroup into the 16-bit fragment layout above, as
-// fp16 values fl16(scale * code + bias) (one packed fused multiply-add per
-// pair, so each is the correctly rounded dequantized value); the rest runs
-// as for an fp16 cache.  The raw loads run two units ahead: in step u the
-// workgroup loads unit u + 2, dequantizes unit u + 1 and computes unit u.
-// The workgroups of one (sequence, kv head) read the same blocks, so the
+// with v_mfma_f32_32x32x16.  S^T row r of a unit is its token
+// 16 (r / 16) + 8 (r / 4 % 2) + 4 (r / 8 % 2) + r % 4, so that a lane's
+// accumulator entries 8 kk .. 8 kk + 7 are tokens 16 kk + 8 (lane / 32) .. + 7
+// of its column: the P^T operand of k-step kk, with no shuffles, against the
+// V fragments as they are stored.  K fragments are read from LDS by row in
+// the same way (16 bytes a lane from the fragment that holds them).
+//
+// The unit pipeline (one workgroup barrier per unit).  In step u a wave
+//  - computes S of unit u + 1 (K from LDS) while it turns S of unit u into P,
+//    then O += V P of unit u: products that depend on nothing in the
+//    softmax, for the matrix cores to run beside it;
+//  - writes its fragments of unit u + 2, which it loaded two steps ago, to
+//    LDS and loads those of unit u + 4.
+// K has two LDS slots (unit u + 1 is read while u + 2 is written over u), V
+// four.  What bounds it: MFMA issue (16 x 32 cycles a wave and unit, two
+// waves per SIMD) beside ~100 VALU and 16 exp2, and LDS reads (16 KiB a wave
+// and unit, 8 cycles per KiB for the CU's 8 waves: as long as the MFMAs of
+// one SIMD's two waves).
+//
+// V of a bf16 cache is converted to fp16 on its way to LDS (exact for
+// |v| < 65520 down to the fp16 normal range) for an fp16 PV product without
+// the hi / lo split of P; a unit holding a value fp16 cannot take is flagged,
+// and its PV runs in bf16 with P as hi + lo from the cache's own fragments.
+// Codes of an affine cache (KB = 4 / 8 bits, fp16 q / out) are dequantized on
+// the way, as fp16 values fl16(scale * code + bias) (one packed fused
+// multiply-add per pair, so each is the correctly rounded value).
+//
+// The workgroups of one (sequence, kv head, part) read the same units, so the
 // flat workgroup index is remapped to give them consecutive indices within
 // one XCD (workgroups are dealt to the 8 XCDs in turn): they then share that
-// XCD's L2 instead of fetching every block into all eight.
-// grid (ceil(L / (W * R * 16 / G)), Hkv, n)
+// XCD's L2 instead of fetching every unit into all eight.  The tiles with the
+// most tokens come first.
+// nsplit > 1: each tile's units are cut into nsplit runs, whose unnormalised
+// (o, m, l) go to po / pml for k_prefill_combine.
+// Measured, 512-token chunks at 32k tokens, Hq 32, Hkv 8, against the kernel
+// before it (16x16x32 MFMAs, 4-wave workgroups, one unit ahead by LDS DMA, a
+// block-table load waited for at the head of every unit): 8 sequences, bf16
+// 2829 -> 2361 us (923 TFLOP/s), int4 2977 -> 2528 us; one sequence, split in
+// 4, 1353 -> 370 us; a prompt of 8191 fp16 tokens 693 -> 610 us.
+// grid (ceil(L / (256 / G)) * Hkv * n * nsplit)
 // ---------------------------------------------------------------------------
-template <int DT, int TB, int G, int R, int W, int OCC, int KB>
-__global__ __launch_bounds__(64 * W, OCC) void k_prefill(Geometry geo, SeqBatch sb, int L,
-                                                   const uint16_t* __restrict__ q, float sl2,
-                                                   uint16_t* __restrict__ out) {
-  constexpr int QPS = 16 / G;   // query tokens per column set
-  constexpr int KS2 = TB / 32;  // 32-token units (PV k-steps) of a block
-  constexpr int FPW = 16 / W;   // fragments of a unit each wave fetches
-  static_assert(16 % W == 0 && (W == 1 || 8 % W == 0), "fragments split evenly over the waves");
-  static_assert(KB == 0 || (DT == 0 && W == 4), "quantized caches: fp16, four waves");
-  // raw quantized unit: K code fragments (2 tiles x KB / 4), V code fragments
-  // (8 dim tiles / (16 / KB) per fragment), then 32 scale / bias entries
-  constexpr int RKF = KB / 2, RVF = KB / 2, RAWF = RKF + RVF;
+template <int DT, int KB>
+__global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatch sb, int L, int lg, int gx,
+                                                          int nsplit, const uint16_t* __restrict__ q,
+                                                          float sl2, uint16_t* __restrict__ out,
+                                                          float* __restrict__ po, float* __restrict__ pml) {
+  static_assert(KB == 0 || DT == 0, "quantized caches: fp16");
   // the running maximum a column's weights are taken against is raised only
-  // when a block's maximum exceeds it by more than 2^kLazy: the weights then
+  // when a unit's maximum exceeds it by more than 2^kLazy: the weights then
   // stay below 2^kLazy, and the rescaling of O^T (a pass over its registers)
-  // is skipped for most blocks; O^T / l is unchanged by the choice
+  // is skipped for most units; O^T / l is unchanged by the choice
   constexpr float kLazy = 8.f;
-  __shared__ __align__(16) u32x4 s_kv0[16 * 64], s_kv1[16 * 64];
-  __shared__ __align__(16) u32x4 s_raw0[KB ? RAWF * 64 + 32 : 1], s_raw1[KB ? RAWF * 64 + 32 : 1];
-  // bf16 caches: the unit's V as fp16 (exact for |v| < 65520 down to the
-  // fp16 normal range) for an fp16 PV product without the hi / lo split of
-  // P; s_big[u & 1] flags a unit holding a value fp16 cannot take (its PV
-  // then runs in bf16 with P as hi + lo)
   constexpr bool CV = KB == 0 && DT == 1;
-  __shared__ __align__(16) u32x4 s_v16[CV ? 8 * 64 : 1];
-  __shared__ int s_big[2];
+  __shared__ __align__(16) u32x4 s_k[2][8 * 64], s_v[4][8 * 64];
+  __shared__ __align__(16) u32x4 s_ent[KB ? kPfWaves : 1][KB ? 32 : 1];  // each wave's copy of a unit's scales / biases
+  __shared__ int s_flag[4][kPfWaves];  // CV: wave w's V fragment of the slot's unit holds a value fp16 cannot take
   const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int n = lane & 15, g = lane >> 4;
+  const int col = lane & 31, hh = lane >> 5;
   // XCD-grouped workgroup order (a bijection on [0, total))
-  const int gx = gridDim.x, gy = gridDim.y;
-  const int total = gx * gy * gridDim.z;
-  const int flat = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-  const int even = total & ~7;
+  const int total = gridDim.x, flat = blockIdx.x, even = total & ~7;
   const int lid = flat < even ? (flat & 7) * (even >> 3) + (flat >> 3) : flat;
-  const int bx = lid % gx, h = (lid / gx) % gy, bi = lid / (gx * gy);
-  const int twg = bx * W * R * QPS;     // the workgroup's first query token
-  const int t0 = twg + wave * R * QPS;  // this wave's
-  const bool active = t0 < L;
-  const int seq = sb.ids[bi];
+  const int tile = gx - 1 - lid % gx, part = lid / gx % nsplit, pair = lid / (gx * nsplit);
+  const int bi = pair / geo.hkv, h = pair - bi * geo.hkv;
+  const int qpw = kPfCols >> lg;            // query tokens per wave
+  const int twg = tile * kPfWaves * qpw;    // the workgroup's first query token
+  const bool active = twg + wave * qpw < L;
+  const int seq = uniform(sb.ids[bi]);
   const int T = uniform(geo.meta[seq]);
-  const int head = h * G + n % G;
+  const int tq = twg + wave * qpw + (col >> lg), head = (h << lg) + (col & ((1 << lg) - 1));
   // scores are taken as (K . Q') * |sl2| with Q' = Q * sign(sl2): the sign
   // flip is exact, and a positive factor lets the block maximum be found on
-  // the raw products
+  // the raw products.  A padding column (no query token) has Q = 0, sees
+  // every token and is not stored.
   const uint32_t qflip = sl2 < 0.f ? 0x80008000u : 0u;
   const float sc = fabsf(sl2);
-  // column n of set r: query token t0 + r * QPS + n / G, at position pos[r];
-  // a padding column (no query token) has Q = 0, sees every token and is not
-  // stored
-  int pos[R];
-  u32x4 qf[R][4];
+  const int pos = tq < L ? T - L + tq : T;
+  u32x4 qf[8];
+  {
+    const uint16_t* src = q + q_row(sb, bi, head) + (size_t)min(tq, L - 1) * kHeadDim + 8 * hh;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int tq = t0 + r * QPS + n / G;
-    pos[r] = tq < L ? T - L + tq : T;
-#pragma unroll
-    for (int s = 0; s < 4; ++s) qf[r][s] = u32x4{0u, 0u, 0u, 0u};
-    if (tq < L) {
-      const uint16_t* src = q + q_row(sb, bi, head) + (size_t)tq * kHeadDim + 8 * g;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) qf[r][s] = *(const u32x4*)(src + 32 * s) ^ qflip;
-    }
+    for (int s = 0; s < 8; ++s) qf[s] = tq < L ? *(const u32x4*)(src + 16 * s) ^ qflip : u32x4{0u, 0u, 0u, 0u};
   }
-  const int last = T - L + min(L - 1, twg + W * R * QPS - 1);  // the workgroup's last position
+  const int ksh = geo.tb == 64 ? 1 : 0;  // log2 of the units of a block
+  const int last = T - L + min(L - 1, twg + kPfWaves * qpw - 1);  // the workgroup's last position
   const int nunit = last / 32 + 1;
-  // units below nfull are whole and visible to every column of the wave
-  const int nfull = (T - L + t0 + 1) / 32;
+  const int ua = (int)((int64_t)nunit * part / nsplit), ub = (int)((int64_t)nunit * (part + 1) / nsplit);
+  // units below nfull are whole and visible to every column of the workgroup
+  const int nfull = min((T - L + twg + 1) / 32, ub);
+
+  // --- units from memory: this wave's fragments, in the slab's own order
   const int32_t* bt = block_table(geo, seq);
-  // this wave's fragments of unit u go straight from memory into LDS
-  // (global_load_lds: lane i's 16 bytes land at dst + 16 i).  Buffer slot
-  // f = wave + i * W: K fragment 8 hh + f of the block for f < 8 (QK tiles
-  // 2 hh, 2 hh + 1), V fragment (f - 8) * KS2 + hh (dims 16 (f - 8) ..,
-  // PV k-step hh) for f >= 8, where hh = u % KS2
-  auto fetch = [&](int u, u32x4* buf) __attribute__((always_inline)) {
-    const int page = uniform(bt[u / KS2]), hh = u % KS2;
+  const int lastblk = last / geo.tb;
+  int pbase = ua >> ksh;  // lane i of pagev: page of block pbase + i
+  int pagev = bt[min(pbase + lane, lastblk)];
+  auto load = [&](int x, Staged<KB>& st) __attribute__((always_inline)) {
+    x = max(min(x, ub - 1), ua);
+    const int blk = x >> ksh, sub = x & ((1 << ksh) - 1);
+    if (blk >= pbase + 64) {
+      pbase += 64;
+      pagev = bt[min(pbase + lane, lastblk)];
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // here, every 64 blocks, and not at each use of pagev
+    }
+    const int page = __builtin_amdgcn_readlane(pagev, blk - pbase);
     const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-    const u32x4* Kf = (const u32x4*)(slab + geo.k_off) + (8 * hh + wave) * 64 + lane;
-    const u32x4* Vf = (const u32x4*)(slab + geo.v_off) + (wave * KS2 + hh) * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < FPW; ++i)
-      __builtin_amdgcn_global_load_lds(
-          (const void*)(i < 8 / W ? Kf + i * W * 64 : Vf + (i - 8 / W) * W * KS2 * 64),
-          (__attribute__((address_space(3))) void*)(buf + (wave + i * W) * 64), 16, 0, 0);
-  };
-  // raw quantized unit u: slots f = wave + i * W; K fragment hh * RKF + f of
-  // the block for f < RKF (QK tiles 2 hh, 2 hh + 1), V fragment
-  // (f - RKF) * KS2 + hh for f >= RKF; the unit's scale / bias entries for
-  // tokens 8 g' + e (g' = 0..3, e = 0..7) go to entries 8 g' + e, loaded by
-  // lanes 0..31 of the last wave
-  auto fetch_raw = [&](int u, u32x4* buf) __attribute__((always_inline)) {
-    const int page = uniform(bt[u / KS2]), hh = u % KS2;
-    const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-    const u32x4* Kf = (const u32x4*)(slab + geo.k_off) + lane;
-    const u32x4* Vf = (const u32x4*)(slab + geo.v_off) + lane;
-#pragma unroll
-    for (int i = 0; i < RAWF / W; ++i) {
-      const int f = wave + i * W;
-      __builtin_amdgcn_global_load_lds(
-          (const void*)(f < RKF ? Kf + (hh * RKF + f) * 64 : Vf + ((f - RKF) * KS2 + hh) * 64),
-          (__attribute__((address_space(3))) void*)(buf + f * 64), 16, 0, 0);
-    }
-    if (wave == W - 1 && lane < 32) {
-      const u32x4* Sf = (const u32x4*)(slab + geo.sb_off) + (lane >> 3) * (TB / 4) + 8 * hh + (lane & 7);
-      __builtin_amdgcn_global_load_lds((const void*)Sf,
-                                       (__attribute__((address_space(3))) void*)(buf + RAWF * 64), 16, 0, 0);
-    }
-  };
-  // dequantize a raw unit into the fp16 fragment layout: wave 0 / 1 writes
-  // the 4 K fragments of QK tile 0 / 1 (one token per lane), wave 2 / 3 the
-  // V fragments of dim tiles 0..3 / 4..7 (8 tokens per lane)
-  auto dequant = [&](const u32x4* raw, u32x4* kv) __attribute__((always_inline)) {
-    using QC = QCode<KB>;
-    const u32x4* ent = raw + RAWF * 64;  // scale / bias entry of token x of the unit
-    // f16 pairs (s * c + b): c from the f16 values OFF + c / INV_UNIT exactly
-    auto deq = [&](u32x4 hv, const uint32_t* sp, const uint32_t* bp) __attribute__((always_inline)) {
-      const f16x2 unit2 = {(_Float16)QC::INV_UNIT, (_Float16)QC::INV_UNIT};
-      const f16x2 off2 = {(_Float16)(-QC::OFF * QC::INV_UNIT), (_Float16)(-QC::OFF * QC::INV_UNIT)};
-      u32x4 r;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        // (a vector element is copied out first: __builtin_bit_cast of
-        // hv[k] itself reads element 0 with this compiler)
-        const uint32_t w = hv[k];
-        const f16x2 c = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, w), unit2, off2);
-        r[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, sp[k]), c,
-                                                                       __builtin_bit_cast(f16x2, bp[k])));
-      }
-      return r;
-    };
-    if (wave < 2) {
-      // row m of QK tile t is token 8 (m / 4) + 4 t + m % 4 of the unit (the
-      // tile's MFMA output rows then land on tok_of(g, 4 t + i))
-      const int t = wave, m = lane & 15;
-      const u32x4 e = ent[8 * (m >> 2) + 4 * t + (m & 3)];
-      // (k scale, k bias) of dim group 0 / 1 in both halves
-      const uint32_t s0 = __builtin_amdgcn_perm(e[0], e[0], 0x01000100u), s1 = __builtin_amdgcn_perm(e[0], e[0], 0x03020302u);
-      const uint32_t b0 = __builtin_amdgcn_perm(e[1], e[1], 0x01000100u), b1 = __builtin_amdgcn_perm(e[1], e[1], 0x03020302u);
-      u32x4 rw[2];
-#pragma unroll
-      for (int f = 0; f < RKF / 2; ++f) rw[f] = raw[(t * (RKF / 2) + f) * 64 + lane];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        u32x4 hv;
-        if constexpr (KB == 4) hv = nib_to_f16(rw[0][s]);
-        else hv = byte_to_f16(rw[s >> 1][2 * (s & 1)], rw[s >> 1][2 * (s & 1) + 1]);
-        const uint32_t sp[4] = {s < 2 ? s0 : s1, s < 2 ? s0 : s1, s < 2 ? s0 : s1, s < 2 ? s0 : s1};
-        const uint32_t bp[4] = {s < 2 ? b0 : b1, s < 2 ? b0 : b1, s < 2 ? b0 : b1, s < 2 ? b0 : b1};
-        kv[(t * 4 + s) * 64 + lane] = deq(hv, sp, bp);
-      }
-    } else {
-      const int half = wave - 2;  // dim group of dim tiles 4 half .. 4 half + 3
-      // (v scale, v bias) of tokens 8 g + 2 k, 8 g + 2 k + 1 as f16 pairs
-      uint32_t sp[4], bp[4];
-      const uint32_t sel = half ? 0x07060302u : 0x05040100u;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const u32x4 e0 = ent[8 * g + 2 * k], e1 = ent[8 * g + 2 * k + 1];
-        sp[k] = __builtin_amdgcn_perm(e1[2], e0[2], sel);
-        bp[k] = __builtin_amdgcn_perm(e1[3], e0[3], sel);
-      }
-      u32x4 rw[2];
-#pragma unroll
-      for (int f = 0; f < RVF / 2; ++f) rw[f] = raw[(RKF + half * (RVF / 2) + f) * 64 + lane];
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        u32x4 hv;
-        if constexpr (KB == 4) hv = nib_to_f16(rw[0][d]);
-        else hv = byte_to_f16(rw[d >> 1][2 * (d & 1)], rw[d >> 1][2 * (d & 1) + 1]);
-        kv[(8 + 4 * half + d) * 64 + lane] = deq(hv, sp, bp);
-      }
-    }
-  };
-  float m[R], l[R], thr[R];
-  f32x4 o[R][8];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    m[r] = -INFINITY;
-    thr[r] = -INFINITY;
-    l[r] = 0.f;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[r][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  // unit u from LDS (tokens 32 u .. 32 u + 31 of the sequence); MASK: the
-  // causal limit and the sequence end apply.  PDT: type of the PV product
-  // (P and V); when it differs from DT, V comes from the fp16 copy vkv.
-  auto unit = [&](int u, const u32x4* kv, const u32x4* vkv, auto mask_tag, auto pdt_tag)
-      __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
-    constexpr int PDT = decltype(pdt_tag)::value;
-    f32x4 acc[R][2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      u32x4 kf[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) kf[s] = kv[(t * 4 + s) * 64];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < 4; ++s) acc[r][t] = mfma16x16x32<DT>(kf[s], qf[r][s], acc[r][t]);
-      }
-    }
-    // P^T operand: lane (column n, group g) -> tokens 32 u + tok_of(g,
-    // 2 jj (+1)); bf16 P is split into hi + lo
-    u32x4 pf[R], pl[R];
-    (void)pl;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      float x[8];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[4 * t + i] = acc[r][t][i];
-      if constexpr (MASK) {
-        // causal: token 32 u + tok_of(g, e) <= pos (which is below T)
-        const int lim = pos[r] - 32 * u;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = tok_of(g, e) <= lim ? x[e] : -INFINITY;
-      }
-      // the column's maximum is needed only when some lane's scores pass
-      // the raising threshold thr = (m + kLazy) / sc
-      const float lm = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-      if (__builtin_amdgcn_ballot_w64(lm > thr[r])) {
-        // every column sees token 0 in block 0, so bm is finite there
-        const float bm = max_over_groups(lm) * sc;
-        const bool raise = bm > m[r] + kLazy;
-        const float mn = raise ? bm : m[r];
-        const float alpha = __builtin_amdgcn_exp2f(m[r] - mn);  // 0 from -inf
-        l[r] *= alpha;
-        m[r] = mn;
-        thr[r] = (mn + kLazy) / sc;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[r][dt][i] *= alpha;
-      }
-      float ps = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[e] = __builtin_amdgcn_exp2f(fmaf(x[e], sc, -m[r]));
-        ps += x[e];
-      }
-      l[r] += ps;  // this lane's tokens; the column's groups are summed at the end
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const float p0 = x[2 * jj], p1 = x[2 * jj + 1];
-        const uint32_t hi = cvt_pk<PDT>(p0, p1);
-        pf[r][jj] = hi;
-        if constexpr (PDT == 1)
-          pl[r][jj] = cvt_pk<1>(p0 - __uint_as_float(hi << 16), p1 - __uint_as_float(hi & 0xFFFF0000u));
-      }
-    }
-    const int valid = min(32, T - 32 * u);
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      u32x4 vf = PDT == DT ? kv[(8 + dt) * 64] : vkv[dt * 64];
-      if constexpr (MASK) {
-        // V of tokens past the sequence end (stale page data) is zeroed
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int tk = 8 * g + 2 * jj;
-          vf[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        o[r][dt] = mfma16x16x32<PDT>(vf, pf[r], o[r][dt]);
-        if constexpr (PDT == 1) o[r][dt] = mfma16x16x32<PDT>(vf, pl[r], o[r][dt]);
-      }
-    }
-  };
-  // 16-bit: unit u is read from buffer u & 1 while unit u + 1 is loaded
-  // into the other one, which held unit u - 1: every wave finished that
-  // before the barrier ending the previous step.  Quantized: raw buffer
-  // u & 1 (unit u, dequantized in the previous step) takes the loads of unit
-  // u + 2 while raw buffer (u + 1) & 1 is dequantized into fp16 buffer
-  // (u + 1) & 1 (which held unit u - 1).  Every wave takes nunit steps (one
-  // barrier each); a wave past the last query token only loads (and
-  // dequantizes).
-  auto step = [&](int u, const u32x4* cur, u32x4* nxt, u32x4* raw_ld, const u32x4* raw_dq, auto act,
-                  auto mask_tag) __attribute__((always_inline)) {
+    const uint8_t *ks = slab + geo.k_off, *vs = slab + geo.v_off;
     if constexpr (KB == 0) {
-      if (u + 1 < nunit) fetch(u + 1, nxt);
+      st.k = *(const u32x4*)(ks + (8 * sub + wave) * 1024 + lane * 16);
+      st.v = *(const u32x4*)(vs + ((wave << ksh) + sub) * 1024 + lane * 16);
     } else {
-      if (u + 2 < nunit) fetch_raw(u + 2, raw_ld);
-      if (u + 1 < nunit) dequant(raw_dq, nxt);
+      if constexpr (KB == 4) {
+        st.k[0] = *(const uint32_t*)(ks + (2 * sub + (wave >> 2)) * 1024 + 4 * (wave & 3) + lane * 16);
+        st.v[0] = *(const uint32_t*)(vs + (((wave >> 2) << ksh) + sub) * 1024 + 4 * (wave & 3) + lane * 16);
+      } else {
+        const uint2 a = *(const uint2*)(ks + (4 * sub + (wave >> 1)) * 1024 + 8 * (wave & 1) + lane * 16);
+        const uint2 b = *(const uint2*)(vs + (((wave >> 1) << ksh) + sub) * 1024 + 8 * (wave & 1) + lane * 16);
+        st.k[0] = a.x;
+        st.k[1] = a.y;
+        st.v[0] = b.x;
+        st.v[1] = b.y;
+      }
+      const int x32 = lane & 31;
+      st.e = *(const u32x4*)(slab + geo.sb_off + (((x32 >> 3) * (geo.tb >> 2)) + 8 * sub + (x32 & 7)) * 16);
     }
-    if constexpr (CV) {
-      // V of unit u to fp16 (two fragment lanes per thread); a bf16 value of
-      // magnitude >= 65536 (or inf / NaN) flags the unit
-      bool big = false;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int it = threadIdx.x + 256 * i;
-        const u32x4 w = cur[(8 + (it >> 6)) * 64 + (it & 63)];
-        u32x4 h;
+  };
+  // --- and into LDS, as 16-bit fragments; r: the unit's index from ua
+  auto stage = [&](int r, const Staged<KB>& st, auto mask_tag) __attribute__((always_inline)) {
+    u32x4 kw, vw;
+    if constexpr (KB == 0) {
+      kw = st.k;
+      vw = st.v;
+      if constexpr (CV) {
+        // a bf16 value of magnitude >= 65536 (or inf / NaN) flags the unit
+        uint32_t big = 0u;
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const uint32_t x = w[k];
-          big |= (x & 0x7FFFu) >= 0x4780u || ((x >> 16) & 0x7FFFu) >= 0x4780u;
-          h[k] = cvt_pk<0>(__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u));
+          const uint32_t x = vw[k];
+          big |= ((x & 0x7FFFu) + 0x3880u) | ((((x >> 16) & 0x7FFFu) + 0x3880u));  // bit 15: >= 0x4780
+          vw[k] = cvt_pk<0>(__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u));
         }
-        s_v16[it] = h;
+        const bool any = __builtin_amdgcn_ballot_w64((big & 0x8000u) != 0u) != 0;
+        if (lane == 0) s_flag[r & 3][wave] = any ? 1 : 0;
       }
-      if (__builtin_amdgcn_ballot_w64(big) != 0 && lane == 0) s_big[u & 1] = 1;
-      if (threadIdx.x == 0) s_big[(u + 1) & 1] = 0;  // last read in step u - 1
-      __syncthreads();
-      if constexpr (decltype(act)::value) {
-        if (s_big[u & 1]) unit(u, cur + lane, s_v16 + lane, mask_tag, std::integral_constant<int, 1>{});
-        else unit(u, cur + lane, s_v16 + lane, mask_tag, std::integral_constant<int, 0>{});
+    } else {
+      using QC = QCode<KB>;
+      // f16 pairs (s * c + b): c from the f16 values OFF + c / INV_UNIT exactly
+      auto deq = [&](u32x4 hv, const uint32_t* sp, const uint32_t* bp) __attribute__((always_inline)) {
+        const f16x2 unit2 = {(_Float16)QC::INV_UNIT, (_Float16)QC::INV_UNIT};
+        const f16x2 off2 = {(_Float16)(-QC::OFF * QC::INV_UNIT), (_Float16)(-QC::OFF * QC::INV_UNIT)};
+        u32x4 o4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          // (a vector element is copied out first: __builtin_bit_cast of
+          // hv[k] itself reads element 0 with this compiler)
+          const uint32_t w = hv[k];
+          const f16x2 c = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, w), unit2, off2);
+          o4[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, sp[k]), c,
+                                                                        __builtin_bit_cast(f16x2, bp[k])));
+        }
+        return o4;
+      };
+      auto codes = [&](const uint32_t* w) __attribute__((always_inline)) {
+        if constexpr (KB == 4) return nib_to_f16(w[0]);
+        else return byte_to_f16(w[0], w[1]);
+      };
+      // the unit's scale / bias entries through this wave's own LDS rows
+      // (a wave's LDS accesses complete in order)
+      s_ent[wave][lane & 31] = st.e;
+      wave_lds_order();
+      const uint32_t* ent = (const uint32_t*)s_ent[wave];
+      {
+        // row m of QK key tile t is token 8 (m / 4) + 4 t + m % 4 of the unit
+        const int t = wave >> 2, m = lane & 15;
+        const int x = 8 * (m >> 2) + 4 * t + (m & 3);
+        const uint32_t sel = (wave & 2) ? 0x03020302u : 0x01000100u;  // dim group of k-step wave & 3
+        const uint32_t s2 = __builtin_amdgcn_perm(ent[4 * x], ent[4 * x], sel);
+        const uint32_t b2 = __builtin_amdgcn_perm(ent[4 * x + 1], ent[4 * x + 1], sel);
+        const uint32_t sp[4] = {s2, s2, s2, s2}, bp[4] = {b2, b2, b2, b2};
+        kw = deq(codes(st.k), sp, bp);
       }
-    } else if constexpr (decltype(act)::value) {
-      unit(u, cur + lane, nullptr, mask_tag, std::integral_constant<int, DT>{});
+      {
+        // (v scale, v bias) of tokens 8 g + 2 k, 8 g + 2 k + 1 as f16 pairs
+        const int g = lane >> 4;
+        uint32_t sp[4], bp[4];
+        const uint32_t sel = (wave >> 2) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint2 e0 = *(const uint2*)(ent + 4 * (8 * g + 2 * k) + 2), e1 = *(const uint2*)(ent + 4 * (8 * g + 2 * k + 1) + 2);
+          sp[k] = __builtin_amdgcn_perm(e1.x, e0.x, sel);
+          bp[k] = __builtin_amdgcn_perm(e1.y, e0.y, sel);
+        }
+        vw = deq(codes(st.v), sp, bp);
+      }
+      wave_lds_order();
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's LDS loads have landed
-    __syncthreads();
+    if constexpr (decltype(mask_tag)::value) {
+      // V of tokens past the sequence end (stale page data) is zeroed
+      const int valid = T - 32 * (ua + r), g = lane >> 4;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const int tk = 8 * g + 2 * jj;
+        vw[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
+      }
+    }
+    s_k[r & 1][wave * 64 + lane] = kw;
+    s_v[r & 3][wave * 64 + lane] = vw;
   };
-  // the mask-free units in pairs (fixed buffers, no branch between the
-  // products of consecutive units), then the rest one by one
-  auto run = [&](auto act) __attribute__((always_inline)) {
-    const int npair = min(nfull, nunit) & ~1;
-    int u = 0;
-#pragma unroll 1
-    for (; u < npair; u += 2) {
-      step(u, s_kv0, s_kv1, s_raw0, s_raw1, act, std::false_type{});
-      step(u + 1, s_kv1, s_kv0, s_raw1, s_raw0, act, std::false_type{});
-    }
-#pragma unroll 1
-    for (; u < nunit; ++u) {
-      const bool odd = u & 1;
-      const u32x4* cur = odd ? s_kv1 : s_kv0;
-      u32x4* nxt = odd ? s_kv0 : s_kv1;
-      u32x4* raw_ld = odd ? s_raw1 : s_raw0;
-      const u32x4* raw_dq = odd ? s_raw0 : s_raw1;
-      if (u < nfull) step(u, cur, nxt, raw_ld, raw_dq, act, std::false_type{});
-      else step(u, cur, nxt, raw_ld, raw_dq, act, std::true_type{});
-    }
+
+  // --- this wave's columns
+  float m = kNoMax, l = 0.f, thr = -INFINITY, lm = -INFINITY;
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.f;
+  // lane offsets (16-byte entries) of the K and V operands in a slot
+  const int kl = ((col >> 3) & 1) * 256 + 8 * (col >> 4) + 4 * ((col >> 2) & 1) + (col & 3) + 16 * hh;
+  const int vl = (col >> 4) * 64 + (col & 15) + 16 * hh;
+  auto scores = [&](int r) __attribute__((always_inline)) {  // S^T of unit ua + r
+    const u32x4* kp = s_k[r & 1] + kl;
+    f32x16 a;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) a[i] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) a = mfma32x32x16<DT>(kp[32 * s], qf[s], a);
+    return a;
   };
-  if constexpr (KB == 0) {
-    if (threadIdx.x == 0) s_big[0] = 0;
-    fetch(0, s_kv0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  } else {
-    fetch_raw(0, s_raw0);
-    if (nunit > 1) fetch_raw(1, s_raw1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    dequant(s_raw0, s_kv0);
-    __syncthreads();
+  // the largest score of this lane's tokens, masked past the column's position
+  auto lane_max = [&](f32x16& a, int r, auto mask_tag) __attribute__((always_inline)) {
+    if constexpr (decltype(mask_tag)::value) {
+      const int lim = pos - 32 * (ua + r) - 8 * hh;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a[i] = 16 * (i >> 3) + (i & 7) <= lim ? a[i] : -INFINITY;
+    }
+    float x = fmaxf(a[0], a[1]);
+#pragma unroll
+    for (int i = 2; i < 16; i += 2) x = fmaxf(x, fmaxf(a[i], a[i + 1]));
+    return x;
+  };
+  // step r: `cur` holds S of unit r, `nxt` takes that of unit r + 1.  BIG: the
+  // unit's V holds a value fp16 cannot take
+  int flag = 0;  // CV: whether the next step's unit does
+  auto step = [&](int r, f32x16& cur, f32x16& nxt, Staged<KB>& st, auto act, auto mask_tag, auto big_tag)
+      __attribute__((always_inline)) {
+    constexpr bool ACT = decltype(act)::value;
+    [[maybe_unused]] int fnext = 0;
+    if constexpr (ACT) {
+      // the column's maximum is needed only when some lane's scores pass the
+      // raising threshold thr = (m + kLazy) / sc
+      if (__builtin_amdgcn_ballot_w64(lm > thr)) {
+        const float bm = pair_max(lm) * sc;
+        const bool raise = bm > m + kLazy;
+        const float mn = raise ? bm : m;
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        l *= alpha;
+        m = mn;
+        thr = (mn + kLazy) / sc;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+      }
+      if constexpr (CV) fnext = s_flag[(r + 1) & 3][lane & 7];
+    }
+    stage(r + 2, st, mask_tag);
+    load(ua + r + 4, st);
+    if constexpr (ACT) {
+      nxt = scores(r + 1);
+      float ps = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        cur[i] = __builtin_amdgcn_exp2f(fmaf(cur[i], sc, -m));
+        ps += cur[i];
+      }
+      l += ps;  // this lane's tokens; the column's halves are summed at the end
+      if constexpr (decltype(big_tag)::value) {
+        // bf16 P as hi + lo against the cache's own V fragments
+        const int x = ua + r, sub = x & ((1 << ksh) - 1);
+        const uint8_t* vs = geo.pool + ((size_t)uniform(bt[x >> ksh]) * geo.hkv + h) * geo.slab_bytes + geo.v_off;
+        const int valid = T - 32 * x;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+          u32x4 ph, pl;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            const float p0 = cur[8 * kk + 2 * jj], p1 = cur[8 * kk + 2 * jj + 1];
+            const uint32_t w = cvt_pk<1>(p0, p1);
+            ph[jj] = w;
+            pl[jj] = cvt_pk<1>(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xFFFF0000u));
+          }
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            u32x4 vf = *(const u32x4*)(vs + (((2 * dt + (col >> 4)) << ksh) + sub) * 1024 +
+                                       ((col & 15) + 16 * (2 * kk + hh)) * 16);
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) {
+              const int tk = 8 * (2 * kk + hh) + 2 * jj;
+              vf[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
+            }
+            o[dt] = mfma32x32x16<1>(vf, ph, o[dt]);
+            o[dt] = mfma32x32x16<1>(vf, pl, o[dt]);
+          }
+        }
+      } else {
+        const u32x4* vp = s_v[r & 3] + vl;
+        u32x4 pf[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) pf[kk][jj] = cvt_pk<0>(cur[8 * kk + 2 * jj], cur[8 * kk + 2 * jj + 1]);
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk) o[dt] = mfma32x32x16<0>(vp[dt * 128 + kk * 32], pf[kk], o[dt]);
+      }
+      lm = lane_max(nxt, r + 1, mask_tag);
+      if constexpr (CV) flag = __builtin_amdgcn_ballot_w64(fnext != 0) != 0 ? 1 : 0;
+    }
+    unit_barrier();
+  };
+
+  Staged<KB> st0, st1;
+  f32x16 sa, sb2;
+  load(ua, st0);
+  load(ua + 1, st1);
+  stage(0, st0, std::true_type{});
+  load(ua + 2, st0);
+  stage(1, st1, std::true_type{});
+  load(ua + 3, st1);
+  unit_barrier();
+  if (active) {
+    sa = scores(0);
+    lm = lane_max(sa, 0, std::true_type{});
+    if constexpr (CV) flag = __builtin_amdgcn_ballot_w64(s_flag[0][lane & 7] != 0) != 0 ? 1 : 0;
   }
+  unit_barrier();
+  // every wave takes ub - ua steps (one barrier each); a wave past the last
+  // query token only loads and stages.  The steps whose units (up to r + 2)
+  // are whole and visible to every column go in pairs (fixed registers for
+  // both score tiles and both staged units), the others one by one.
+  auto run = [&](auto act) __attribute__((always_inline)) {
+    const int n = ub - ua, plain = nfull - ua - 3;  // pairs r, r + 1 with r + 3 < nfull - ua
+    int r = 0;
+    auto flip = [&]() __attribute__((always_inline)) {
+      const f32x16 sx = sa;
+      sa = sb2;
+      sb2 = sx;
+      const Staged<KB> tx = st0;
+      st0 = st1;
+      st1 = tx;
+    };
+#pragma unroll 1
+    while (r < n) {
+      if constexpr (CV && decltype(act)::value) {
+        if (flag) {
+          step(r++, sa, sb2, st0, act, std::true_type{}, std::true_type{});
+          flip();
+          continue;
+        }
+      }
+      if (r < plain) {
+#pragma unroll 1
+        do {
+          step(r++, sa, sb2, st0, act, std::false_type{}, std::false_type{});
+          if (CV && flag) {
+            flip();
+            break;
+          }
+          step(r++, sb2, sa, st1, act, std::false_type{}, std::false_type{});
+        } while (r < plain && !(CV && flag));
+        continue;
+      }
+      step(r++, sa, sb2, st0, act, std::true_type{}, std::false_type{});
+      flip();
+    }
+  };
   if (active) run(std::true_type{});
   else run(std::false_type{});
   if (!active) return;
-  // O^T: lane (column n, group g) holds dims 16 dt + 4 g + i of its column
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const float lt = sum_over_groups(l[r]);
-    const int tq = t0 + r * QPS + n / G;
-    if (tq >= L) continue;
+  // O^T: entry i of a lane is dim 32 dt + 8 (i / 4) + 4 hh + i % 4 of its column
+  const float lt = pair_sum(l);
+  if (tq >= L) return;
+  if (nsplit == 1) {
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
-    uint16_t* dst = out + q_row(sb, bi, head) + (size_t)tq * kHeadDim + 4 * g;
+    uint16_t* dst = out + q_row(sb, bi, head) + (size_t)tq * kHeadDim + 4 * hh;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
-      const uint32_t lo = (uint32_t)from_f32<DT>(o[r][dt][0] * inv) | ((uint32_t)from_f32<DT>(o[r][dt][1] * inv) << 16);
-      const uint32_t hi = (uint32_t)from_f32<DT>(o[r][dt][2] * inv) | ((uint32_t)from_f32<DT>(o[r][dt][3] * inv) << 16);
-      *(uint2*)(dst + 16 * dt) = make_uint2(lo, hi);
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *(uint2*)(dst + 32 * dt + 8 * i) = make_uint2(pack2<DT>(o[dt][4 * i] * inv, o[dt][4 * i + 1] * inv),
+                                                     pack2<DT>(o[dt][4 * i + 2] * inv, o[dt][4 * i + 3] * inv));
+  } else {
+    const size_t rows = (size_t)sb.n * geo.hq * L;
+    const size_t row = part * rows + ((size_t)bi * geo.hq + head) * L + tq;
+    float* dst = po + row * kHeadDim + 4 * hh;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *(f32x4*)(dst + 32 * dt + 8 * i) = f32x4{o[dt][4 * i], o[dt][4 * i + 1], o[dt][4 * i + 2], o[dt][4 * i + 3]};
+    if (hh == 0) *(float2*)(pml + 2 * row) = make_float2(m, lt);
+  }
+}
+
+// merges the parts of each output row: 32 threads a row, 4 dims each
+template <int DT>
+__global__ __launch_bounds__(256) void k_prefill_combine(int rows, int nsplit, const float* __restrict__ po,
+                                                        const float* __restrict__ pml,
+                                                        uint16_t* __restrict__ out) {
+  const int row = blockIdx.x * 8 + (threadIdx.x >> 5), c = threadIdx.x & 31;
+  if (row >= rows) return;
+  float M = kNoMax;
+  for (int p = 0; p < nsplit; ++p) M = fmaxf(M, pml[2 * ((size_t)p * rows + row)]);
+  float l = 0.f;
+  f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < nsplit; ++p) {
+    const size_t at = (size_t)p * rows + row;
+    const float2 ml = *(const float2*)(pml + 2 * at);
+    const f32x4 x = *(const f32x4*)(po + at * kHeadDim + 4 * c);
+    const float w = __builtin_amdgcn_exp2f(ml.x - M);
+    l += w * ml.y;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] += w * x[i];
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  *(uint2*)(out + (size_t)row * kHeadDim + 4 * c) =
+      make_uint2(pack2<DT>(a[0] * inv, a[1] * inv), pack2<DT>(a[2] * inv, a[3] * inv));
+}
+
+// Parts for n sequences of at most `tokens` tokens: the number with the least
+// rounds of workgroups (one per CU at a time) times the units a round takes,
+// where a split adds the merge.  A chunk whose tiles fill the CUs once or a
+// whole number of times is not split (8 sequences of 512 tokens: 512 tiles);
+// one sequence's 64 tiles are split in 4 (370 us; unsplit they take 4 times
+// the units of a round).
+int prefill_splits(const Geometry& g, int n, int L, int tokens) {
+  if (g.cus <= 0) return 1;
+  const int64_t tiles = (int64_t)((L * g.group + kPfWaves * kPfCols - 1) / (kPfWaves * kPfCols)) * g.hkv * n;
+  const int64_t rows = (int64_t)n * g.hq * L;
+  const int units = (tokens + 31) / 32;
+  int best = 1;
+  double cost = 0.0;
+  for (int s = 1; s <= kPfSplits; ++s) {
+    if (s > 1 && (rows * s > kPrefillRows || units < 8 * s)) break;
+    // rounds of workgroups, each the units of its part and about 4 more for its start and end
+    const double c = (double)((tiles * s + g.cus - 1) / g.cus) * ((double)units / s + 4.0) +
+                     (s > 1 ? 8.0 + (double)rows * s * 4e-4 : 0.0);
+    if (s == 1 || c < 0.97 * cost) {
+      best = s;
+      cost = c;
     }
   }
+  return best;
 }
 
-template <int DT, int TB, int KB>
-static void prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, const uint16_t* q, float sl2,
-                             uint16_t* out, hipStream_t s, Timing* prof) {
-  constexpr int W = 4, R = 2, OCC = 2;
-  const int per_wg = W * R * (16 / g.group);
-  const dim3 grid((L + per_wg - 1) / per_wg, g.hkv, b.n), blk(64 * W);
-  const int kd = kProfPrefill;
-  switch (g.group) {
-    case 1: launch(k_prefill<DT, TB, 1, R, W, OCC, KB>, grid, blk, 0, s, prof, kd, g, b, L, q, sl2, out); break;
-    case 2: launch(k_prefill<DT, TB, 2, R, W, OCC, KB>, grid, blk, 0, s, prof, kd, g, b, L, q, sl2, out); break;
-    case 4: launch(k_prefill<DT, TB, 4, R, W, OCC, KB>, grid, blk, 0, s, prof, kd, g, b, L, q, sl2, out); break;
-    case 8: launch(k_prefill<DT, TB, 8, R, W, OCC, KB>, grid, blk, 0, s, prof, kd, g, b, L, q, sl2, out); break;
-    default: launch(k_prefill<DT, TB, 16, R, W, OCC, KB>, grid, blk, 0, s, prof, kd, g, b, L, q, sl2, out); break;
-  }
+template <int DT, int KB>
+static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, int nsplit, const uint16_t* q, float sl2,
+                                   uint16_t* out, float* ws, hipStream_t s, Timing* prof) {
+  const int lg = __builtin_ctz((unsigned)g.group);
+  const int per_wg = (kPfWaves * kPfCols) >> lg;
+  const int gx = (L + per_wg - 1) / per_wg;
+  const int rows = b.n * g.hq * L;
+  float* pml = ws ? ws + (size_t)nsplit * rows * kHeadDim : nullptr;
+  launch(k_prefill<DT, KB>, dim3((unsigned)gx * g.hkv * b.n * nsplit), dim3(64 * kPfWaves), 0, s, prof, kProfPrefill, g,
+         b, L, lg, gx, nsplit, q, sl2, out, ws, pml);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || nsplit == 1) return e;
+  hipLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0, s, rows, nsplit, ws, pml, out);
+  return hipGetLastError();
 }
 
-hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, const void* q, float scale,
-                          void* out, hipStream_t s, Timing* prof) {
+hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, int nsplit, const void* q, float scale,
+                          void* out, float* ws, hipStream_t s, Timing* prof) {
   const float sl2 = scale * 1.4426950408889634f;
   const uint16_t* qq = (const uint16_t*)q;
   uint16_t* oo = (uint16_t*)out;
-  if (g.kv_bits == 4) {
-    if (g.tb == 64) prefill_dispatch<0, 64, 4>(g, b, L, qq, sl2, oo, s, prof);
-    else prefill_dispatch<0, 32, 4>(g, b, L, qq, sl2, oo, s, prof);
-  } else if (g.kv_bits == 8) {
-    if (g.tb == 64) prefill_dispatch<0, 64, 8>(g, b, L, qq, sl2, oo, s, prof);
-    else prefill_dispatch<0, 32, 8>(g, b, L, qq, sl2, oo, s, prof);
-  } else if (g.dtype == 0) {
-    if (g.tb == 64) prefill_dispatch<0, 64, 0>(g, b, L, qq, sl2, oo, s, prof);
-    else prefill_dispatch<0, 32, 0>(g, b, L, qq, sl2, oo, s, prof);
-  } else {
-    if (g.tb == 64) prefill_dispatch<1, 64, 0>(g, b, L, qq, sl2, oo, s, prof);
-    else prefill_dispatch<1, 32, 0>(g, b, L, qq, sl2, oo, s, prof);
-  }
-  return hipGetLastError();
+  if (g.kv_bits == 4) return prefill_dispatch<0, 4>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.kv_bits == 8) return prefill_dispatch<0, 8>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.dtype == 0) return prefill_dispatch<0, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  return prefill_dispatch<1, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
 }
 
 }  // namespace bsattn
