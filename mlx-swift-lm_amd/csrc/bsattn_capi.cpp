@@ -853,15 +853,14 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
   const int tb = c->d.block_size;
   int max_nc = 0;
   // (create requires recent_blocks >= 1: the block a token completes is never scored)
-  bool one_launch = c->d.kv_bits == 0 && n_seqs <= kMaxBatch;
+  bool one_launch = n_seqs <= kMaxBatch;
   for (int sq : seqs) {
     if ((int64_t)c->len[sq] + 1 > (int64_t)c->d.max_blocks_per_seq * tb) one_launch = false;
     else max_nc = std::max(max_nc, candidates(g, c->len[sq] + 1));
   }
-  // fused: the append launch, then the fused decode kernel (scoring inside);
-  // otherwise append + scoring in one launch, then selection + attention
+  // fused: the fused decode kernel, append and scoring inside; otherwise
+  // append + scoring in one launch, then selection + attention
   const bool fused = one_launch && fused_decode_ok(g, n_seqs, max_nc);
-  one_launch = one_launch && (fused || max_nc <= fused_select_limit(g.top_k));
   if (!one_launch) {
     rc = bsattn_append(c, k, v, seq_ids, n_seqs, 1, stream);
     if (rc) return rc;
@@ -878,14 +877,15 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
     rc = flush_patches(c, patches, s);
     if (rc) return rc;
   }
-  PatchBatch pb{};
-  pb.n = (int32_t)patches.size();
-  for (int i = 0; i < pb.n; ++i) {
-    pb.idx[i] = patches[i].first;
-    pb.val[i] = patches[i].second;
+  StepAppend ap{};
+  ap.k = (const uint16_t*)k;
+  ap.v = (const uint16_t*)v;
+  ap.pb.n = (int32_t)patches.size();
+  for (int i = 0; i < ap.pb.n; ++i) {
+    ap.pb.idx[i] = patches[i].first;
+    ap.pb.val[i] = patches[i].second;
   }
   SeqBatch b{};
-  StepPages sp{};
   b.n = n_seqs;
   b.qhs = kHeadDim;
   for (int i = 0; i < n_seqs; ++i) {
@@ -893,11 +893,11 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
     b.ids[i] = sq;
     b.len[i] = c->len[sq] + 1;
     b.qoff[i] = (int32_t)((int64_t)i * g.hq * kHeadDim);
-    sp.page[i] = c->pages[sq][c->len[sq] / tb];
+    ap.sp.page[i] = c->pages[sq][c->len[sq] / tb];
   }
   Timing tm[kProfKinds];
   Timing* prof = prof_slots(c, s, tm);
-  hipError_t e = launch_append_decode(g, b, sp, pb, k, v, q, c->scores, idx_out, max_nc, fused,
+  hipError_t e = launch_append_decode(g, b, ap, q, c->scores, c->err_ws, c->idx_ws, idx_out, max_nc, fused,
                                      attend_waves(g, n_seqs), scale, out, c->partials, s, prof);
   prof_collect(c, prof);
   if (e != hipSuccess) return hip_fail(e, "append-decode launch");

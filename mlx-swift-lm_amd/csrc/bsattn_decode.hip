@@ -35,18 +35,10 @@ namespace bsattn {
 // attend (fused append)
 constexpr int kModeFused = 0, kModeGiven = 1, kModeFusedAppend = 2;
 
-// the fused append's extra arguments: the page of each entry's newest block,
-// metadata words to patch for the launches that follow, and the new tokens'
-// keys and values ([n][Hkv][128])
-struct AppendArgs {
-  StepPages sp;
-  PatchBatch pb;
-  const uint16_t* k;
-  const uint16_t* v;
-};
+// the fused append's extra arguments
 struct NoAppend {};
 template <int MODE>
-using ModeArgs = std::conditional_t<MODE == kModeFusedAppend, AppendArgs, NoAppend>;
+using ModeArgs = std::conditional_t<MODE == kModeFusedAppend, StepAppend, NoAppend>;
 
 // candidate blocks of a pair the fused kernel scores and selects from
 constexpr int kFusedMaxCand = 2048;
@@ -586,11 +578,9 @@ hipError_t launch_fused_decode(const Geometry& g, const SeqBatch& b, int nseq, c
   return decode_impl<kModeFused>(g, b, nseq, q, idx_out, len_first, scale, out, partials, NoAppend{}, s, prof);
 }
 
-hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepPages& sp,
-                                      const PatchBatch& pb, const void* k, const void* v, const void* q,
-                                      int32_t* idx_out, float scale, void* out, float* partials,
+hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap,
+                                      const void* q, int32_t* idx_out, float scale, void* out, float* partials,
                                       hipStream_t s, Timing* prof) {
-  const AppendArgs ap{sp, pb, (const uint16_t*)k, (const uint16_t*)v};
   return decode_impl<kModeFusedAppend>(g, b, b.n, q, idx_out, true, scale, out, partials, ap, s, prof);
 }
 

@@ -91,6 +91,16 @@ struct StepPages {
   int32_t page[kMaxBatch];
 };
 
+// A decode step's append, run inside another launch (the fused decode, or the
+// scoring): the pages, the metadata words to patch for the launches that
+// follow, and the new tokens' keys and values ([n][Hkv][128])
+struct StepAppend {
+  StepPages sp;
+  PatchBatch pb;
+  const uint16_t* k;
+  const uint16_t* v;
+};
+
 // Opt-in per-kernel profiling: a launcher given a Timing array records the
 // start/stop events of slot `kind` around that kernel's dispatch (when the
 // slot's events are set) and marks the slot used.
@@ -137,14 +147,17 @@ int candidates(const Geometry& g, int len);
 // scoring + top-K for a batch whose largest candidate count is max_nc;
 // err: bound and floor workspace of 2 * mfma_err_stride(g) floats per
 // (sequence, kv head)
+// ap (not null): the scoring launch also appends one token per entry (b.len
+// = the lengths after it)
 hipError_t launch_select(const Geometry& g, const SeqBatch& b, const void* q, float* scores,
-                         float* err, int32_t* idx, int max_nc, hipStream_t s, Timing* prof);
+                         float* err, int32_t* idx, int max_nc, hipStream_t s, Timing* prof,
+                         const StepAppend* ap = nullptr);
 int mfma_err_stride(const Geometry& g);
 // block-wide selection (bsattn_select.hip); scores_ready: exact scores are
 // in `scores`, else (group >= 8) MFMA scores with the band rescored exactly
 hipError_t launch_select_large(const Geometry& g, const SeqBatch& b, const void* q, float* scores,
                                float* err, int max_nc, int32_t* idx, hipStream_t s, Timing* prof,
-                               bool scores_ready);
+                               bool scores_ready, const StepAppend* ap);
 // Waves per attention workgroup (kWaves or kWavesWide) for one call over
 // nseq sequences, from the geometry and nseq alone.  Every launch of a call
 // takes the same count, and calls that must agree bit for bit (decode and
@@ -165,18 +178,17 @@ hipError_t launch_decode(const Geometry& g, const SeqBatch& b, const void* q, fl
 hipError_t launch_decode_attend(const Geometry& g, const SeqBatch& b, const void* q, float* scores,
                                 int32_t* idx_out, int max_nc, int waves, float scale, void* out,
                                 float* partials, hipStream_t s, Timing* prof);
-// one decode step of a 16-bit cache with one new token per entry (b.len =
-// the lengths after it): fused (requires fused_decode_ok): one launch of the
-// fused decode kernel that also applies the patches pb and the appends (k / v
-// [n, Hkv, 1, D] into the pages sp), plus the combine when it splits;
-// otherwise the patches, the appends and the scoring in one launch, then the
-// selection + attention (+ combine) launches of launch_decode (requires
-// max_nc <= fused_select_limit(top_k)).  Every cache has recent
-// >= 1, so the block an append completes is forced, never scored.
-hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepPages& sp,
-                                const PatchBatch& pb, const void* k, const void* v, const void* q,
-                                float* scores, int32_t* idx_out, int max_nc, bool fused, int waves,
-                                float scale, void* out, float* partials, hipStream_t s, Timing* prof);
+// one decode step with one new token per entry (b.len = the lengths after
+// it): fused (requires fused_decode_ok): one launch of the fused decode
+// kernel that also applies the step's patches and appends, plus the combine
+// when it splits; otherwise the patches, the appends and the scoring in one
+// launch, then the launches of the decode that follow its scoring (idx: where
+// a separate selection goes).  Every cache has recent >= 1, so the block an
+// append completes is forced, never scored.
+hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap, const void* q,
+                                float* scores, float* err, int32_t* idx, int32_t* idx_out, int max_nc,
+                                bool fused, int waves, float scale, void* out, float* partials,
+                                hipStream_t s, Timing* prof);
 // split combine of nsplit partials per (entry, q head) into out
 hipError_t launch_combine(const Geometry& g, const SeqBatch& b, const float* partials, int nsplit,
                           void* out, hipStream_t s, Timing* prof);
@@ -190,7 +202,7 @@ hipError_t launch_combine(const Geometry& g, const SeqBatch& b, const float* par
 bool fused_decode_ok(const Geometry& g, int nseq, int max_nc);
 // exact (canonical) block scores of every ranked candidate into `scores`
 hipError_t launch_score(const Geometry& g, const SeqBatch& b, const void* q, float* scores, int max_nc,
-                        hipStream_t s, Timing* prof);
+                        hipStream_t s, Timing* prof, const StepAppend* ap = nullptr);
 
 hipError_t launch_fused_decode(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
                                int32_t* idx_out, bool len_first, float scale, void* out, float* partials,
@@ -201,13 +213,12 @@ hipError_t launch_fused_decode(const Geometry& g, const SeqBatch& b, int nseq, c
 hipError_t launch_fused_attend(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
                                const int32_t* idx, float scale, void* out, float* partials, hipStream_t s,
                                Timing* prof);
-// one launch per decode step: each entry's new token (k, v: [n][Hkv][128]) is
-// stored at position b.len[i] - 1 on page sp.page[i] before the fused decode
-// gathers it, the block it fills gets its summary, and the metadata patches
-// pb are applied for the launches that follow (requires recent >= 1)
-hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepPages& sp,
-                                      const PatchBatch& pb, const void* k, const void* v, const void* q,
-                                      int32_t* idx_out, float scale, void* out, float* partials,
+// one launch per decode step: each entry's new token is stored at position
+// b.len[i] - 1 on page ap.sp.page[i] before the fused decode gathers it, the
+// block it fills gets its summary, and the metadata patches ap.pb are applied
+// for the launches that follow (requires recent >= 1)
+hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap,
+                                      const void* q, int32_t* idx_out, float scale, void* out, float* partials,
                                       hipStream_t s, Timing* prof);
 // dense causal attention of the last L tokens of each sequence.  nsplit > 1:
 // every query's tokens are split into that many parts, whose partials (ws:

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bsattn_append.h"
 #include "bsattn_device.h"
 
 namespace bsattn {
@@ -63,56 +64,6 @@ __device__ __forceinline__ void summary16(const Geometry& geo, const uint16_t* _
 // fold the block in token order from LDS, as summary16 does from memory.
 // grid (ceil(L/16), Hkv, n)
 // ---------------------------------------------------------------------------
-// Body of one append workgroup: tokens blockIdx.x * 16 .. +15 of entry bi,
-// kv head h, starting at position base.  page_given >= 0 is the page of the
-// (single) token's block, passed by a caller that patches the block table in
-// the same launch; otherwise the page is read from the block table.
-template <int DT>
-__device__ __forceinline__ void append_body(const Geometry& geo, int seq, int bi, int h, int L,
-                                            int base, int page_given,
-                                            const uint16_t* __restrict__ k,
-                                            const uint16_t* __restrict__ v, bool fuse_summary,
-                                            u32x4 (*s_blk)[16]) {
-  const int tg = threadIdx.x >> 4, c = threadIdx.x & 15;
-  const int tok = blockIdx.x * 16 + tg;
-  const int32_t* bt = block_table(geo, seq);
-  // the workgroup's token 0 (the only one) fills its block: uniform.  Then
-  // the keys of the block's other tokens (written by earlier launches) are
-  // requested first, all at once and without a branch (token indices
-  // clamped; blocks of 32 or 64 tokens: at most four keys per thread), so
-  // that they arrive with the token's own
-  const int blk0 = base / geo.tb;
-  const bool fills = fuse_summary && base - blk0 * geo.tb == geo.tb - 1;
-  u32x4 pre[4];
-  if (fills) {
-    const int page = page_given >= 0 ? page_given : bt[blk0];
-    const uint16_t* Kt =
-        (const uint16_t*)(geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes + geo.k_off);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pre[i] = *(const u32x4*)(Kt + k_elem(min(tg + 16 * i, geo.tb - 2), 8 * c));
-  }
-  u32x4 kr = u32x4{0u, 0u, 0u, 0u};
-  if (tok < L) {
-    const int pos = base + tok;
-    const int blk = pos / geo.tb, slot = pos - blk * geo.tb;
-    const int page = page_given >= 0 ? page_given : bt[blk];
-    const size_t src = (((size_t)bi * geo.hkv + h) * L + tok) * kHeadDim + 8 * c;
-    kr = *(const u32x4*)(k + src);
-    const u32x4 vr = *(const u32x4*)(v + src);
-    put_token(geo, page, h, slot, c, kr, vr);
-  }
-  if (!fills) return;
-  const int blk = blk0;
-  // keys 0 .. Tb-2 (loaded above); key Tb-1 is kr of tg 0
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    if (tg + 16 * i < geo.tb - 1) s_blk[tg + 16 * i][c] = pre[i];
-  if (tg == 0) s_blk[geo.tb - 1][c] = kr;
-  __syncthreads();
-  if (tg != 0) return;
-  *(u32x4*)(summary_row(geo, seq, h, blk) + 8 * c) = fold_block<DT>(s_blk, geo.tb, c);
-}
-
 template <int DT>
 __global__ __launch_bounds__(256) void k_append(Geometry geo, AppendBatch ab,
                                                 const uint16_t* __restrict__ k,
@@ -128,7 +79,7 @@ __global__ __launch_bounds__(256) void k_append(Geometry geo, AppendBatch ab,
     base = geo.meta[seq];
     if (base >= geo.meta[geo.cap_off + seq]) return;
   }
-  append_body<DT>(geo, seq, bi, h, ab.L, base, -1, k, v, fuse_summary, s_blk);
+  append_body<DT>(geo, seq, bi, h, ab.L, base, -1, blockIdx.x, k, v, fuse_summary, s_blk);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,26 +164,17 @@ __global__ __launch_bounds__(256) void k_score(Geometry geo, SeqBatch sb,
 // ---------------------------------------------------------------------------
 // One decode step's append and scoring in one launch (attentionWithCacheUpdate
 // with one new token per sequence): workgroups x = 0 append entry bi's token
-// to kv head h (writing the summary of the block it completes), the rest
-// score candidate chunk x - 1.  The host patches of this step (lengths,
-// capacities, table entries of new pages) are applied here by workgroup
-// (0, 0, 0) for the launches that follow; nothing in this launch reads them:
-// the append takes its position and page from the arguments, the scoring
-// takes each entry's length from sb, and the block an append completes is
-// the newest block, which is forced (recent >= 1) and never scored.
+// to kv head h (append_step_body), the rest score candidate chunk x - 1.
 // grid (chunks + 1, Hkv, n)
 // ---------------------------------------------------------------------------
 template <int DT, int G, int CH>
-__global__ __launch_bounds__(256) void k_append_score(Geometry geo, SeqBatch sb, StepPages sp,
-                                                      PatchBatch pb, const uint16_t* __restrict__ k,
-                                                      const uint16_t* __restrict__ v,
+__global__ __launch_bounds__(256) void k_append_score(Geometry geo, SeqBatch sb, StepAppend ap,
                                                       const uint16_t* __restrict__ q,
                                                       float* __restrict__ scores) {
-  __shared__ u32x4 s_blk[64][16];
+  __shared__ AppendLds lds;
   const int h = blockIdx.y, bi = blockIdx.z;
   if (blockIdx.x == 0) {
-    if (h == 0 && bi == 0 && (int)threadIdx.x < pb.n) geo.meta[pb.idx[threadIdx.x]] = pb.val[threadIdx.x];
-    append_body<DT>(geo, sb.ids[bi], bi, h, 1, sb.len[bi] - 1, sp.page[bi], k, v, true, s_blk);
+    append_step_body<DT>(geo, sb, ap, h, bi, lds);
     return;
   }
   score_body<DT, G, CH>(geo, sb, q, scores, blockIdx.x - 1, h, bi);
@@ -621,31 +563,23 @@ hipError_t launch_summary(const Geometry& g, const SummaryBatch& sb, int max_cou
   return hipGetLastError();
 }
 
-template <int DT, int CH>
-static void score_dispatch(const Geometry& g, const SeqBatch& b, int max_nc, const uint16_t* q,
-                           float* sc, hipStream_t s, Timing* prof) {
-  const dim3 grid((max_nc + CH - 1) / CH, g.hkv, b.n), blk(256);
-  switch (g.group) {
-    case 1: launch(k_score<DT, 1, CH>, grid, blk, 0, s, prof, kProfScore, g, b, q, sc); break;
-    case 2: launch(k_score<DT, 2, CH>, grid, blk, 0, s, prof, kProfScore, g, b, q, sc); break;
-    case 4: launch(k_score<DT, 4, CH>, grid, blk, 0, s, prof, kProfScore, g, b, q, sc); break;
-    case 8: launch(k_score<DT, 8, CH>, grid, blk, 0, s, prof, kProfScore, g, b, q, sc); break;
-    default: launch(k_score<DT, 16, CH>, grid, blk, 0, s, prof, kProfScore, g, b, q, sc); break;
-  }
+template <int DT, int G, int CH>
+static void score_launch(const Geometry& g, const SeqBatch& b, int chunks, const uint16_t* q, float* sc,
+                         hipStream_t s, Timing* prof, const StepAppend* ap) {
+  if (ap) launch(k_append_score<DT, G, CH>, dim3(chunks + 1, g.hkv, b.n), dim3(256), 0, s, prof, kProfScore, g, b, *ap, q, sc);
+  else launch(k_score<DT, G, CH>, dim3(chunks, g.hkv, b.n), dim3(256), 0, s, prof, kProfScore, g, b, q, sc);
 }
 
 template <int DT, int CH>
-static void append_score_dispatch(const Geometry& g, const SeqBatch& b, const StepPages& sp,
-                                  const PatchBatch& pb, int chunks, const uint16_t* k,
-                                  const uint16_t* v, const uint16_t* q, float* sc, hipStream_t s,
-                                  Timing* prof) {
-  const dim3 grid(chunks + 1, g.hkv, b.n), blk(256);
+static void score_dispatch(const Geometry& g, const SeqBatch& b, int max_nc, const uint16_t* q,
+                           float* sc, hipStream_t s, Timing* prof, const StepAppend* ap) {
+  const int chunks = ranked_select(g, max_nc) ? (max_nc + CH - 1) / CH : 0;
   switch (g.group) {
-    case 1: launch(k_append_score<DT, 1, CH>, grid, blk, 0, s, prof, kProfScore, g, b, sp, pb, k, v, q, sc); break;
-    case 2: launch(k_append_score<DT, 2, CH>, grid, blk, 0, s, prof, kProfScore, g, b, sp, pb, k, v, q, sc); break;
-    case 4: launch(k_append_score<DT, 4, CH>, grid, blk, 0, s, prof, kProfScore, g, b, sp, pb, k, v, q, sc); break;
-    case 8: launch(k_append_score<DT, 8, CH>, grid, blk, 0, s, prof, kProfScore, g, b, sp, pb, k, v, q, sc); break;
-    default: launch(k_append_score<DT, 16, CH>, grid, blk, 0, s, prof, kProfScore, g, b, sp, pb, k, v, q, sc); break;
+    case 1: score_launch<DT, 1, CH>(g, b, chunks, q, sc, s, prof, ap); break;
+    case 2: score_launch<DT, 2, CH>(g, b, chunks, q, sc, s, prof, ap); break;
+    case 4: score_launch<DT, 4, CH>(g, b, chunks, q, sc, s, prof, ap); break;
+    case 8: score_launch<DT, 8, CH>(g, b, chunks, q, sc, s, prof, ap); break;
+    default: score_launch<DT, 16, CH>(g, b, chunks, q, sc, s, prof, ap); break;
   }
 }
 
@@ -660,8 +594,8 @@ static bool wave_selectable(const Geometry& g, int max_nc) {
 
 // exact (canonical) scores of every ranked candidate
 hipError_t launch_score(const Geometry& g, const SeqBatch& b, const void* q, float* scores, int max_nc,
-                        hipStream_t s, Timing* prof) {
-  if (!ranked_select(g, max_nc)) return hipSuccess;
+                        hipStream_t s, Timing* prof, const StepAppend* ap) {
+  if (!ap && !ranked_select(g, max_nc)) return hipSuccess;
   // 32-candidate chunks while the 64-candidate grid has at most 1024
   // workgroups (8 sequences x 8 kv heads at 32k tokens: 512 -> 1024
   // workgroups, ~0.4 us faster; 4 x 8 at 131k tokens, 1024 -> 2048: 0.2 us
@@ -670,23 +604,24 @@ hipError_t launch_score(const Geometry& g, const SeqBatch& b, const void* q, flo
   const bool small = (int64_t)((max_nc + 63) / 64) * g.hkv * b.n <= 1024;
   const uint16_t* qq = (const uint16_t*)q;
   if (g.dtype == 0) {
-    if (small) score_dispatch<0, 32>(g, b, max_nc, qq, scores, s, prof);
-    else score_dispatch<0, 64>(g, b, max_nc, qq, scores, s, prof);
+    if (small) score_dispatch<0, 32>(g, b, max_nc, qq, scores, s, prof, ap);
+    else score_dispatch<0, 64>(g, b, max_nc, qq, scores, s, prof, ap);
   } else {
-    if (small) score_dispatch<1, 32>(g, b, max_nc, qq, scores, s, prof);
-    else score_dispatch<1, 64>(g, b, max_nc, qq, scores, s, prof);
+    if (small) score_dispatch<1, 32>(g, b, max_nc, qq, scores, s, prof, ap);
+    else score_dispatch<1, 64>(g, b, max_nc, qq, scores, s, prof, ap);
   }
   return hipGetLastError();
 }
 
 hipError_t launch_select(const Geometry& g, const SeqBatch& b, const void* q, float* scores,
-                         float* err, int32_t* idx, int max_nc, hipStream_t s, Timing* prof) {
+                         float* err, int32_t* idx, int max_nc, hipStream_t s, Timing* prof,
+                         const StepAppend* ap) {
   const bool small = wave_selectable(g, max_nc);
   if (!small && g.group >= 8)  // MFMA scores + exact rescoring of the band
-    return launch_select_large(g, b, q, scores, err, max_nc, idx, s, prof, false);
-  hipError_t e = launch_score(g, b, q, scores, max_nc, s, prof);
+    return launch_select_large(g, b, q, scores, err, max_nc, idx, s, prof, false, ap);
+  hipError_t e = launch_score(g, b, q, scores, max_nc, s, prof, ap);
   if (e != hipSuccess) return e;
-  if (!small) return launch_select_large(g, b, q, scores, err, max_nc, idx, s, prof, true);
+  if (!small) return launch_select_large(g, b, q, scores, err, max_nc, idx, s, prof, true, nullptr);
   launch(k_topk, dim3(g.hkv, b.n), dim3(64), 0, s, prof, kProfTopk, g, b, (const float*)scores, idx);
   return hipGetLastError();
 }
@@ -831,26 +766,20 @@ hipError_t launch_decode(const Geometry& g, const SeqBatch& b, const void* q, fl
   return launch_decode_attend(g, b, q, scores, idx_out, max_nc, waves, scale, out, partials, s, prof);
 }
 
-hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepPages& sp,
-                                const PatchBatch& pb, const void* k, const void* v, const void* q,
-                                float* scores, int32_t* idx_out, int max_nc, bool fused, int waves,
-                                float scale, void* out, float* partials, hipStream_t s, Timing* prof) {
+hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap, const void* q,
+                                float* scores, float* err, int32_t* idx, int32_t* idx_out, int max_nc,
+                                bool fused, int waves, float scale, void* out, float* partials,
+                                hipStream_t s, Timing* prof) {
   // the fused decode appends, scores and attends in one launch
-  if (fused)
-    return launch_fused_append_decode(g, b, sp, pb, k, v, q, idx_out, scale, out, partials, s, prof);
-  // the scoring chunk size follows launch_score
-  const bool small = (int64_t)((max_nc + 63) / 64) * g.hkv * b.n <= 1024;
-  const int ch = small ? 32 : 64;
-  const int chunks = ranked_select(g, max_nc) ? (max_nc + ch - 1) / ch : 0;
-  const uint16_t *kk = (const uint16_t*)k, *vv = (const uint16_t*)v, *qq = (const uint16_t*)q;
-  if (g.dtype == 0) {
-    if (small) append_score_dispatch<0, 32>(g, b, sp, pb, chunks, kk, vv, qq, scores, s, prof);
-    else append_score_dispatch<0, 64>(g, b, sp, pb, chunks, kk, vv, qq, scores, s, prof);
-  } else {
-    if (small) append_score_dispatch<1, 32>(g, b, sp, pb, chunks, kk, vv, qq, scores, s, prof);
-    else append_score_dispatch<1, 64>(g, b, sp, pb, chunks, kk, vv, qq, scores, s, prof);
+  if (fused) return launch_fused_append_decode(g, b, ap, q, idx_out, scale, out, partials, s, prof);
+  hipError_t e;
+  if (max_nc > fused_select_limit(g.top_k)) {
+    int32_t* sel = idx_out ? idx_out : idx;
+    e = launch_select(g, b, q, scores, err, sel, max_nc, s, prof, &ap);
+    if (e != hipSuccess) return e;
+    return launch_attend(g, b, q, sel, waves, scale, out, partials, s, prof);
   }
-  hipError_t e = hipGetLastError();
+  e = launch_score(g, b, q, scores, max_nc, s, prof, &ap);
   if (e != hipSuccess) return e;
   return launch_decode_attend(g, b, q, scores, idx_out, max_nc, waves, scale, out, partials, s, prof);
 }

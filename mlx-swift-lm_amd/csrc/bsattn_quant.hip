@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "bsattn_append.h"
 #include "bsattn_device.h"
 
 namespace bsattn {
@@ -34,12 +35,6 @@ namespace bsattn {
 // ---------------------------------------------------------------------------
 // helpers
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float h2f(uint32_t bits16) {
-  return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
-}
-__device__ __forceinline__ float lo_f(uint32_t w) { return h2f(w & 0xFFFFu); }
-__device__ __forceinline__ float hi_f(uint32_t w) { return h2f(w >> 16); }
-
 // Codes as the decode kernel's MFMA operands: int8 code c is the fp16
 // 1024 + c (byte_to_f16); an int4 word (element e in nibble q_nib(e)) gives
 // pairs 0 and 2 (elements 0, 1, 4, 5) as 1024 + c and pairs 1 and 3
@@ -120,61 +115,6 @@ __device__ __forceinline__ float bank_from0(float old, float src, int t) {
 }
 
 // ---------------------------------------------------------------------------
-// quantize 8 consecutive dims of one row (lane c of the 16 lanes holding the
-// row; lanes c & ~7 .. +7 hold one 64-dim group) by mlx's affine rule, in
-// fp32 with correctly rounded divisions:
-//   scale = max((max - min) / (2^b - 1), 1e-7), negated unless
-//   |min| > |max|; edge = min if |min| > |max| else max;
-//   q0 = rint(edge / scale); q0 != 0: scale = edge / q0, bias = edge;
-//   q0 == 0 (an all-zero group): bias = 0;
-//   code = clamp(rint((x - bias) / scale), 0, 2^b - 1) from the fp32 scale
-//   and bias, which are stored rounded to fp16.
-// (Signed zeros cannot matter: q0 == 0 only when edge is a zero, and then
-// bias is +0.)
-// ---------------------------------------------------------------------------
-template <int KB>
-__device__ __forceinline__ void quantize8(const uint16_t* __restrict__ src, int c, uint8_t* codes,
-                                          uint16_t* scale_out, uint16_t* bias_out) {
-  const u32x4 raw = *(const u32x4*)src;
-  float x[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = (e & 1) ? hi_f(raw[e >> 1]) : lo_f(raw[e >> 1]);
-  float mn = x[0], mx = x[0];
-#pragma unroll
-  for (int e = 1; e < 8; ++e) {
-    mn = fminf(mn, x[e]);
-    mx = fmaxf(mx, x[e]);
-  }
-#pragma unroll
-  for (int off = 1; off < 8; off <<= 1) {
-    mn = fminf(mn, __shfl_xor(mn, off, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  }
-  constexpr float nbins = (float)((1 << KB) - 1);
-  float scale = fmaxf(__fdiv_rn(__fsub_rn(mx, mn), nbins), (float)1e-7);
-  const bool side = fabsf(mn) > fabsf(mx);
-  scale = side ? scale : -scale;
-  const float edge = side ? mn : mx;
-  const float q0 = __builtin_rintf(__fdiv_rn(edge, scale));
-  float bias = 0.0f;
-  if (q0 != 0.0f) {
-    scale = __fdiv_rn(edge, q0);
-    bias = edge;
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    float qv = __builtin_rintf(__fdiv_rn(__fsub_rn(x[e], bias), scale));
-    qv = qv < 0.0f ? 0.0f : qv;
-    qv = qv > nbins ? nbins : qv;
-    codes[e] = (uint8_t)qv;
-  }
-  if ((c & 7) == 0) {
-    *scale_out = __builtin_bit_cast(uint16_t, (_Float16)scale);
-    *bias_out = __builtin_bit_cast(uint16_t, (_Float16)bias);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // append: workgroup x covers the 8-aligned positions [P0, P0 + 8),
 // P0 = 8 * (old_len / 8 + x), of one (sequence, kv head); the tokens
 // appended there are [max(P0, old), min(P0 + 8, old + L)).  Stage 1 puts
@@ -215,8 +155,19 @@ __global__ __launch_bounds__(128) void k_append_q(Geometry geo, AppendBatch ab,
       uint16_t* sbh = (uint16_t*)s_sb[i];
       if constexpr (QUANTIZE) {
         const int grp = c >> 3;
-        quantize8<KB>(k16 + row * kHeadDim + 8 * c, c, &s_kc[i][8 * c], sbh + grp, sbh + 2 + grp);
-        quantize8<KB>(v16 + row * kHeadDim + 8 * c, c, &s_vc[i][8 * c], sbh + 4 + grp, sbh + 6 + grp);
+        auto quantize = [&](const uint16_t* src, uint8_t* dst, uint16_t* sc, uint16_t* bs) {
+          uint32_t codes[8];
+          uint16_t s, b;
+          quantize8<KB>(*(const u32x4*)src, codes, s, b);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) dst[e] = (uint8_t)codes[e];
+          if ((c & 7) == 0) {
+            *sc = s;
+            *bs = b;
+          }
+        };
+        quantize(k16 + row * kHeadDim + 8 * c, &s_kc[i][8 * c], sbh + grp, sbh + 2 + grp);
+        quantize(v16 + row * kHeadDim + 8 * c, &s_vc[i][8 * c], sbh + 4 + grp, sbh + 6 + grp);
       } else {
         if constexpr (KB == 4) {
           const uint32_t a = kw[row * WPR + c], b = vw[row * WPR + c];
@@ -313,20 +264,10 @@ __global__ __launch_bounds__(128) void k_summary_q(Geometry geo, SummaryBatch sb
   const int seq = sb.seq[bi];
   const int j = sb.first[bi] + blockIdx.x;
   const int page = block_table(geo, seq)[j];
-  const int d = threadIdx.x, grp = d >> 6;
+  const int d = threadIdx.x;
   const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  const uint8_t* Kc = slab + geo.k_off;
-  const uint16_t* Sb = (const uint16_t*)(slab + geo.sb_off);
-  float acc = 0.0f;
-  for (int t = 0; t < geo.tb; ++t) {
-    int sh;
-    const int code = (Kc[kq_byte(KB, t, d, &sh)] >> sh) & ((1 << KB) - 1);
-    const uint16_t* f = Sb + 8 * sb_entry(geo.tb, t);
-    const float w = __builtin_fmaf(h2f(f[grp]), (float)code, h2f(f[2 + grp]));
-    acc = (t == 0) ? w : __fadd_rn(acc, w);
-  }
   summary_row(geo, seq, h, j)[d] =
-      __builtin_bit_cast(uint16_t, (_Float16)__fmul_rn(acc, 1.0f / (float)geo.tb));
+      fold_block_q<KB>(slab + geo.k_off, (const uint16_t*)(slab + geo.sb_off), geo.tb, d);
 }
 
 // ---------------------------------------------------------------------------

@@ -39,6 +39,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
+#include "bsattn_append.h"
 #include "bsattn_device.h"
 
 namespace bsattn {
@@ -107,19 +110,31 @@ __device__ __forceinline__ float wave_max_f32(float x) {
 // err[seq row][chunk].  The query loads are issued before the rows: loads
 // complete in issue order, so each tile's MFMAs wait only for that tile's
 // rows, and the tiles are computed while the later rows arrive.
-// grid (chunks, Hkv, n)
+// APPEND: a decode step's append and scoring in one launch; workgroups x = 0
+// append (append_step_body), the rest score chunk x - 1 (16 KiB of LDS for
+// the append leaves the four workgroups per CU that the registers allow).
+// grid (chunks [+ 1], Hkv, n)
 // ---------------------------------------------------------------------------
-template <int DT, int G>
+struct NoStep {};
+template <int DT, int G, bool APPEND>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_score_mfma(Geometry geo, SeqBatch sb,
                                                     const uint16_t* __restrict__ q,
                                                     float* __restrict__ scores,
                                                     float* __restrict__ err, int err_stride,
-                                                    int floor_rank) {
+                                                    int floor_rank,
+                                                    std::conditional_t<APPEND, StepAppend, NoStep> ap) {
+  if constexpr (APPEND) {
+    if (blockIdx.x == 0) {
+      __shared__ AppendLds lds;
+      append_step_body<DT>(geo, sb, ap, blockIdx.y, blockIdx.z, lds);
+      return;
+    }
+  }
   __shared__ float s_e[4];
   __shared__ int s_bad[4];
   __shared__ float s_tm[4 * kMfmaTiles];  // each tile's largest approximate score (-inf: no candidate)
   __shared__ float s_sc[kMfmaChunk];      // the chunk's approximate scores (-inf: no candidate)
-  const int chunk = blockIdx.x, h = blockIdx.y, bi = blockIdx.z;
+  const int chunk = blockIdx.x - APPEND, h = blockIdx.y, bi = blockIdx.z;
   const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   // (the entries of wave w are written below by the same wave)
   s_sc[threadIdx.x] = -INFINITY;
@@ -1023,27 +1038,32 @@ static void select_per(const Geometry& g, const SeqBatch& b, const uint16_t* q, 
 
 template <int DT, int G>
 static void select_wide(const Geometry& g, const SeqBatch& b, const uint16_t* q, float* scores,
-                        float* err, int max_nc, int32_t* idx, hipStream_t s, Timing* prof) {
+                        float* err, int max_nc, int32_t* idx, hipStream_t s, Timing* prof,
+                        const StepAppend* ap) {
   const int chunks = (max_nc + kMfmaChunk - 1) / kMfmaChunk;
   const int stride = mfma_err_stride(g);
   // each chunk's floor_rank-th largest score, so that the chunks hold K
   const int floor_rank = std::min(8, std::max(1, (g.top_k + chunks - 1) / chunks));
-  launch(k_score_mfma<DT, G>, dim3(chunks, g.hkv, b.n), dim3(256), 0, s, prof, kProfScore, g, b, q,
-         scores, err, stride, floor_rank);
+  if (ap)
+    launch(k_score_mfma<DT, G, true>, dim3(chunks + 1, g.hkv, b.n), dim3(256), 0, s, prof, kProfScore, g, b, q,
+           scores, err, stride, floor_rank, *ap);
+  else
+    launch(k_score_mfma<DT, G, false>, dim3(chunks, g.hkv, b.n), dim3(256), 0, s, prof, kProfScore, g, b, q,
+           scores, err, stride, floor_rank, NoStep{});
   select_per<DT, G, true>(g, b, q, scores, err, stride, chunks, floor_rank, max_nc, idx, s, prof);
 }
 
 hipError_t launch_select_large(const Geometry& g, const SeqBatch& b, const void* q, float* scores,
                                float* err, int max_nc, int32_t* idx, hipStream_t s, Timing* prof,
-                               bool scores_ready) {
+                               bool scores_ready, const StepAppend* ap) {
   const uint16_t* qq = (const uint16_t*)q;
   if (!scores_ready && g.group >= 8) {
     if (g.dtype == 0) {
-      if (g.group == 8) select_wide<0, 8>(g, b, qq, scores, err, max_nc, idx, s, prof);
-      else select_wide<0, 16>(g, b, qq, scores, err, max_nc, idx, s, prof);
+      if (g.group == 8) select_wide<0, 8>(g, b, qq, scores, err, max_nc, idx, s, prof, ap);
+      else select_wide<0, 16>(g, b, qq, scores, err, max_nc, idx, s, prof, ap);
     } else {
-      if (g.group == 8) select_wide<1, 8>(g, b, qq, scores, err, max_nc, idx, s, prof);
-      else select_wide<1, 16>(g, b, qq, scores, err, max_nc, idx, s, prof);
+      if (g.group == 8) select_wide<1, 8>(g, b, qq, scores, err, max_nc, idx, s, prof, ap);
+      else select_wide<1, 16>(g, b, qq, scores, err, max_nc, idx, s, prof, ap);
     }
     return hipGetLastError();
   }
