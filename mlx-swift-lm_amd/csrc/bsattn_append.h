@@ -13,46 +13,35 @@ __device__ __forceinline__ float h2f(uint32_t bits16) {
 __device__ __forceinline__ float lo_f(uint32_t w) { return h2f(w & 0xFFFFu); }
 __device__ __forceinline__ float hi_f(uint32_t w) { return h2f(w >> 16); }
 
-// Body of one append workgroup: tokens chunk * 16 .. +15 of entry bi,
-// kv head h, starting at position base.  page_given >= 0 is the page of the
-// (single) token's block, passed by a caller that patches the block table in
-// the same launch; otherwise the page is read from the block table.
+// One token of entry bi (row bi of k / v [n][Hkv][D]) into a 16-bit slab by a
+// 256-thread workgroup, lanes 0..15 with 8 dims each.  A token that fills its
+// block also writes the block's summary: the keys of the block's other tokens
+// (written by earlier launches) are requested first, all at once and without
+// a branch (token indices clamped; at most four keys per thread), pass
+// through LDS with the new key from the registers of the lanes that store it,
+// and 16 lanes fold them in token order.
 template <int DT>
-__device__ __forceinline__ void append_body(const Geometry& geo, int seq, int bi, int h, int L,
-                                            int base, int page_given, int chunk,
-                                            const uint16_t* __restrict__ k,
-                                            const uint16_t* __restrict__ v, bool fuse_summary,
-                                            u32x4 (*s_blk)[16]) {
+__device__ __forceinline__ void append_token(const Geometry& geo, int seq, int bi, int h, int pos, int page,
+                                             const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                             u32x4 (*s_blk)[16]) {
   const int tg = threadIdx.x >> 4, c = threadIdx.x & 15;
-  const int tok = chunk * 16 + tg;
-  const int32_t* bt = block_table(geo, seq);
-  // the workgroup's token 0 (the only one) fills its block: uniform.  Then
-  // the keys of the block's other tokens (written by earlier launches) are
-  // requested first, all at once and without a branch (token indices
-  // clamped; blocks of 32 or 64 tokens: at most four keys per thread), so
-  // that they arrive with the token's own
-  const int blk0 = base / geo.tb;
-  const bool fills = fuse_summary && base - blk0 * geo.tb == geo.tb - 1;
+  const int blk = pos / geo.tb, slot = pos - blk * geo.tb;
+  const bool fills = slot == geo.tb - 1;
   u32x4 pre[4];
   if (fills) {
-    const int page = page_given >= 0 ? page_given : bt[blk0];
     const uint16_t* Kt =
         (const uint16_t*)(geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes + geo.k_off);
 #pragma unroll
     for (int i = 0; i < 4; ++i) pre[i] = *(const u32x4*)(Kt + k_elem(min(tg + 16 * i, geo.tb - 2), 8 * c));
   }
   u32x4 kr = u32x4{0u, 0u, 0u, 0u};
-  if (tok < L) {
-    const int pos = base + tok;
-    const int blk = pos / geo.tb, slot = pos - blk * geo.tb;
-    const int page = page_given >= 0 ? page_given : bt[blk];
-    const size_t src = (((size_t)bi * geo.hkv + h) * L + tok) * kHeadDim + 8 * c;
+  if (tg == 0) {
+    const size_t src = ((size_t)bi * geo.hkv + h) * kHeadDim + 8 * c;
     kr = *(const u32x4*)(k + src);
     const u32x4 vr = *(const u32x4*)(v + src);
     put_token(geo, page, h, slot, c, kr, vr);
   }
   if (!fills) return;
-  const int blk = blk0;
   // keys 0 .. Tb-2 (loaded above); key Tb-1 is kr of tg 0
 #pragma unroll
   for (int i = 0; i < 4; ++i)
@@ -262,7 +251,7 @@ __device__ __forceinline__ void append_step_body(const Geometry& geo, const SeqB
       return;
     }
   }
-  append_body<DT>(geo, seq, bi, h, 1, pos, page, 0, ap.k, ap.v, true, lds.blk);
+  append_token<DT>(geo, seq, bi, h, pos, page, ap.k, ap.v, lds.blk);
 }
 
 }  // namespace bsattn

@@ -160,14 +160,19 @@ int seq_list(const bsattn_cache* c, const int32_t* ids, int32_t n, std::vector<i
   return BSATTN_OK;
 }
 
+PatchBatch patch_batch(const std::pair<int32_t, int32_t>* p, size_t n) {
+  PatchBatch pb{};
+  pb.n = (int32_t)n;
+  for (size_t i = 0; i < n; ++i) {
+    pb.idx[i] = p[i].first;
+    pb.val[i] = p[i].second;
+  }
+  return pb;
+}
+
 int flush_patches(bsattn_cache* c, std::vector<std::pair<int32_t, int32_t>>& p, hipStream_t s) {
   for (size_t i = 0; i < p.size(); i += kMaxPatch) {
-    PatchBatch pb{};
-    pb.n = (int32_t)std::min<size_t>(kMaxPatch, p.size() - i);
-    for (int k = 0; k < pb.n; ++k) {
-      pb.idx[k] = p[i + k].first;
-      pb.val[k] = p[i + k].second;
-    }
+    const PatchBatch pb = patch_batch(p.data() + i, std::min<size_t>(kMaxPatch, p.size() - i));
     HIP_TRY(launch_patch(c->geo, pb, s), "patch launch");
   }
   p.clear();
@@ -535,8 +540,10 @@ int bsattn_sync(bsattn_cache* c, void* stream) try {
 }
 
 // Shared append flow: reserve pages, patch lengths / block tables, then per
-// batch of sequences launch `kernels(batch, first row)` (token writes) and the
-// summaries of the blocks that become full.
+// batch of sequences launch `kernels` (token writes and, for 16-bit caches,
+// the summaries of the blocks that become full).  A 16-bit append that takes
+// one launch, with few enough patches and touched blocks for its arguments,
+// patches the metadata itself: a launch less.
 extern "C++" template <typename F>
 int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t n_tokens,
                        hipStream_t s, F kernels) {
@@ -552,12 +559,33 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   rc = reserve_pages(c, seqs, n_tokens, patches);
   if (rc) return rc;
   const int tb = c->d.block_size;
+  const bool quant = c->d.kv_bits != 0;
   for (int s_ : seqs) patches.emplace_back(s_, c->len[s_] + n_tokens);
-  rc = flush_patches(c, patches, s);
-  if (rc) return rc;
+  // first block that a sequence's append touches, and the one past the last
+  auto touched = [&](int sq) {
+    return std::make_pair(c->len[sq] / tb, (int)(((int64_t)c->len[sq] + n_tokens + tb - 1) / tb));
+  };
+  int64_t blocks = 0;
+  for (int s_ : seqs) blocks += touched(s_).second - touched(s_).first;
+  AppendPages pg{};
+  PatchBatch pb{};
+  if (!quant && n_seqs <= kMaxBatch && patches.size() <= (size_t)kMaxPatch && blocks <= kAppendPages) {
+    pb = patch_batch(patches.data(), patches.size());
+    pg.given = 1;
+    int at = 0;
+    for (int i = 0; i < n_seqs; ++i) {
+      pg.off[i] = (int16_t)at;
+      const auto [b0, b1] = touched(seqs[i]);
+      for (int b = b0; b < b1; ++b) pg.page[at++] = c->pages[seqs[i]][b];
+    }
+  } else {
+    rc = flush_patches(c, patches, s);
+    if (rc) return rc;
+  }
   for (int i0 = 0; i0 < n_seqs; i0 += kMaxBatch) {
     AppendBatch ab{};
     SummaryBatch sb{};
+    int max_blocks = 0;
     ab.n = std::min(kMaxBatch, n_seqs - i0);
     ab.L = n_tokens;
     int max_count = 0;
@@ -571,14 +599,13 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
       sb.first[i] = first;
       sb.count[i] = last - first;
       max_count = std::max(max_count, last - first);
+      max_blocks = std::max(max_blocks, touched(sq).second - first);
     }
     sb.n = ab.n;
     Timing tm[kProfKinds];
     Timing* prof = prof_slots(c, s, tm);
-    // one token into a 16-bit cache: the append kernel writes the summaries
-    const bool fused = n_tokens == 1 && c->d.kv_bits == 0;
-    hipError_t e = kernels(ab, (size_t)i0, fused, prof);
-    if (e == hipSuccess && max_count > 0 && !fused) e = launch_summary(c->geo, sb, max_count, s, prof);
+    hipError_t e = kernels(ab, pg, pb, max_blocks, (size_t)i0, prof);
+    if (e == hipSuccess && max_count > 0 && quant) e = launch_summary_q(c->geo, sb, max_count, s, prof);
     prof_collect(c, prof);
     if (e != hipSuccess) return hip_fail(e, "append launch");
   }
@@ -592,12 +619,13 @@ int bsattn_append(bsattn_cache* c, const void* k, const void* v, const int32_t* 
   hipStream_t s = (hipStream_t)stream;
   const size_t row = (size_t)c->geo.hkv * n_tokens * kHeadDim;  // elements per sequence
   const bool quant = c->d.kv_bits != 0;
-  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, size_t i0, bool fused,
+  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, const AppendPages& pg,
+                                                           const PatchBatch& pb, int blocks, size_t i0,
                                                            Timing* prof) {
     const uint16_t* kk = (const uint16_t*)k + i0 * row;
     const uint16_t* vv = (const uint16_t*)v + i0 * row;
     return quant ? launch_append_q16(c->geo, ab, kk, vv, s, prof)
-                 : launch_append(c->geo, ab, kk, vv, fused, s, prof);
+                 : launch_append(c->geo, ab, pg, pb, blocks, kk, vv, s, prof);
   });
 } catch (...) {
   return on_exception();
@@ -612,8 +640,8 @@ int bsattn_append_quantized(bsattn_cache* c, const uint32_t* k_w, const void* k_
   hipStream_t s = (hipStream_t)stream;
   const size_t rows = (size_t)c->geo.hkv * n_tokens;  // token rows per sequence
   const size_t words = kHeadDim * c->d.kv_bits / 32, groups = kHeadDim / c->d.group_size;
-  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, size_t i0, bool,
-                                                           Timing* prof) {
+  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, const AppendPages&,
+                                                           const PatchBatch&, int, size_t i0, Timing* prof) {
     const size_t wo = i0 * rows * words, go = i0 * rows * groups;
     return launch_append_quantized(c->geo, ab, k_w + wo, (const uint16_t*)k_s + go,
                                    (const uint16_t*)k_b + go, v_w + wo, (const uint16_t*)v_s + go,
@@ -880,11 +908,7 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
   StepAppend ap{};
   ap.k = (const uint16_t*)k;
   ap.v = (const uint16_t*)v;
-  ap.pb.n = (int32_t)patches.size();
-  for (int i = 0; i < ap.pb.n; ++i) {
-    ap.pb.idx[i] = patches[i].first;
-    ap.pb.val[i] = patches[i].second;
-  }
+  ap.pb = patch_batch(patches.data(), patches.size());
   SeqBatch b{};
   b.n = n_seqs;
   b.qhs = kHeadDim;

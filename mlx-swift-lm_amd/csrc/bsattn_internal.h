@@ -73,6 +73,17 @@ struct AppendBatch {
   int32_t old_len[kMaxBatch];
 };
 
+// Pages of the blocks that each entry's append touches, oldest first
+// (page[off[i]] ..): given when they fit, so that the launch can apply the
+// block table's patches itself; otherwise the kernel reads the block table.
+// 192 pages and 240 patches keep a launch's arguments under 4 KiB.
+constexpr int kAppendPages = 192;
+struct AppendPages {
+  int32_t given;
+  int16_t off[kMaxBatch];
+  int32_t page[kAppendPages];
+};
+
 struct SummaryBatch {
   int32_t n;
   int32_t seq[kMaxBatch];
@@ -119,10 +130,11 @@ hipError_t noalloc_scratch(int device, void** out);
 
 // launchers (bsattn_kernels.hip); return hipError_t of the launch
 hipError_t launch_patch(const Geometry& g, const PatchBatch& pb, hipStream_t s);
-// fuse_summary (one token per sequence): blocks completed by the append get
-// their summary from the append kernel itself (no launch_summary needed)
-hipError_t launch_append(const Geometry& g, const AppendBatch& ab, const void* k,
-                         const void* v, bool fuse_summary, hipStream_t s, Timing* prof);
+// append to a 16-bit cache, with the summaries of the blocks it completes
+// (bsattn_blocks.hip); blocks: the most blocks that an entry's append touches;
+// pb: metadata patches that the launch applies (only with pg.given)
+hipError_t launch_append(const Geometry& g, const AppendBatch& ab, const AppendPages& pg, const PatchBatch& pb,
+                         int blocks, const void* k, const void* v, hipStream_t s, Timing* prof);
 // quantized caches (bsattn_quant.hip): append from fp16 (quantize on append)
 // or from the MLX layout; block summaries of dequantized keys; attention
 // one token per listed sequence at its device-side length, then the lengths
@@ -140,8 +152,6 @@ hipError_t launch_summary_q(const Geometry& g, const SummaryBatch& sb, int max_c
 hipError_t launch_attend_q(const Geometry& g, const SeqBatch& b, const void* q, int32_t* idx,
                            const float* scores, int sel_mode, int waves, float sl2, void* out,
                            float* partials, hipStream_t s, Timing* prof);
-hipError_t launch_summary(const Geometry& g, const SummaryBatch& sb, int max_count,
-                          hipStream_t s, Timing* prof);
 // candidate blocks (neither sink nor recent) of a sequence of `len` tokens
 int candidates(const Geometry& g, int len);
 // scoring + top-K for a batch whose largest candidate count is max_nc;

@@ -1,6 +1,6 @@
 // bsattn_kernels.hip -- gfx950 (CDNA4) kernels of the block-sparse decode
-// path: append, block summary, block scoring, top-K select, gathered
-// split-K attention and the split combine.
+// path: one-token append, block scoring, top-K select, gathered split-K
+// attention and the split combine.
 //
 // Page slab layout (one slab per (physical page, kv head), Tb tokens): the
 // K and V tiles are stored in MFMA-fragment-major order, i.e. as the
@@ -30,74 +30,19 @@ __global__ __launch_bounds__(256) void k_patch(int32_t* meta, PatchBatch pb) {
 }
 
 // ---------------------------------------------------------------------------
-// block summary of one (block, kv head) by the 16 lanes that own its dims
-// 8c .. 8c+7: sequential fp32 fold over the block's tokens from token 0,
-// times 1/Tb, rounded to the cache dtype.  Each lane reads 16 contiguous
-// bytes per token (its chunk of the fragment-major K tile).
+// append of one token per sequence at its device-side length (a sequence
+// without a reserved page for it takes nothing).  grid (Hkv, n)
 // ---------------------------------------------------------------------------
 template <int DT>
-__device__ __forceinline__ void summary16(const Geometry& geo, const uint16_t* __restrict__ Kt, int c,
-                                          uint16_t* __restrict__ dst) {
-  float acc[8];
-  unpack8<DT>(*(const u32x4*)(Kt + k_elem(0, 8 * c)), acc);
-#pragma unroll 8
-  for (int t = 1; t < geo.tb; ++t) {
-    float x[8];
-    unpack8<DT>(*(const u32x4*)(Kt + k_elem(t, 8 * c)), x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = __fadd_rn(acc[e], x[e]);
-  }
-  const float inv = 1.0f / (float)geo.tb;
-  u32x4 o;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = pack2<DT>(__fmul_rn(acc[2 * e], inv), __fmul_rn(acc[2 * e + 1], inv));
-  *(u32x4*)(dst + 8 * c) = o;
-}
-
-// ---------------------------------------------------------------------------
-// append: 16 tokens x 16 lanes (8 dims each) per workgroup.  With
-// fuse_summary (one token per sequence: the workgroup's token 0), a token
-// that fills its block also writes the block's summary: the whole workgroup
-// loads the block's other keys into LDS in one round of loads (the new key
-// comes from the registers of the lanes that wrote it), and its 16 lanes then
-// fold the block in token order from LDS, as summary16 does from memory.
-// grid (ceil(L/16), Hkv, n)
-// ---------------------------------------------------------------------------
-template <int DT>
-__global__ __launch_bounds__(256) void k_append(Geometry geo, AppendBatch ab,
-                                                const uint16_t* __restrict__ k,
-                                                const uint16_t* __restrict__ v, bool fuse_summary,
-                                                bool device_len) {
+__global__ __launch_bounds__(256) void k_append_step(Geometry geo, AppendBatch ab,
+                                                     const uint16_t* __restrict__ k,
+                                                     const uint16_t* __restrict__ v) {
   __shared__ u32x4 s_blk[64][16];  // the filled block's keys, [token][8-dim chunk]
-  const int bi = blockIdx.z, h = blockIdx.y;
+  const int h = blockIdx.x, bi = blockIdx.y;
   const int seq = ab.seq[bi];
-  // device_len: the position is the device-side length (one token; a
-  // sequence without a reserved page for it takes nothing)
-  int base = ab.old_len[bi];
-  if (device_len) {
-    base = geo.meta[seq];
-    if (base >= geo.meta[geo.cap_off + seq]) return;
-  }
-  append_body<DT>(geo, seq, bi, h, ab.L, base, -1, blockIdx.x, k, v, fuse_summary, s_blk);
-}
-
-// ---------------------------------------------------------------------------
-// block summaries of the blocks completed by an append: 4 (block, kv head)
-// pairs per 64-thread workgroup, 16 lanes each.  Summaries are stored by
-// logical block: summ[seq][kv head][block][D].
-// grid (max_count, ceil(Hkv / 4), n)
-// ---------------------------------------------------------------------------
-template <int DT>
-__global__ __launch_bounds__(64) void k_summary(Geometry geo, SummaryBatch sb) {
-  const int bi = blockIdx.z;
-  const int h = blockIdx.y * 4 + (threadIdx.x >> 4), c = threadIdx.x & 15;
-  if ((int)blockIdx.x >= sb.count[bi] || h >= geo.hkv) return;
-  const int seq = sb.seq[bi];
-  const int j = sb.first[bi] + blockIdx.x;
-  const int page = block_table(geo, seq)[j];
-  const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  summary16<DT>(geo, (const uint16_t*)(slab + geo.k_off), c, summary_row(geo, seq, h, j));
+  const int pos = geo.meta[seq];
+  if (pos >= geo.meta[geo.cap_off + seq]) return;
+  append_token<DT>(geo, seq, bi, h, pos, block_table(geo, seq)[pos / geo.tb], k, v, s_blk);
 }
 
 // ---------------------------------------------------------------------------
@@ -482,30 +427,6 @@ __global__ __launch_bounds__(128) void k_combine_r(Geometry geo, SeqBatch sb,
 }
 
 // ---------------------------------------------------------------------------
-// export: pages -> [n, Hkv, T, D]; grid (ceil(T/16), Hkv, n)
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_export(Geometry geo, SeqBatch sb, int T,
-                                                uint16_t* __restrict__ ko,
-                                                uint16_t* __restrict__ vo) {
-  const int bi = blockIdx.z, h = blockIdx.y;
-  const int tok = blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int c = threadIdx.x & 15;
-  if (tok >= T) return;
-  const int seq = sb.ids[bi];
-  const int blk = tok / geo.tb, slot = tok - blk * geo.tb;
-  const int page = block_table(geo, seq)[blk];
-  const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  const size_t dst = (((size_t)bi * geo.hkv + h) * T + tok) * kHeadDim + 8 * c;
-  *(u32x4*)(ko + dst) = *(const u32x4*)((const uint16_t*)(slab + geo.k_off) + k_elem(slot, 8 * c));
-  const uint16_t* Vt = (const uint16_t*)(slab + geo.v_off);
-  u32x4 w;
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    w[e] = (uint32_t)Vt[v_elem(geo.tb, slot, 8 * c + 2 * e)] |
-           ((uint32_t)Vt[v_elem(geo.tb, slot, 8 * c + 2 * e + 1)] << 16);
-  *(u32x4*)(vo + dst) = w;
-}
-
 // summaries of one sequence -> [Hkv, nfull, D]; grid (nfull, Hkv)
 __global__ __launch_bounds__(128) void k_export_summaries(Geometry geo, int seq, int nfull,
                                                           uint16_t* __restrict__ out) {
@@ -521,17 +442,8 @@ hipError_t launch_patch(const Geometry& g, const PatchBatch& pb, hipStream_t s) 
   return hipGetLastError();
 }
 
-hipError_t launch_append(const Geometry& g, const AppendBatch& ab, const void* k, const void* v,
-                         bool fuse_summary, hipStream_t s, Timing* prof) {
-  dim3 grid((ab.L + 15) / 16, g.hkv, ab.n);
-  const uint16_t *kk = (const uint16_t*)k, *vv = (const uint16_t*)v;
-  if (g.dtype == 0) launch(k_append<0>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv, fuse_summary, false);
-  else launch(k_append<1>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv, fuse_summary, false);
-  return hipGetLastError();
-}
-
 // advances the device-side length of each listed sequence by one token when
-// a reserved page held it (after k_append's device-length step)
+// a reserved page held it (after k_append_step)
 __global__ __launch_bounds__(64) void k_advance(Geometry geo, AppendBatch ab) {
   for (int i = threadIdx.x; i < ab.n; i += 64) {
     const int seq = ab.seq[i];
@@ -542,24 +454,13 @@ __global__ __launch_bounds__(64) void k_advance(Geometry geo, AppendBatch ab) {
 
 hipError_t launch_append_step(const Geometry& g, const AppendBatch& ab, const void* k, const void* v,
                               hipStream_t s, Timing* prof) {
-  dim3 grid(1, g.hkv, ab.n);
+  const dim3 grid(g.hkv, ab.n);
   const uint16_t *kk = (const uint16_t*)k, *vv = (const uint16_t*)v;
-  if (g.dtype == 0) launch(k_append<0>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv, true, true);
-  else launch(k_append<1>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv, true, true);
+  if (g.dtype == 0) launch(k_append_step<0>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv);
+  else launch(k_append_step<1>, grid, dim3(256), 0, s, prof, kProfAppend, g, ab, kk, vv);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, g, ab);
-  return hipGetLastError();
-}
-
-hipError_t launch_summary(const Geometry& g, const SummaryBatch& sb, int max_count,
-                          hipStream_t s, Timing* prof) {
-  if (g.kv_bits != 0) return launch_summary_q(g, sb, max_count, s, prof);
-  dim3 grid(max_count, (g.hkv + 3) / 4, sb.n);
-  if (g.dtype == 0)
-    launch(k_summary<0>, grid, dim3(64), 0, s, prof, kProfSummary, g, sb);
-  else
-    launch(k_summary<1>, grid, dim3(64), 0, s, prof, kProfSummary, g, sb);
   return hipGetLastError();
 }
 
@@ -782,13 +683,6 @@ hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const Step
   e = launch_score(g, b, q, scores, max_nc, s, prof, &ap);
   if (e != hipSuccess) return e;
   return launch_decode_attend(g, b, q, scores, idx_out, max_nc, waves, scale, out, partials, s, prof);
-}
-
-hipError_t launch_export(const Geometry& g, const SeqBatch& b, int T, void* k_out, void* v_out,
-                         hipStream_t s) {
-  dim3 grid((T + 15) / 16, g.hkv, b.n);
-  hipLaunchKernelGGL(k_export, grid, dim3(256), 0, s, g, b, T, (uint16_t*)k_out, (uint16_t*)v_out);
-  return hipGetLastError();
 }
 
 hipError_t launch_export_summaries(const Geometry& g, int seq, int nfull, void* out,
