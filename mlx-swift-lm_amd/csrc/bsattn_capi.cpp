@@ -540,10 +540,10 @@ int bsattn_sync(bsattn_cache* c, void* stream) try {
 }
 
 // Shared append flow: reserve pages, patch lengths / block tables, then per
-// batch of sequences launch `kernels` (token writes and, for 16-bit caches,
-// the summaries of the blocks that become full).  A 16-bit append that takes
-// one launch, with few enough patches and touched blocks for its arguments,
-// patches the metadata itself: a launch less.
+// batch of sequences launch `kernels` (token writes and the summaries of the
+// blocks that become full).  An append that takes one launch, with few enough
+// patches and touched blocks for its arguments, patches the metadata itself: a
+// launch less.
 extern "C++" template <typename F>
 int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t n_tokens,
                        hipStream_t s, F kernels) {
@@ -559,7 +559,6 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   rc = reserve_pages(c, seqs, n_tokens, patches);
   if (rc) return rc;
   const int tb = c->d.block_size;
-  const bool quant = c->d.kv_bits != 0;
   for (int s_ : seqs) patches.emplace_back(s_, c->len[s_] + n_tokens);
   // first block that a sequence's append touches, and the one past the last
   auto touched = [&](int sq) {
@@ -569,7 +568,7 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   for (int s_ : seqs) blocks += touched(s_).second - touched(s_).first;
   AppendPages pg{};
   PatchBatch pb{};
-  if (!quant && n_seqs <= kMaxBatch && patches.size() <= (size_t)kMaxPatch && blocks <= kAppendPages) {
+  if (n_seqs <= kMaxBatch && patches.size() <= (size_t)kMaxPatch && blocks <= kAppendPages) {
     pb = patch_batch(patches.data(), patches.size());
     pg.given = 1;
     int at = 0;
@@ -584,28 +583,18 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   }
   for (int i0 = 0; i0 < n_seqs; i0 += kMaxBatch) {
     AppendBatch ab{};
-    SummaryBatch sb{};
     int max_blocks = 0;
     ab.n = std::min(kMaxBatch, n_seqs - i0);
     ab.L = n_tokens;
-    int max_count = 0;
     for (int i = 0; i < ab.n; ++i) {
       const int sq = seqs[i0 + i];
       ab.seq[i] = sq;
       ab.old_len[i] = c->len[sq];
-      const int first = c->len[sq] / tb;
-      const int last = (c->len[sq] + n_tokens) / tb;  // exclusive: full blocks after
-      sb.seq[i] = sq;
-      sb.first[i] = first;
-      sb.count[i] = last - first;
-      max_count = std::max(max_count, last - first);
-      max_blocks = std::max(max_blocks, touched(sq).second - first);
+      max_blocks = std::max(max_blocks, touched(sq).second - touched(sq).first);
     }
-    sb.n = ab.n;
     Timing tm[kProfKinds];
     Timing* prof = prof_slots(c, s, tm);
     hipError_t e = kernels(ab, pg, pb, max_blocks, (size_t)i0, prof);
-    if (e == hipSuccess && max_count > 0 && quant) e = launch_summary_q(c->geo, sb, max_count, s, prof);
     prof_collect(c, prof);
     if (e != hipSuccess) return hip_fail(e, "append launch");
   }
@@ -624,7 +613,7 @@ int bsattn_append(bsattn_cache* c, const void* k, const void* v, const int32_t* 
                                                            Timing* prof) {
     const uint16_t* kk = (const uint16_t*)k + i0 * row;
     const uint16_t* vv = (const uint16_t*)v + i0 * row;
-    return quant ? launch_append_q16(c->geo, ab, kk, vv, s, prof)
+    return quant ? launch_append_q16(c->geo, ab, pg, pb, blocks, kk, vv, s, prof)
                  : launch_append(c->geo, ab, pg, pb, blocks, kk, vv, s, prof);
   });
 } catch (...) {
@@ -640,10 +629,11 @@ int bsattn_append_quantized(bsattn_cache* c, const uint32_t* k_w, const void* k_
   hipStream_t s = (hipStream_t)stream;
   const size_t rows = (size_t)c->geo.hkv * n_tokens;  // token rows per sequence
   const size_t words = kHeadDim * c->d.kv_bits / 32, groups = kHeadDim / c->d.group_size;
-  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, const AppendPages&,
-                                                           const PatchBatch&, int, size_t i0, Timing* prof) {
+  return append_impl(c, seq_ids, n_seqs, n_tokens, s, [&](const AppendBatch& ab, const AppendPages& pg,
+                                                           const PatchBatch& pb, int blocks, size_t i0,
+                                                           Timing* prof) {
     const size_t wo = i0 * rows * words, go = i0 * rows * groups;
-    return launch_append_quantized(c->geo, ab, k_w + wo, (const uint16_t*)k_s + go,
+    return launch_append_quantized(c->geo, ab, pg, pb, blocks, k_w + wo, (const uint16_t*)k_s + go,
                                    (const uint16_t*)k_b + go, v_w + wo, (const uint16_t*)v_s + go,
                                    (const uint16_t*)v_b + go, s, prof);
   });

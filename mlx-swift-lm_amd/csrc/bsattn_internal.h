@@ -84,13 +84,6 @@ struct AppendPages {
   int32_t page[kAppendPages];
 };
 
-struct SummaryBatch {
-  int32_t n;
-  int32_t seq[kMaxBatch];
-  int32_t first[kMaxBatch];
-  int32_t count[kMaxBatch];
-};
-
 struct PatchBatch {
   int32_t n;
   int32_t idx[kMaxPatch];
@@ -130,25 +123,24 @@ hipError_t noalloc_scratch(int device, void** out);
 
 // launchers (bsattn_kernels.hip); return hipError_t of the launch
 hipError_t launch_patch(const Geometry& g, const PatchBatch& pb, hipStream_t s);
-// append to a 16-bit cache, with the summaries of the blocks it completes
-// (bsattn_blocks.hip); blocks: the most blocks that an entry's append touches;
-// pb: metadata patches that the launch applies (only with pg.given)
+// appends of many tokens, with the summaries of the blocks they complete
+// (bsattn_blocks.hip), to a 16-bit cache; to a quantized one from fp16
+// (quantize on append) or from the MLX layout.  blocks: the most blocks that
+// an entry's append touches; pb: metadata patches that the launch applies
+// (only with pg.given)
 hipError_t launch_append(const Geometry& g, const AppendBatch& ab, const AppendPages& pg, const PatchBatch& pb,
                          int blocks, const void* k, const void* v, hipStream_t s, Timing* prof);
-// quantized caches (bsattn_quant.hip): append from fp16 (quantize on append)
-// or from the MLX layout; block summaries of dequantized keys; attention
+hipError_t launch_append_q16(const Geometry& g, const AppendBatch& ab, const AppendPages& pg, const PatchBatch& pb,
+                             int blocks, const void* k, const void* v, hipStream_t s, Timing* prof);
+hipError_t launch_append_quantized(const Geometry& g, const AppendBatch& ab, const AppendPages& pg,
+                                   const PatchBatch& pb, int blocks, const uint32_t* kw, const void* ks,
+                                   const void* kb, const uint32_t* vw, const void* vs, const void* vb,
+                                   hipStream_t s, Timing* prof);
 // one token per listed sequence at its device-side length, then the lengths
 // advanced (no host bookkeeping: capturable in a HIP graph)
 hipError_t launch_append_step(const Geometry& g, const AppendBatch& ab, const void* k, const void* v,
                               hipStream_t s, Timing* prof);
-hipError_t launch_append_q16(const Geometry& g, const AppendBatch& ab, const void* k,
-                             const void* v, hipStream_t s, Timing* prof);
-hipError_t launch_append_quantized(const Geometry& g, const AppendBatch& ab,
-                                   const uint32_t* kw, const void* ks, const void* kb,
-                                   const uint32_t* vw, const void* vs, const void* vb,
-                                   hipStream_t s, Timing* prof);
-hipError_t launch_summary_q(const Geometry& g, const SummaryBatch& sb, int max_count,
-                            hipStream_t s, Timing* prof);
+// attention over a quantized cache (bsattn_quant.hip)
 hipError_t launch_attend_q(const Geometry& g, const SeqBatch& b, const void* q, int32_t* idx,
                            const float* scores, int sel_mode, int waves, float sl2, void* out,
                            float* partials, hipStream_t s, Timing* prof);

@@ -115,162 +115,6 @@ __device__ __forceinline__ float bank_from0(float old, float src, int t) {
 }
 
 // ---------------------------------------------------------------------------
-// append: workgroup x covers the 8-aligned positions [P0, P0 + 8),
-// P0 = 8 * (old_len / 8 + x), of one (sequence, kv head); the tokens
-// appended there are [max(P0, old), min(P0 + 8, old + L)).  Stage 1 puts
-// their codes and scales / biases in LDS (quantizing fp16 input, or
-// unpacking the MLX layout: element i of a row in word i / (32/b), bits
-// b * (i % (32/b)) up, LSB first; scales / biases [.., D / 64]); stage 2
-// writes whole 32-bit words: K words belong to one token, a V word to one dim
-// and the 8 (int4) or 4 (int8) tokens of this group, merged with the codes
-// already there when the group is only partly new.
-// grid (L / 8 + 2, Hkv, n), 128 threads
-// ---------------------------------------------------------------------------
-template <int KB, bool QUANTIZE>
-__global__ __launch_bounds__(128) void k_append_q(Geometry geo, AppendBatch ab,
-                                                  const uint16_t* __restrict__ k16,
-                                                  const uint16_t* __restrict__ v16,
-                                                  const uint32_t* __restrict__ kw,
-                                                  const uint16_t* __restrict__ ks,
-                                                  const uint16_t* __restrict__ kb,
-                                                  const uint32_t* __restrict__ vw,
-                                                  const uint16_t* __restrict__ vs,
-                                                  const uint16_t* __restrict__ vb) {
-  constexpr int WPR = QCode<KB>::WPR;
-  __shared__ uint8_t s_kc[8][kHeadDim];
-  __shared__ uint8_t s_vc[8][kHeadDim];
-  __shared__ uint32_t s_sb[8][4];
-  const int bi = blockIdx.z, h = blockIdx.y;
-  const int old = ab.old_len[bi], L = ab.L;
-  const int P0 = 8 * (old / 8 + (int)blockIdx.x);
-  const int lo = max(P0, old), hi = min(P0 + 8, old + L);
-  if (lo >= hi) return;
-  const int seq = ab.seq[bi];
-  const int tid = threadIdx.x;
-  {
-    const int i = tid >> 4, c = tid & 15;  // token P0 + i, dims 8c .. 8c+7
-    const int pos = P0 + i;
-    if (pos >= lo && pos < hi) {
-      const size_t row = ((size_t)bi * geo.hkv + h) * L + (pos - old);
-      uint16_t* sbh = (uint16_t*)s_sb[i];
-      if constexpr (QUANTIZE) {
-        const int grp = c >> 3;
-        auto quantize = [&](const uint16_t* src, uint8_t* dst, uint16_t* sc, uint16_t* bs) {
-          uint32_t codes[8];
-          uint16_t s, b;
-          quantize8<KB>(*(const u32x4*)src, codes, s, b);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) dst[e] = (uint8_t)codes[e];
-          if ((c & 7) == 0) {
-            *sc = s;
-            *bs = b;
-          }
-        };
-        quantize(k16 + row * kHeadDim + 8 * c, &s_kc[i][8 * c], sbh + grp, sbh + 2 + grp);
-        quantize(v16 + row * kHeadDim + 8 * c, &s_vc[i][8 * c], sbh + 4 + grp, sbh + 6 + grp);
-      } else {
-        if constexpr (KB == 4) {
-          const uint32_t a = kw[row * WPR + c], b = vw[row * WPR + c];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            s_kc[i][8 * c + e] = (uint8_t)((a >> (4 * e)) & 15u);
-            s_vc[i][8 * c + e] = (uint8_t)((b >> (4 * e)) & 15u);
-          }
-        } else {
-#pragma unroll
-          for (int w = 0; w < 2; ++w) {
-            const uint32_t a = kw[row * WPR + 2 * c + w], b = vw[row * WPR + 2 * c + w];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              s_kc[i][8 * c + 4 * w + e] = (uint8_t)(a >> (8 * e));
-              s_vc[i][8 * c + 4 * w + e] = (uint8_t)(b >> (8 * e));
-            }
-          }
-        }
-        if (c < 2) {
-          sbh[c] = ks[row * 2 + c];
-          sbh[2 + c] = kb[row * 2 + c];
-          sbh[4 + c] = vs[row * 2 + c];
-          sbh[6 + c] = vb[row * 2 + c];
-        }
-      }
-    }
-  }
-  __syncthreads();
-  const int blk = P0 / geo.tb, slot0 = P0 - blk * geo.tb;
-  const int page = block_table(geo, seq)[blk];
-  uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  uint8_t* Kc = slab + geo.k_off;
-  uint8_t* Vc = slab + geo.v_off;
-  // K: 8 tokens x WPR words
-  for (int u = tid; u < 8 * WPR; u += 128) {
-    const int i = u / WPR, wd = u - i * WPR;
-    const int pos = P0 + i;
-    if (pos < lo || pos >= hi) continue;
-    int sh;
-    uint32_t word = 0u;
-    if constexpr (KB == 4) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) word |= (uint32_t)s_kc[i][8 * wd + e] << (4 * q_nib(e));
-      *(uint32_t*)(Kc + kq_byte(4, slot0 + i, 8 * wd, &sh)) = word;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) word |= (uint32_t)s_kc[i][4 * wd + e] << (8 * e);
-      *(uint32_t*)(Kc + kq_byte(8, slot0 + i, 4 * wd, &sh)) = word;
-    }
-  }
-  // V: thread = dim; words of this group's tokens
-  {
-    const int d = tid;
-    constexpr int TPW = 32 / KB;  // tokens per word
-#pragma unroll
-    for (int w = 0; w < 8 / TPW; ++w) {
-      const int t0 = P0 + w * TPW;
-      if (t0 + TPW <= lo || t0 >= hi) continue;
-      int sh;
-      uint32_t* dst = (uint32_t*)(Vc + vq_byte(KB, geo.tb, slot0 + w * TPW, d, &sh));
-      const bool whole = t0 >= lo && t0 + TPW <= hi;
-      uint32_t word = whole ? 0u : *dst;
-#pragma unroll
-      for (int e = 0; e < TPW; ++e) {
-        const int pos = t0 + e;
-        if (pos < lo || pos >= hi) continue;
-        const int at = KB == 4 ? 4 * q_nib(e) : 8 * e;
-        const uint32_t mask = ((1u << KB) - 1u) << at;
-        word = (word & ~mask) | ((uint32_t)s_vc[pos - P0][d] << at);
-      }
-      *dst = word;
-    }
-  }
-  // scales / biases: 16 B per token
-  if (tid < 8) {
-    const int pos = P0 + tid;
-    if (pos >= lo && pos < hi) {
-      u32x4* dst = (u32x4*)(slab + geo.sb_off) + sb_entry(geo.tb, slot0 + tid);
-      *dst = u32x4{s_sb[tid][0], s_sb[tid][1], s_sb[tid][2], s_sb[tid][3]};
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// block summary of a quantized block: thread per dim, sequential fp32 fold
-// of the dequantized keys fmaf(scale, code, bias) from token 0, times 1/Tb,
-// to fp16.  grid (max_count, Hkv, n)
-// ---------------------------------------------------------------------------
-template <int KB>
-__global__ __launch_bounds__(128) void k_summary_q(Geometry geo, SummaryBatch sb) {
-  const int bi = blockIdx.z, h = blockIdx.y;
-  if ((int)blockIdx.x >= sb.count[bi]) return;
-  const int seq = sb.seq[bi];
-  const int j = sb.first[bi] + blockIdx.x;
-  const int page = block_table(geo, seq)[j];
-  const int d = threadIdx.x;
-  const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  summary_row(geo, seq, h, j)[d] =
-      fold_block_q<KB>(slab + geo.k_off, (const uint16_t*)(slab + geo.sb_off), geo.tb, d);
-}
-
-// ---------------------------------------------------------------------------
 // gathered attention over quantized blocks: the 16-bit kernel's structure
 // (one block per wave, W waves per workgroup, selection fused when SEL,
 // split partials merged by k_combine), with the dequantisation folded into
@@ -618,90 +462,9 @@ __global__ __launch_bounds__(64 * W, W > 4 ? (G > 8 && SEL == 0 ? 2 : 1) : G > 4
   }
 }
 
-// ---------------------------------------------------------------------------
-// export in the MLX layout: kw / vw [n, Hkv, T, D*b/32] uint32 (LSB first),
-// scales / biases [n, Hkv, T, D/64] fp16.  grid (ceil(T/16), Hkv, n)
-// ---------------------------------------------------------------------------
-template <int KB>
-__global__ __launch_bounds__(256) void k_export_q(Geometry geo, SeqBatch sb, int T,
-                                                  uint32_t* __restrict__ kw, uint16_t* __restrict__ ks,
-                                                  uint16_t* __restrict__ kb, uint32_t* __restrict__ vw,
-                                                  uint16_t* __restrict__ vs, uint16_t* __restrict__ vb) {
-  constexpr int WPR = QCode<KB>::WPR;
-  constexpr int EPW = 32 / KB;  // elements per MLX word
-  const int bi = blockIdx.z, h = blockIdx.y;
-  const int tok = blockIdx.x * 16 + (threadIdx.x >> 4);
-  const int c = threadIdx.x & 15;
-  if (tok >= T) return;
-  const int seq = sb.ids[bi];
-  const int blk = tok / geo.tb, slot = tok - blk * geo.tb;
-  const int page = block_table(geo, seq)[blk];
-  const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
-  const size_t row = ((size_t)bi * geo.hkv + h) * T + tok;
-  constexpr uint32_t mask = (1u << KB) - 1u;
-#pragma unroll
-  for (int w = 0; w < WPR / 16; ++w) {
-    const int wd = (WPR / 16) * c + w;
-    uint32_t a = 0u, b = 0u;
-#pragma unroll
-    for (int e = 0; e < EPW; ++e) {
-      const int d = wd * EPW + e;
-      int sh;
-      a |= ((uint32_t)(slab[geo.k_off + kq_byte(KB, slot, d, &sh)] >> sh) & mask) << (KB * e);
-      b |= ((uint32_t)(slab[geo.v_off + vq_byte(KB, geo.tb, slot, d, &sh)] >> sh) & mask) << (KB * e);
-    }
-    kw[row * WPR + wd] = a;
-    vw[row * WPR + wd] = b;
-  }
-  if (c < 2) {
-    const uint16_t* f = (const uint16_t*)(slab + geo.sb_off) + 8 * sb_entry(geo.tb, slot);
-    ks[row * 2 + c] = f[c];
-    kb[row * 2 + c] = f[2 + c];
-    vs[row * 2 + c] = f[4 + c];
-    vb[row * 2 + c] = f[6 + c];
-  }
-}
-
 // ===========================================================================
 // launchers
 // ===========================================================================
-hipError_t launch_append_q16(const Geometry& g, const AppendBatch& ab, const void* k,
-                             const void* v, hipStream_t s, Timing* prof) {
-  const dim3 grid(ab.L / 8 + 2, g.hkv, ab.n);
-  const uint16_t *k16 = (const uint16_t*)k, *v16 = (const uint16_t*)v;
-  if (g.kv_bits == 4)
-    launch(k_append_q<4, true>, grid, dim3(128), 0, s, prof, kProfAppend, g, ab, k16, v16,
-             (const uint32_t*)nullptr, (const uint16_t*)nullptr, (const uint16_t*)nullptr,
-             (const uint32_t*)nullptr, (const uint16_t*)nullptr, (const uint16_t*)nullptr);
-  else
-    launch(k_append_q<8, true>, grid, dim3(128), 0, s, prof, kProfAppend, g, ab, k16, v16,
-             (const uint32_t*)nullptr, (const uint16_t*)nullptr, (const uint16_t*)nullptr,
-             (const uint32_t*)nullptr, (const uint16_t*)nullptr, (const uint16_t*)nullptr);
-  return hipGetLastError();
-}
-
-hipError_t launch_append_quantized(const Geometry& g, const AppendBatch& ab, const uint32_t* kw,
-                                   const void* ks, const void* kb, const uint32_t* vw,
-                                   const void* vs, const void* vb, hipStream_t s, Timing* prof) {
-  const dim3 grid(ab.L / 8 + 2, g.hkv, ab.n);
-  const uint16_t* nul = nullptr;
-  if (g.kv_bits == 4)
-    launch(k_append_q<4, false>, grid, dim3(128), 0, s, prof, kProfAppend, g, ab, nul, nul, kw,
-             (const uint16_t*)ks, (const uint16_t*)kb, vw, (const uint16_t*)vs, (const uint16_t*)vb);
-  else
-    launch(k_append_q<8, false>, grid, dim3(128), 0, s, prof, kProfAppend, g, ab, nul, nul, kw,
-             (const uint16_t*)ks, (const uint16_t*)kb, vw, (const uint16_t*)vs, (const uint16_t*)vb);
-  return hipGetLastError();
-}
-
-hipError_t launch_summary_q(const Geometry& g, const SummaryBatch& sb, int max_count,
-                            hipStream_t s, Timing* prof) {
-  const dim3 grid(max_count, g.hkv, sb.n);
-  if (g.kv_bits == 4) launch(k_summary_q<4>, grid, dim3(128), 0, s, prof, kProfSummary, g, sb);
-  else launch(k_summary_q<8>, grid, dim3(128), 0, s, prof, kProfSummary, g, sb);
-  return hipGetLastError();
-}
-
 template <int TB, int SEL, int KB>
 static void attend_q_group(const Geometry& g, int waves, dim3 grid, const SeqBatch& b, const uint16_t* q,
                            int32_t* idx, const float* sc, float sl2, uint16_t* out, float* part,
@@ -754,19 +517,6 @@ hipError_t launch_attend_q(const Geometry& g, const SeqBatch& b, const void* q, 
   if (sel_mode == 1) attend_q_sel<1>(g, waves, grid, b, qq, idx, scores, sl2, oo, partials, s, prof);
   else if (sel_mode == 2) attend_q_sel<2>(g, waves, grid, b, qq, idx, scores, sl2, oo, partials, s, prof);
   else attend_q_sel<0>(g, waves, grid, b, qq, idx, scores, sl2, oo, partials, s, prof);
-  return hipGetLastError();
-}
-
-hipError_t launch_export_quantized(const Geometry& g, const SeqBatch& b, int T, uint32_t* kw,
-                                   void* ks, void* kb, uint32_t* vw, void* vs, void* vb,
-                                   hipStream_t s) {
-  const dim3 grid((T + 15) / 16, g.hkv, b.n);
-  if (g.kv_bits == 4)
-    hipLaunchKernelGGL(k_export_q<4>, grid, dim3(256), 0, s, g, b, T, kw, (uint16_t*)ks,
-                       (uint16_t*)kb, vw, (uint16_t*)vs, (uint16_t*)vb);
-  else
-    hipLaunchKernelGGL(k_export_q<8>, grid, dim3(256), 0, s, g, b, T, kw, (uint16_t*)ks,
-                       (uint16_t*)kb, vw, (uint16_t*)vs, (uint16_t*)vb);
   return hipGetLastError();
 }
 
