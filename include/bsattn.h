@@ -266,7 +266,10 @@ int bsattn_export_summaries(const bsattn_cache* cache, int32_t seq, void* out,
  * start/stop events attached to its dispatch (launches captured into a
  * graph are not timed).  bsattn_profile_read waits for the recorded events
  * and returns the summed kernel time and launch count of one kernel kind
- * since profiling was last enabled.  Enabling (or disabling) resets the sums. */
+ * since profiling was last enabled.  Enabling (or disabling) resets the sums.
+ * (A small batch's decode merges its splits inside the attention launch; a
+ * timed one launches the combine by itself, so that its time is seen.  The
+ * results are the same bits.) */
 #define BSATTN_KERNEL_SCORE 0   /* block scoring */
 #define BSATTN_KERNEL_TOPK 1    /* top-K selection (bsattn_select) */
 #define BSATTN_KERNEL_ATTEND 2  /* gather + attention (selection fused in bsattn_decode) */

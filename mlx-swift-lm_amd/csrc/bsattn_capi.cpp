@@ -78,6 +78,7 @@ struct bsattn_cache {
   float* scores = nullptr;    // [rows][hkv][sstride] + kScoreSlack
   int32_t* idx_ws = nullptr;  // [rows][hkv][nsel_max]
   float* partials = nullptr;  // [rows][hq][nsplit][D + 2]
+  uint32_t* arrive = nullptr; // [kArriveWords] arrival counters of split merges, 0 between launches
   float* err_ws = nullptr;    // [rows][hkv][2][mfma_err_stride]: MFMA score bounds, chunk floors
   float* prefill_ws = nullptr;  // split prefill partials (allocated by the first call that splits)
   std::vector<int32_t> len;
@@ -363,6 +364,7 @@ int bsattn_cache_create(const bsattn_desc* desc, bsattn_cache** out) try {
     (void)hipFree(c->idx_ws);
     (void)hipFree(c->partials);
     (void)hipFree(c->err_ws);
+    (void)hipFree(c->arrive);
     delete c;
     return code;
   };
@@ -380,9 +382,12 @@ int bsattn_cache_create(const bsattn_desc* desc, bsattn_cache** out) try {
     return cleanup(hip_fail(e, "hipMalloc(partials)"));
   if ((e = hipMalloc((void**)&c->err_ws, rows * g.hkv * 2 * mfma_err_stride(g) * 4)) != hipSuccess)
     return cleanup(hip_fail(e, "hipMalloc(bounds)"));
+  if ((e = hipMalloc((void**)&c->arrive, kArriveWords * 4)) != hipSuccess)
+    return cleanup(hip_fail(e, "hipMalloc(counters)"));
   // zeroed pages: never-written token slots hold finite values
   if ((e = hipMemset(g.pool, 0, c->pool_bytes)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(pool)"));
   if ((e = hipMemset(g.summ, 0, c->summ_bytes)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(summaries)"));
+  if ((e = hipMemset(c->arrive, 0, kArriveWords * 4)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(counters)"));
   if ((e = hipMemset(g.meta, 0, c->meta_words * 4)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(meta)"));
   if ((e = hipDeviceSynchronize()) != hipSuccess) return cleanup(hip_fail(e, "hipDeviceSynchronize"));
   *out = c;
@@ -403,6 +408,7 @@ int bsattn_cache_destroy(bsattn_cache* c) try {
   (void)hipFree(c->idx_ws);
   (void)hipFree(c->partials);
   (void)hipFree(c->err_ws);
+  (void)hipFree(c->arrive);
   (void)hipFree(c->prefill_ws);
   delete c;
   return BSATTN_OK;
@@ -708,10 +714,11 @@ struct Workspace {
   float* err;
   int32_t* idx;
   float* partials;
+  uint32_t* arrive;
 };
 
 static Workspace cache_workspace(const bsattn_cache* c) {
-  return Workspace{c->scores, c->err_ws, c->idx_ws, c->partials};
+  return Workspace{c->scores, c->err_ws, c->idx_ws, c->partials, c->arrive};
 }
 
 // Selection, attention or both for the entries, in launches of at most
@@ -742,11 +749,12 @@ static int run_entries(bsattn_cache* c, Op op, const void* q, const Entry* es, i
       e = launch_select(g, b, qq, ws.scores, ws.err, io, max_nc, s, prof);
     } else if (op == Op::Attend) {
       if (fused_decode_ok(g, nseq, max_nc))
-        e = launch_fused_attend(g, b, nseq, qq, idx_in + e0 * idx_row, scale, oo, ws.partials, s, prof);
+        e = launch_fused_attend(g, b, nseq, qq, idx_in + e0 * idx_row, scale, oo, ws.partials, ws.arrive, s, prof);
       else
         e = launch_attend(g, b, qq, idx_in + e0 * idx_row, waves, scale, oo, ws.partials, s, prof);
     } else if (fused_decode_ok(g, nseq, max_nc)) {
-      e = launch_fused_decode(g, b, nseq, qq, io, len_first(c, es, e0, b.n), scale, oo, ws.partials, s, prof);
+      e = launch_fused_decode(g, b, nseq, qq, io, len_first(c, es, e0, b.n), scale, oo, ws.partials, ws.arrive, s,
+                              prof);
     } else if (max_nc > fused_select_limit(g.top_k)) {
       int32_t* sel = io ? io : ws.idx;
       e = launch_select(g, b, qq, ws.scores, ws.err, sel, max_nc, s, prof);
@@ -850,9 +858,10 @@ int bsattn_decode_noalloc(bsattn_cache* c, const void* q, const int32_t* seq_ids
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
   void* base = nullptr;
-  HIP_TRY(noalloc_scratch(c->d.device, &base), "hipGetSymbolAddress(scratch)");
+  uint32_t* arrive = nullptr;
+  HIP_TRY(noalloc_scratch(c->d.device, &base, &arrive), "hipGetSymbolAddress(scratch)");
   char* b = (char*)base;
-  const Workspace ws{(float*)(b + o_sc), (float*)(b + o_err), (int32_t*)(b + o_idx), (float*)(b + o_part)};
+  const Workspace ws{(float*)(b + o_sc), (float*)(b + o_err), (int32_t*)(b + o_idx), (float*)(b + o_part), arrive};
   return run_entries(c, Op::Decode, q, es, n_seqs, n_seqs, kHeadDim, nullptr, idx_out, scale, out,
                      (hipStream_t)stream, ws, false);
 } catch (...) {
@@ -912,7 +921,7 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
   Timing tm[kProfKinds];
   Timing* prof = prof_slots(c, s, tm);
   hipError_t e = launch_append_decode(g, b, ap, q, c->scores, c->err_ws, c->idx_ws, idx_out, max_nc, fused,
-                                     attend_waves(g, n_seqs), scale, out, c->partials, s, prof);
+                                     attend_waves(g, n_seqs), scale, out, c->partials, c->arrive, s, prof);
   prof_collect(c, prof);
   if (e != hipSuccess) return hip_fail(e, "append-decode launch");
   for (int sq : seqs) c->len[sq] += 1;

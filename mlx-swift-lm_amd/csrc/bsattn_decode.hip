@@ -13,7 +13,8 @@
 // the scores in LDS, and then gathers its share of the selected blocks:
 // slot (r * W + wave) * S + split, round r < R.  A wave keeps an online
 // softmax over its rounds; the W waves merge through LDS into the output
-// (S == 1) or into split partials for k_combine.
+// (S == 1) or into split partials, which the pair's last workgroup merges
+// (arrive_merge; the combine kernel beyond kArriveSplits or when profiled).
 //
 // Scoring is the canonical order of the oracle (16 lanes per block, 8 dims
 // per lane, left fold of the 8 products, pairwise tree over the 16 chunks,
@@ -90,6 +91,69 @@ __device__ __forceinline__ void score_chunk(const float (&qv)[G][8], const u32x4
   }
 }
 
+// ---------------------------------------------------------------------------
+// Top-K of at most 64 * kPickKeys candidates by each wave for itself, from
+// the scores in LDS: the same selection as wg_topk (K largest keys, ties to
+// the lower index), as masks over the candidates (candidate 64 k + lane is
+// bit `lane` of take[k]).  A bitwise search of the K-th largest key, one
+// ballot per 64 candidates and bit, ends as soon as a prefix is reached by
+// exactly K keys; no barrier and no LDS traffic, where wg_topk takes seven
+// barriers: 0.3-1.1 us less a launch (one sequence of 4k tokens, top-32 of 62,
+// 11.8 -> 10.7 us; 16 of 16k, top-32 of 254, 31.3 -> 30.8).
+// ---------------------------------------------------------------------------
+constexpr int kPickKeys = 4;
+__device__ __forceinline__ int mask_rank(uint64_t m) {  // bits of m below this lane
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+__device__ __forceinline__ void wave_pick(const float* s_score, int nc, int K, uint64_t (&take)[kPickKeys]) {
+  const int lane = threadIdx.x & 63;
+  uint32_t key[kPickKeys];
+  bool real[kPickKeys];
+#pragma unroll
+  for (int k = 0; k < kPickKeys; ++k) {
+    real[k] = 64 * k + lane < nc;
+    key[k] = real[k] ? score_key(s_score[64 * k + lane]) : 0u;
+  }
+  uint32_t t = 0u;
+  for (int bit = 31; bit >= 0; --bit) {
+    const uint32_t cand = t | (1u << bit);
+    int n = 0;
+#pragma unroll
+    for (int k = 0; k < kPickKeys; ++k) {
+      take[k] = __ballot(key[k] >= cand);  // (a padded key, 0, is never counted)
+      n += __popcll(take[k]);
+    }
+    if (n == K) return;
+    if (n > K) t = cand;
+  }
+  // t is the K-th largest key: those above it, then the first of those at it
+  int need = K;
+#pragma unroll
+  for (int k = 0; k < kPickKeys; ++k) {
+    take[k] = __ballot(key[k] > t);
+    need -= __popcll(take[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < kPickKeys; ++k) {
+    const uint64_t eq = __ballot(real[k] && key[k] == t);
+    take[k] |= __ballot(((eq >> lane) & 1ull) && mask_rank(eq) < need);
+    need = max(0, need - __popcll(eq));
+  }
+}
+// candidate with `rank` taken ones before it (rank < K, uniform)
+__device__ __forceinline__ int picked(const uint64_t (&take)[kPickKeys], int rank) {
+  const int lane = threadIdx.x & 63;
+  int at = 0;
+#pragma unroll
+  for (int k = 0; k < kPickKeys; ++k) {
+    const int n = __popcll(take[k]);
+    if (rank >= 0 && rank < n)
+      at = 64 * k + __ffsll((unsigned long long)__ballot(((take[k] >> lane) & 1ull) && mask_rank(take[k]) == rank)) - 1;
+    rank -= n;
+  }
+  return at;
+}
+
 // Adds one 16-dim tile of a block's O (accumulator layout: lane (dim n,
 // group g) holds heads 4g .. 4g+3) to the wave's running O in s_o, whose
 // heads are first rescaled by a[i] (the online-softmax factor of head 4g+i).
@@ -130,7 +194,8 @@ __global__ __launch_bounds__(64 * W) void k_decode(Geometry geo, SeqBatch sb,
                                                    const uint16_t* __restrict__ q,
                                                    int32_t* __restrict__ idx, float sl2,
                                                    uint16_t* __restrict__ out,
-                                                   float* __restrict__ partials, int S, int R,
+                                                   float* __restrict__ partials,
+                                                   uint32_t* __restrict__ arrive, int S, int R,
                                                    int len_first, ModeArgs<MODE> ap) {
   constexpr bool GIVEN = MODE == kModeGiven, APPEND = MODE == kModeFusedAppend;
   constexpr int NT = TB / 16;   // QK token tiles
@@ -291,8 +356,12 @@ __global__ __launch_bounds__(64 * W) void k_decode(Geometry geo, SeqBatch sb,
     // holds candidate c0 + 64 (W k + w) + l
     // (unconditional: slots from lim on read entry lim - 1 and are never
     // selected)
+    // (few candidates, each wave picking for itself: slot k, lane l holds
+    // candidate c0 + 64 k + l)
+    const bool few = nc <= 64 * kPickKeys;
 #pragma unroll
-    for (int k = 0; k < kWgKeys; ++k) wgc.page[k] = bt[min(c0 + 64 * (W * k + wave) + lane, max(lim - 1, 0))];
+    for (int k = 0; k < kWgKeys; ++k)
+      wgc.page[k] = bt[min(c0 + 64 * (few ? k : W * k + wave) + lane, max(lim - 1, 0))];
     // slots known from the length alone (sinks, recent, every block when
     // nothing is ranked): their pages are requested now
     {
@@ -330,20 +399,48 @@ __global__ __launch_bounds__(64 * W) void k_decode(Geometry geo, SeqBatch sb,
       }
       append_stage();
       __syncthreads();
-#pragma unroll
-      for (int k = 0; k < kWgKeys; ++k) {
-        const int i = 64 * (W * k + wave) + lane;
-        wgc.score[k] = i < nc ? s_score[i] : 0.0f;
-      }
-      wg_topk<W>(wgc, c0, nc, K, s_sel, s_selp, s_ws);
-      __syncthreads();
-      if (lane == 0) {
+      if (few) {
+        uint64_t take[kPickKeys];
+        wave_pick(s_score, nc, K, take);
 #pragma unroll 1
         for (int rr = 0; rr < R; ++rr) {
           const int slot = (rr * W + wave) * S + split;
-          if (slot >= geo.ns && slot < geo.ns + K) {
-            s_jr[wave][rr] = s_sel[slot - geo.ns];
-            s_pr[wave][rr] = s_selp[slot - geo.ns];
+          if (slot < geo.ns || slot >= geo.ns + K) continue;
+          const int cand = picked(take, slot - geo.ns);
+          int page = 0;
+#pragma unroll
+          for (int k = 0; k < kPickKeys; ++k)
+            if (cand >> 6 == k) page = __builtin_amdgcn_readlane(wgc.page[k], cand & 63);
+          if (lane == 0) {
+            s_jr[wave][rr] = c0 + cand;
+            s_pr[wave][rr] = page;
+          }
+        }
+        if (idx != nullptr && split == 0 && wave == 0) {
+          int before = 0;
+#pragma unroll
+          for (int k = 0; k < kPickKeys; ++k) {
+            if ((take[k] >> lane) & 1ull) s_sel[before + mask_rank(take[k])] = c0 + 64 * k + lane;
+            before += __popcll(take[k]);
+          }
+          wave_lds_order();
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < kWgKeys; ++k) {
+          const int i = 64 * (W * k + wave) + lane;
+          wgc.score[k] = i < nc ? s_score[i] : 0.0f;
+        }
+        wg_topk<W>(wgc, c0, nc, K, s_sel, s_selp, s_ws);
+        __syncthreads();
+        if (lane == 0) {
+#pragma unroll 1
+          for (int rr = 0; rr < R; ++rr) {
+            const int slot = (rr * W + wave) * S + split;
+            if (slot >= geo.ns && slot < geo.ns + K) {
+              s_jr[wave][rr] = s_sel[slot - geo.ns];
+              s_pr[wave][rr] = s_selp[slot - geo.ns];
+            }
           }
         }
       }
@@ -470,7 +567,8 @@ __global__ __launch_bounds__(64 * W) void k_decode(Geometry geo, SeqBatch sb,
     store_empty<G>(s_m[wave], s_l[wave], s_o[wave], lane);
   }
   __syncthreads();
-  attend_merge<DT, G, W>(geo, sb, bi, h, split, S, s_m, s_l, s_o, out, partials);
+  attend_merge<DT, G, W, true>(geo, sb, bi, h, split, S, s_m, s_l, s_o, out, partials);
+  if (arrive) arrive_merge<DT, G, W>(geo, sb, bi, h, S, arrive + pair, partials, out);
   if constexpr (APPEND) {
     // the completed block's summary: 16 lanes fold its keys from LDS (written
     // before the barriers of the merge) in token order
@@ -507,27 +605,27 @@ FusedPlan fused_plan(const Geometry& g, int n) {
 
 template <int DT, int TB, int G, int MD>
 void decode_w(const Geometry& g, const FusedPlan& p, dim3 grid, const SeqBatch& b, const uint16_t* q,
-              int32_t* idx, float sl2, uint16_t* out, float* part, int lf, const ModeArgs<MD>& ap,
+              int32_t* idx, float sl2, uint16_t* out, float* part, uint32_t* arr, int lf, const ModeArgs<MD>& ap,
               hipStream_t s, Timing* prof) {
   const int kd = kProfAttend;
   switch (p.W) {
-    case 4: launch(k_decode<DT, TB, G, 4, MD>, grid, dim3(256), 0, s, prof, kd, g, b, q, idx, sl2, out, part, p.S, p.R, lf, ap); break;
-    case 8: launch(k_decode<DT, TB, G, 8, MD>, grid, dim3(512), 0, s, prof, kd, g, b, q, idx, sl2, out, part, p.S, p.R, lf, ap); break;
+    case 4: launch(k_decode<DT, TB, G, 4, MD>, grid, dim3(256), 0, s, prof, kd, g, b, q, idx, sl2, out, part, arr, p.S, p.R, lf, ap); break;
+    case 8: launch(k_decode<DT, TB, G, 8, MD>, grid, dim3(512), 0, s, prof, kd, g, b, q, idx, sl2, out, part, arr, p.S, p.R, lf, ap); break;
     default:  // fused_plan gives W = 12 for 32-token blocks only
       if constexpr (TB == 32)
-        launch(k_decode<DT, TB, G, 12, MD>, grid, dim3(768), 0, s, prof, kd, g, b, q, idx, sl2, out, part, p.S, p.R, lf, ap);
+        launch(k_decode<DT, TB, G, 12, MD>, grid, dim3(768), 0, s, prof, kd, g, b, q, idx, sl2, out, part, arr, p.S, p.R, lf, ap);
       break;
   }
 }
 
 template <int DT, int TB, int MD>
 void decode_g(const Geometry& g, const FusedPlan& p, dim3 grid, const SeqBatch& b, const uint16_t* q,
-              int32_t* idx, float sl2, uint16_t* out, float* part, int lf, const ModeArgs<MD>& ap,
+              int32_t* idx, float sl2, uint16_t* out, float* part, uint32_t* arr, int lf, const ModeArgs<MD>& ap,
               hipStream_t s, Timing* prof) {
   switch (g.group) {
-    case 1: decode_w<DT, TB, 1, MD>(g, p, grid, b, q, idx, sl2, out, part, lf, ap, s, prof); break;
-    case 2: decode_w<DT, TB, 2, MD>(g, p, grid, b, q, idx, sl2, out, part, lf, ap, s, prof); break;
-    default: decode_w<DT, TB, 4, MD>(g, p, grid, b, q, idx, sl2, out, part, lf, ap, s, prof); break;
+    case 1: decode_w<DT, TB, 1, MD>(g, p, grid, b, q, idx, sl2, out, part, arr, lf, ap, s, prof); break;
+    case 2: decode_w<DT, TB, 2, MD>(g, p, grid, b, q, idx, sl2, out, part, arr, lf, ap, s, prof); break;
+    default: decode_w<DT, TB, 4, MD>(g, p, grid, b, q, idx, sl2, out, part, arr, lf, ap, s, prof); break;
   }
 }
 
@@ -535,7 +633,7 @@ void decode_g(const Geometry& g, const FusedPlan& p, dim3 grid, const SeqBatch& 
 // a multi-token decode holds several entries per sequence)
 template <int MD>
 hipError_t decode_impl(const Geometry& g, const SeqBatch& b, int nseq, const void* q, int32_t* idx,
-                       bool len_first, float scale, void* out, float* partials,
+                       bool len_first, float scale, void* out, float* partials, uint32_t* arrive,
                        const ModeArgs<MD>& ap, hipStream_t s, Timing* prof) {
   const FusedPlan p = fused_plan(g, nseq);
   const int pairs = b.n * g.hkv;
@@ -544,15 +642,17 @@ hipError_t decode_impl(const Geometry& g, const SeqBatch& b, int nseq, const voi
   const uint16_t* qq = (const uint16_t*)q;
   uint16_t* oo = (uint16_t*)out;
   const int lf = len_first ? 1 : 0;
+  const bool merge = p.S > 1 && p.S <= kArriveSplits && !prof;
+  arrive = merge ? arrive + (p.S - 1) * kArrivePairs : nullptr;
   if (g.dtype == 0) {
-    if (g.tb == 64) decode_g<0, 64, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, lf, ap, s, prof);
-    else decode_g<0, 32, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, lf, ap, s, prof);
+    if (g.tb == 64) decode_g<0, 64, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, arrive, lf, ap, s, prof);
+    else decode_g<0, 32, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, arrive, lf, ap, s, prof);
   } else {
-    if (g.tb == 64) decode_g<1, 64, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, lf, ap, s, prof);
-    else decode_g<1, 32, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, lf, ap, s, prof);
+    if (g.tb == 64) decode_g<1, 64, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, arrive, lf, ap, s, prof);
+    else decode_g<1, 32, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, arrive, lf, ap, s, prof);
   }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.S == 1) return e;
+  if (e != hipSuccess || p.S == 1 || merge) return e;
   return launch_combine(g, b, partials, p.S, out, s, prof);
 }
 
@@ -574,20 +674,20 @@ bool fused_decode_ok(const Geometry& g, int nseq, int max_nc) {
 
 hipError_t launch_fused_decode(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
                                int32_t* idx_out, bool len_first, float scale, void* out, float* partials,
-                               hipStream_t s, Timing* prof) {
-  return decode_impl<kModeFused>(g, b, nseq, q, idx_out, len_first, scale, out, partials, NoAppend{}, s, prof);
+                               uint32_t* arrive, hipStream_t s, Timing* prof) {
+  return decode_impl<kModeFused>(g, b, nseq, q, idx_out, len_first, scale, out, partials, arrive, NoAppend{}, s, prof);
 }
 
 hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap,
                                       const void* q, int32_t* idx_out, float scale, void* out, float* partials,
-                                      hipStream_t s, Timing* prof) {
-  return decode_impl<kModeFusedAppend>(g, b, b.n, q, idx_out, true, scale, out, partials, ap, s, prof);
+                                      uint32_t* arrive, hipStream_t s, Timing* prof) {
+  return decode_impl<kModeFusedAppend>(g, b, b.n, q, idx_out, true, scale, out, partials, arrive, ap, s, prof);
 }
 
 hipError_t launch_fused_attend(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
-                               const int32_t* idx, float scale, void* out, float* partials, hipStream_t s,
-                               Timing* prof) {
-  return decode_impl<kModeGiven>(g, b, nseq, q, const_cast<int32_t*>(idx), false, scale, out, partials,
+                               const int32_t* idx, float scale, void* out, float* partials, uint32_t* arrive,
+                               hipStream_t s, Timing* prof) {
+  return decode_impl<kModeGiven>(g, b, nseq, q, const_cast<int32_t*>(idx), false, scale, out, partials, arrive,
                                  NoAppend{}, s, prof);
 }
 

@@ -1227,7 +1227,9 @@ __device__ __forceinline__ void store_empty(float* s_m, float* s_l, float (*s_o)
 // written back while the next layer's scoring streams its summaries; narrow
 // groups' small partials are cheaper cached, for the combine right after.
 // (A runtime choice between the two stores compiles to the cached one.)
-template <int DT, int G>
+// THROUGH: device-scope stores, for a partial that another workgroup of the
+// launch reads (arrive_merge).
+template <int DT, int G, bool THROUGH = false>
 __device__ __forceinline__ void merge_emit(const Geometry& geo, const SeqBatch& sb, int bi, int h,
                                            int split, int nsplit, int head, int d, float M,
                                            float L, float a, uint16_t* __restrict__ out,
@@ -1238,7 +1240,14 @@ __device__ __forceinline__ void merge_emit(const Geometry& geo, const SeqBatch& 
   } else {
     const size_t row = (size_t)bi * geo.hq + h * G + head;
     float* pp = partials + (row * nsplit + split) * (kHeadDim + 2);
-    if constexpr (nt) {
+    if constexpr (THROUGH) {
+      auto put = [](float* p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+      put(pp + d, a);
+      if (d == 0) {
+        put(pp + kHeadDim, M);
+        put(pp + kHeadDim + 1, L);
+      }
+    } else if constexpr (nt) {
       __builtin_nontemporal_store(a, pp + d);
       if (d == 0) {
         __builtin_nontemporal_store(M, pp + kHeadDim);
@@ -1280,7 +1289,7 @@ __device__ __forceinline__ void merge_weights(const float (*s_m)[16], const floa
 // Dims d0 .. d0 + OD - 1 of the merged split from the waves' outputs in
 // s_o[w][head][d - d0], with the weights of merge_weights (behind a
 // barrier): each element is sum_w s_f[w][head] * o_w, summed from wave 0 up.
-template <int DT, int G, int W, int OD>
+template <int DT, int G, int W, int OD, bool THROUGH = false>
 __device__ __forceinline__ void merge_dims(const Geometry& geo, const SeqBatch& sb, int bi, int h,
                                            int split, int nsplit, const float (*s_f)[16],
                                            const float (*s_ML)[16], const float (*s_o)[G][OD],
@@ -1291,15 +1300,15 @@ __device__ __forceinline__ void merge_dims(const Geometry& geo, const SeqBatch& 
     float a = 0.f;
 #pragma unroll
     for (int w = 0; w < W; ++w) a += s_f[w][head] * s_o[w][head][d];
-    merge_emit<DT, G>(geo, sb, bi, h, split, nsplit, head, d0 + d, s_ML[0][head], s_ML[1][head], a,
-                      out, partials);
+    merge_emit<DT, G, THROUGH>(geo, sb, bi, h, split, nsplit, head, d0 + d, s_ML[0][head], s_ML[1][head], a,
+                               out, partials);
   }
 }
 
 // Merges the W waves' (m, l, o) (after a workgroup barrier) and writes the
 // normalised output (nsplit == 1) or the unnormalised partial (o, m, l) of
 // split `split` of nsplit for k_combine.
-template <int DT, int G, int W>
+template <int DT, int G, int W, bool THROUGH = false>
 __device__ __forceinline__ void attend_merge(const Geometry& geo, const SeqBatch& sb, int bi, int h,
                                              int split, int nsplit,
                                              const float (*s_m)[16], const float (*s_l)[16],
@@ -1326,14 +1335,70 @@ __device__ __forceinline__ void attend_merge(const Geometry& geo, const SeqBatch
         L += f * s_l[w][head];
         a += f * s_o[w][head][d];
       }
-      merge_emit<DT, G>(geo, sb, bi, h, split, nsplit, head, d, M, L, a, out, partials);
+      merge_emit<DT, G, THROUGH>(geo, sb, bi, h, split, nsplit, head, d, M, L, a, out, partials);
     }
   } else {
     __shared__ float s_f[W][16], s_ML[2][16];
     merge_weights<G, W>(s_m, s_l, s_f, s_ML);
     __syncthreads();
-    merge_dims<DT, G, W, kHeadDim>(geo, sb, bi, h, split, nsplit, s_f, s_ML, s_o, 0, out, partials);
+    merge_dims<DT, G, W, kHeadDim, THROUGH>(geo, sb, bi, h, split, nsplit, s_f, s_ML, s_o, 0, out, partials);
   }
+}
+
+// The split combine inside the launch that computes the splits: the workgroup
+// of a pair that arrives last merges the S <= kArriveSplits partials of its G
+// heads into the output, in the order of the combine kernel (the same bits).
+// It takes the launch 0.5-1.2 us where the combine kernel takes 3.9: per step
+// of the fused decode, fp16, 32 query and 8 kv heads (kernel times): one
+// sequence of 4k tokens 14.6 -> 12.0 us, 4 of 8k 18.1 -> 14.8, 8 of 16k
+// 24.2 -> 20.5, 16 of 16k (256 workgroups) 35.5 -> 32.2.
+// No workgroup waits for another.  Each thread's partials have reached device
+// scope (THROUGH stores, waited for) before its workgroup counts itself in;
+// the last one's loads are issued after its count returns and are
+// device-scope too, so they pass by stale cache lines.  The counter wraps to 0
+// with the S-th arrival, ready for the next launch; counters of different S
+// lie apart, so each only ever sees whole sets of S.
+template <int DT, int G, int W, int NS>
+__device__ __forceinline__ void merge_parts(const Geometry& geo, const SeqBatch& sb, int bi, int h, int S,
+                                            const float* __restrict__ partials, uint16_t* __restrict__ out) {
+  auto get = [](const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  for (int e = threadIdx.x; e < G * kHeadDim; e += 64 * W) {
+    const int head = h * G + e / kHeadDim, d = e % kHeadDim;
+    const float* pp = partials + ((size_t)bi * geo.hq + head) * S * (kHeadDim + 2);
+    float m[NS], l[NS], o[NS];
+#pragma unroll
+    for (int sp = 0; sp < NS; ++sp) {  // parts past S read the last one and weigh nothing
+      const float* p = pp + min(sp, S - 1) * (kHeadDim + 2);
+      m[sp] = get(p + kHeadDim);
+      l[sp] = get(p + kHeadDim + 1);
+      o[sp] = get(p + d);
+    }
+    float M = m[0];
+#pragma unroll
+    for (int sp = 1; sp < NS; ++sp) M = fmaxf(M, m[sp]);
+    float L = 0.f, a = 0.f;
+#pragma unroll
+    for (int sp = 0; sp < NS; ++sp) {
+      const float w = (sp >= S || m[sp] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m[sp] - M);
+      L += w * l[sp];
+      a += w * o[sp];
+    }
+    out[q_row(sb, bi, head) + d] = from_f32<DT>(a * (L > 0.f ? 1.f / L : 0.f));
+  }
+}
+template <int DT, int G, int W>
+__device__ __forceinline__ void arrive_merge(const Geometry& geo, const SeqBatch& sb, int bi, int h, int S,
+                                             uint32_t* counter, const float* __restrict__ partials,
+                                             uint16_t* __restrict__ out) {
+  __shared__ int s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) s_last = atomicInc(counter, (uint32_t)S - 1u) == (uint32_t)S - 1u;
+  __syncthreads();
+  if (!s_last) return;
+  if (S <= 4) merge_parts<DT, G, W, 4>(geo, sb, bi, h, S, partials, out);
+  else if (S <= 8) merge_parts<DT, G, W, 8>(geo, sb, bi, h, S, partials, out);
+  else merge_parts<DT, G, W, kArriveSplits>(geo, sb, bi, h, S, partials, out);
 }
 
 // ---------------------------------------------------------------------------

@@ -23,6 +23,11 @@ constexpr int kWaves = BSATTN_WAVES;  // waves per attention workgroup (one bloc
 // some CUs and 2 on the rest.
 constexpr int kWavesWide = 9;
 constexpr int kMaxSplits = 512;       // attention splits per (sequence, kv head)
+// Splits that a launch can merge itself, and its arrival counters: one per
+// (entry, kv head) for each split count, all 0 between launches
+constexpr int kArriveSplits = 16;
+constexpr int kArrivePairs = kMaxBatch * 16;
+constexpr int kArriveWords = kArriveSplits * kArrivePairs;
 // device scratch of the no-allocation decode (bsattn_noalloc.hip), per GPU
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
 // rows of prefill partials (query rows times parts) a cache's workspace holds
@@ -117,9 +122,10 @@ struct Timing {
   bool used = false;
 };
 
-// address of the no-allocation scratch on `device`, which must be current
-// (looked up once per device; bsattn_noalloc.hip)
-hipError_t noalloc_scratch(int device, void** out);
+// addresses of the no-allocation scratch and of its arrival counters on
+// `device`, which must be current (looked up once per device;
+// bsattn_noalloc.hip)
+hipError_t noalloc_scratch(int device, void** out, uint32_t** arrive);
 
 // launchers (bsattn_kernels.hip); return hipError_t of the launch
 hipError_t launch_patch(const Geometry& g, const PatchBatch& pb, hipStream_t s);
@@ -190,7 +196,7 @@ hipError_t launch_decode_attend(const Geometry& g, const SeqBatch& b, const void
 hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap, const void* q,
                                 float* scores, float* err, int32_t* idx, int32_t* idx_out, int max_nc,
                                 bool fused, int waves, float scale, void* out, float* partials,
-                                hipStream_t s, Timing* prof);
+                                uint32_t* arrive, hipStream_t s, Timing* prof);
 // split combine of nsplit partials per (entry, q head) into out
 hipError_t launch_combine(const Geometry& g, const SeqBatch& b, const float* partials, int nsplit,
                           void* out, hipStream_t s, Timing* prof);
@@ -201,6 +207,9 @@ hipError_t launch_combine(const Geometry& g, const SeqBatch& b, const float* par
 // candidate blocks per entry fit it.  len_first: each workgroup reads its
 // entry's length before the summaries (for ragged batches; otherwise every
 // row of the block-table width is read at once).  idx_out may be null.
+// arrive: arrival counters (kArriveWords); with up to kArriveSplits splits
+// the launch merges them itself, unless it is profiled: the combine is then a
+// launch of its own, timed as such, with the same result.
 bool fused_decode_ok(const Geometry& g, int nseq, int max_nc);
 // exact (canonical) block scores of every ranked candidate into `scores`
 hipError_t launch_score(const Geometry& g, const SeqBatch& b, const void* q, float* scores, int max_nc,
@@ -208,20 +217,20 @@ hipError_t launch_score(const Geometry& g, const SeqBatch& b, const void* q, flo
 
 hipError_t launch_fused_decode(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
                                int32_t* idx_out, bool len_first, float scale, void* out, float* partials,
-                               hipStream_t s, Timing* prof);
+                               uint32_t* arrive, hipStream_t s, Timing* prof);
 // the same kernel's gather + attention over given indices (used by
 // bsattn_attend exactly where decode takes the fused path, so that
 // decode == select + attend bit for bit)
 hipError_t launch_fused_attend(const Geometry& g, const SeqBatch& b, int nseq, const void* q,
-                               const int32_t* idx, float scale, void* out, float* partials, hipStream_t s,
-                               Timing* prof);
+                               const int32_t* idx, float scale, void* out, float* partials, uint32_t* arrive,
+                               hipStream_t s, Timing* prof);
 // one launch per decode step: each entry's new token is stored at position
 // b.len[i] - 1 on page ap.sp.page[i] before the fused decode gathers it, the
 // block it fills gets its summary, and the metadata patches ap.pb are applied
 // for the launches that follow (requires recent >= 1)
 hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap,
                                       const void* q, int32_t* idx_out, float scale, void* out, float* partials,
-                                      hipStream_t s, Timing* prof);
+                                      uint32_t* arrive, hipStream_t s, Timing* prof);
 // dense causal attention of the last L tokens of each sequence.  nsplit > 1:
 // every query's tokens are split into that many parts, whose partials (ws:
 // nsplit * n * hq * L rows of kHeadDim + 2 floats, at most kPrefillRows rows)

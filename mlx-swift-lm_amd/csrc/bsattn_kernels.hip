@@ -670,9 +670,9 @@ hipError_t launch_decode(const Geometry& g, const SeqBatch& b, const void* q, fl
 hipError_t launch_append_decode(const Geometry& g, const SeqBatch& b, const StepAppend& ap, const void* q,
                                 float* scores, float* err, int32_t* idx, int32_t* idx_out, int max_nc,
                                 bool fused, int waves, float scale, void* out, float* partials,
-                                hipStream_t s, Timing* prof) {
+                                uint32_t* arrive, hipStream_t s, Timing* prof) {
   // the fused decode appends, scores and attends in one launch
-  if (fused) return launch_fused_append_decode(g, b, ap, q, idx_out, scale, out, partials, s, prof);
+  if (fused) return launch_fused_append_decode(g, b, ap, q, idx_out, scale, out, partials, arrive, s, prof);
   hipError_t e;
   if (max_nc > fused_select_limit(g.top_k)) {
     int32_t* sel = idx_out ? idx_out : idx;
