@@ -27,11 +27,13 @@ _DTYPES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16}
 
 
 def _stream(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The raw handle of the device's current stream (an int, as the foreign
+    functions' argument types take it)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _ptr(t: torch.Tensor):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 class BlockSparseKVCache:
@@ -60,6 +62,13 @@ class BlockSparseKVCache:
             self._h = h
         else:
             self._h = _handle
+        torch.cuda.init()  # (the raw stream is asked for without torch's own lazy start)
+        # What a decode step's checks and call read.  A small step is bound by
+        # the host: with the checks as one comparison each and plain integers
+        # for pointers and stream, four steps of one sequence and their trim
+        # take it 38 us, 63 before (one launch a step less included).
+        self._lib = lib()
+        self._hq, self._hkv, self._dim = num_q_heads, num_kv_heads, head_dim
         info = _lib.Info()
         check(lib().bsattn_cache_info(self._h, ctypes.byref(info)))
         self.nselMax = info.nsel_max
@@ -146,6 +155,11 @@ class BlockSparseKVCache:
             raise ValueError(f"{name} must be a contiguous {self.dtype} tensor on {self.device}")
         if t.dim() != 4 or t.shape[1] != self.desc.num_kv_heads or t.shape[3] != self.desc.head_dim:
             raise ValueError(f"{name} must be [B, {self.desc.num_kv_heads}, L, {self.desc.head_dim}], got {tuple(t.shape)}")
+
+    def _plain(self, t: torch.Tensor, shape) -> bool:
+        """A contiguous tensor of the cache's type and device, of this shape."""
+        return (t.shape == shape and t.dtype is self.dtype and t.get_device() == self.device.index
+                and t.is_contiguous())
 
     def append(self, keys: torch.Tensor, values: torch.Tensor,
                seq_ids: Optional[Sequence[int]] = None) -> None:
@@ -298,7 +312,7 @@ class BlockSparseKVCache:
             raise ValueError("idx must be a contiguous int32 [B, Hkv, nselMax] tensor on the cache device")
         out = torch.empty_like(queries)
         check(lib().bsattn_attend(self._h, _ptr(queries), i32_array(seq_ids), B, _ptr(idx),
-                                  ctypes.c_float(scale), _ptr(out), _stream(self.device)))
+                                  scale, _ptr(out), _stream(self.device)))
         return out
 
     def decode(self, queries: torch.Tensor, scale: float,
@@ -312,7 +326,7 @@ class BlockSparseKVCache:
                 raise ValueError("idx_out must be int32 [B, Hkv, nselMax]")
             idx_p = _ptr(idx_out)
         check(lib().bsattn_decode(self._h, _ptr(queries), i32_array(seq_ids), B,
-                                  ctypes.c_float(scale), _ptr(out), idx_p, _stream(self.device)))
+                                  scale, _ptr(out), idx_p, _stream(self.device)))
         return out
 
     def decodeNoAlloc(self, queries: torch.Tensor, scale: float, out: torch.Tensor,
@@ -331,7 +345,7 @@ class BlockSparseKVCache:
                 raise ValueError("idx_out must be int32 [B, Hkv, nselMax]")
             idx_p = _ptr(idx_out)
         check(lib().bsattn_decode_noalloc(self._h, _ptr(queries), i32_array(seq_ids), B,
-                                          ctypes.c_float(scale), _ptr(out), idx_p, _stream(self.device)))
+                                          scale, _ptr(out), idx_p, _stream(self.device)))
         return out
 
     def appendDecode(self, keys: torch.Tensor, values: torch.Tensor, queries: torch.Tensor,
@@ -343,22 +357,28 @@ class BlockSparseKVCache:
         decode(), in one launch (the append inside the fused decode) or with
         the append and the block scoring in one launch where the cache allows
         it."""
-        self._check_kv(keys, "keys")
-        self._check_kv(values, "values")
-        if keys.shape != values.shape or keys.shape[2] != 1:
-            raise ValueError("keys and values must both be [B, Hkv, 1, D]")
-        B = self._check_q(queries)
-        if keys.shape[0] != B:
+        B = queries.size(0) if queries.dim() == 4 else -1
+        kv = (B, self._hkv, 1, self._dim)
+        if not (self._plain(keys, kv) and self._plain(values, kv)
+                and self._plain(queries, (B, self._hq, 1, self._dim))):
+            # say what is wrong
+            self._check_kv(keys, "keys")
+            self._check_kv(values, "values")
+            if keys.shape != values.shape or keys.shape[2] != 1:
+                raise ValueError("keys and values must both be [B, Hkv, 1, D]")
+            self._check_q(queries)
             raise ValueError("keys / values and queries disagree on B")
         out = torch.empty_like(queries)
         idx_p = None
         if idx_out is not None:
-            if idx_out.dtype != torch.int32 or tuple(idx_out.shape) != (B, self.desc.num_kv_heads, self.nselMax):
+            if idx_out.dtype != torch.int32 or tuple(idx_out.shape) != (B, self._hkv, self.nselMax):
                 raise ValueError("idx_out must be int32 [B, Hkv, nselMax]")
             idx_p = _ptr(idx_out)
-        check(lib().bsattn_append_decode(self._h, _ptr(keys), _ptr(values), _ptr(queries),
-                                         i32_array(seq_ids), B, ctypes.c_float(scale), _ptr(out),
-                                         idx_p, _stream(self.device)))
+        rc = self._lib.bsattn_append_decode(self._h, keys.data_ptr(), values.data_ptr(), queries.data_ptr(),
+                                            None if seq_ids is None else i32_array(seq_ids), B, scale,
+                                            out.data_ptr(), idx_p, _stream(self.device))
+        if rc:
+            check(rc)
         return out
 
     def decodeMulti(self, queries: torch.Tensor, scale: float,
@@ -380,7 +400,7 @@ class BlockSparseKVCache:
                 raise ValueError("idx_out must be a contiguous int32 [B, L, Hkv, nselMax] tensor")
             idx_p = _ptr(idx_out)
         check(lib().bsattn_decode_multi(self._h, _ptr(queries), i32_array(seq_ids), B, L,
-                                        ctypes.c_float(scale), _ptr(out), idx_p, _stream(self.device)))
+                                        scale, _ptr(out), idx_p, _stream(self.device)))
         return out
 
     def prefill(self, queries: torch.Tensor, scale: float,
@@ -393,7 +413,7 @@ class BlockSparseKVCache:
         B = self._check_q(queries, multi=True)
         out = torch.empty_like(queries)
         check(lib().bsattn_prefill(self._h, _ptr(queries), i32_array(seq_ids), B, queries.shape[2],
-                                   ctypes.c_float(scale), _ptr(out), _stream(self.device)))
+                                   scale, _ptr(out), _stream(self.device)))
         return out
 
     # -- kernel timing -------------------------------------------------------
