@@ -19,6 +19,7 @@
 namespace bsattn {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 template <int DT>
 __device__ __forceinline__ f32x16 mfma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
@@ -81,17 +82,21 @@ struct Staged<0> {
 // V fragments as they are stored.  K fragments are read from LDS by row in
 // the same way (16 bytes a lane from the fragment that holds them).
 //
-// The unit pipeline (one workgroup barrier per unit).  In step u a wave
+// The unit pipeline (one workgroup barrier per two units).  In step u a wave
 //  - computes S of unit u + 1 (K from LDS) while it turns S of unit u into P,
 //    then O += V P of unit u: products that depend on nothing in the
 //    softmax, for the matrix cores to run beside it;
-//  - writes its fragments of unit u + 2, which it loaded two steps ago, to
-//    LDS and loads those of unit u + 4.
-// K has two LDS slots (unit u + 1 is read while u + 2 is written over u), V
-// four.  What bounds it: MFMA issue (16 x 32 cycles a wave and unit, two
-// waves per SIMD) beside ~100 VALU and 16 exp2, and LDS reads (16 KiB a wave
-// and unit, 8 cycles per KiB for the CU's 8 waves: as long as the MFMAs of
-// one SIMD's two waves).
+//  - writes its fragments of unit u + 3, which it loaded two steps ago, to
+//    LDS and loads those of unit u + 5.
+// The barrier ends the odd steps.  Between two of them (steps u and u + 1, u
+// even) the waves read K of u + 1 and u + 2 and write u + 3 and u + 4: four
+// slots; they read V of u and u + 1, keep that of u + 2 and write the same
+// two: eight slots, by the unit's low bits.  What bounds it: the power that
+// MFMAs and LDS reads take together (the clock falls to ~2.0 GHz), LDS reads
+// (16 KiB a wave and unit) and the VALU work of a wave's softmax between its
+// MFMAs (16 x 32 cycles a wave and unit, two waves per SIMD): ~70 VALU a unit
+// and 16 exp2, 20 more for bf16 V.  Four waves of 64 columns, which halve the
+// LDS reads and leave one wave per SIMD, take 2575 us where this takes 2198.
 //
 // V of a bf16 cache is converted to fp16 on its way to LDS (exact for
 // |v| < 65520 down to the fp16 normal range) for an fp16 PV product without
@@ -108,11 +113,15 @@ struct Staged<0> {
 // most tokens come first.
 // nsplit > 1: each tile's units are cut into nsplit runs, whose unnormalised
 // (o, m, l) go to po / pml for k_prefill_combine.
-// Measured, 512-token chunks at 32k tokens, Hq 32, Hkv 8, against the kernel
-// before it (16x16x32 MFMAs, 4-wave workgroups, one unit ahead by LDS DMA, a
-// block-table load waited for at the head of every unit): 8 sequences, bf16
-// 2829 -> 2361 us (923 TFLOP/s), int4 2977 -> 2528 us; one sequence, split in
-// 4, 1353 -> 370 us; a prompt of 8191 fp16 tokens 693 -> 610 us.
+// The loop's counters, page lookup and addresses are scalar: workgroup indexes
+// that come from divisions, and bounds made from them, pass through uniform(),
+// or the compiler keeps them in vector registers and 64-bit vector products
+// at every unit.
+// Measured, 512-token chunks at 32k tokens, Hq 32, Hkv 8, with vector counters
+// and a barrier at every unit -> now: 8 sequences, bf16 2388 -> 2198 us (993
+// TFLOP/s), int4 2494 -> 2373 us; one sequence, split in 4, 362 -> 296 us; a
+// prompt of 8191 fp16 tokens 575 -> 581 us (16x16x32 MFMAs in 4-wave
+// workgroups, one unit ahead: 2839, 3000, 1125 and 687 us).
 // grid (ceil(L / (256 / G)) * Hkv * n * nsplit)
 // ---------------------------------------------------------------------------
 template <int DT, int KB>
@@ -127,22 +136,24 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   // is skipped for most units; O^T / l is unchanged by the choice
   constexpr float kLazy = 8.f;
   constexpr bool CV = KB == 0 && DT == 1;
-  __shared__ __align__(16) u32x4 s_k[2][8 * 64], s_v[4][8 * 64];
+  __shared__ __align__(16) u32x4 s_k[4][8 * 64], s_v[8][8 * 64];
   __shared__ __align__(16) u32x4 s_ent[KB ? kPfWaves : 1][KB ? 32 : 1];  // each wave's copy of a unit's scales / biases
-  __shared__ int s_flag[4][kPfWaves];  // CV: wave w's V fragment of the slot's unit holds a value fp16 cannot take
+  __shared__ int s_flag[8][kPfWaves];  // CV: wave w's V fragment of the slot's unit holds a value fp16 cannot take
   const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 31, hh = lane >> 5;
   // XCD-grouped workgroup order (a bijection on [0, total))
   const int total = gridDim.x, flat = blockIdx.x, even = total & ~7;
   const int lid = flat < even ? (flat & 7) * (even >> 3) + (flat >> 3) : flat;
-  const int tile = gx - 1 - lid % gx, part = lid / gx % nsplit, pair = lid / (gx * nsplit);
-  const int bi = pair / geo.hkv, h = pair - bi * geo.hkv;
+  const int run_of = uniform(lid / gx), tile = gx - 1 - (lid - run_of * gx);
+  const int pair = uniform(run_of / nsplit), part = run_of - pair * nsplit;
+  const int bi = uniform(pair / geo.hkv), h = pair - bi * geo.hkv;
   const int qpw = kPfCols >> lg;            // query tokens per wave
   const int twg = tile * kPfWaves * qpw;    // the workgroup's first query token
-  const bool active = twg + wave * qpw < L;
+  const bool active = uniform(twg + wave * qpw < L);
   const int seq = uniform(sb.ids[bi]);
   const int T = uniform(geo.meta[seq]);
-  const int tq = twg + wave * qpw + (col >> lg), head = (h << lg) + (col & ((1 << lg) - 1));
+  const int head = (h << lg) + (col & ((1 << lg) - 1));
+  const int tq = twg + wave * qpw + (col >> lg);
   // scores are taken as (K . Q') * |sl2| with Q' = Q * sign(sl2): the sign
   // flip is exact, and a positive factor lets the block maximum be found on
   // the raw products.  A padding column (no query token) has Q = 0, sees
@@ -159,15 +170,18 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   const int ksh = geo.tb == 64 ? 1 : 0;  // log2 of the units of a block
   const int last = T - L + min(L - 1, twg + kPfWaves * qpw - 1);  // the workgroup's last position
   const int nunit = last / 32 + 1;
-  const int ua = (int)((int64_t)nunit * part / nsplit), ub = (int)((int64_t)nunit * (part + 1) / nsplit);
+  // (at most 2^26 units in at most 16 parts; kept in scalar registers, so that
+  // the loop's counters, page lookups and addresses are scalar too)
+  const int ua = uniform((int)((uint32_t)nunit * part / nsplit)), ub = uniform((int)((uint32_t)nunit * (part + 1) / nsplit));
   // units below nfull are whole and visible to every column of the workgroup
-  const int nfull = min((T - L + twg + 1) / 32, ub);
+  const int nfull = uniform(min((T - L + twg + 1) / 32, ub));
 
   // --- units from memory: this wave's fragments, in the slab's own order
   const int32_t* bt = block_table(geo, seq);
   const int lastblk = last / geo.tb;
   int pbase = ua >> ksh;  // lane i of pagev: page of block pbase + i
   int pagev = bt[min(pbase + lane, lastblk)];
+  const uint32_t lane16 = 16 * (threadIdx.x & 63);
   auto load = [&](int x, Staged<KB>& st) __attribute__((always_inline)) {
     x = max(min(x, ub - 1), ua);
     const int blk = x >> ksh, sub = x & ((1 << ksh) - 1);
@@ -180,15 +194,15 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
     const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
     const uint8_t *ks = slab + geo.k_off, *vs = slab + geo.v_off;
     if constexpr (KB == 0) {
-      st.k = *(const u32x4*)(ks + (8 * sub + wave) * 1024 + lane * 16);
-      st.v = *(const u32x4*)(vs + ((wave << ksh) + sub) * 1024 + lane * 16);
+      st.k = *(const u32x4*)(ks + (8 * sub + wave) * 1024 + lane16);
+      st.v = *(const u32x4*)(vs + ((wave << ksh) + sub) * 1024 + lane16);
     } else {
       if constexpr (KB == 4) {
-        st.k[0] = *(const uint32_t*)(ks + (2 * sub + (wave >> 2)) * 1024 + 4 * (wave & 3) + lane * 16);
-        st.v[0] = *(const uint32_t*)(vs + (((wave >> 2) << ksh) + sub) * 1024 + 4 * (wave & 3) + lane * 16);
+        st.k[0] = *(const uint32_t*)(ks + (2 * sub + (wave >> 2)) * 1024 + 4 * (wave & 3) + lane16);
+        st.v[0] = *(const uint32_t*)(vs + (((wave >> 2) << ksh) + sub) * 1024 + 4 * (wave & 3) + lane16);
       } else {
-        const uint2 a = *(const uint2*)(ks + (4 * sub + (wave >> 1)) * 1024 + 8 * (wave & 1) + lane * 16);
-        const uint2 b = *(const uint2*)(vs + (((wave >> 1) << ksh) + sub) * 1024 + 8 * (wave & 1) + lane * 16);
+        const uint2 a = *(const uint2*)(ks + (4 * sub + (wave >> 1)) * 1024 + 8 * (wave & 1) + lane16);
+        const uint2 b = *(const uint2*)(vs + (((wave >> 1) << ksh) + sub) * 1024 + 8 * (wave & 1) + lane16);
         st.k[0] = a.x;
         st.k[1] = a.y;
         st.v[0] = b.x;
@@ -200,21 +214,29 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   };
   // --- and into LDS, as 16-bit fragments; r: the unit's index from ua
   auto stage = [&](int r, const Staged<KB>& st, auto mask_tag) __attribute__((always_inline)) {
+    if constexpr (KB != 0) {
+      // the unit's scale / bias entries through this wave's own LDS rows
+      // (a wave's LDS accesses complete in order)
+      s_ent[wave][lane & 31] = st.e;
+      wave_lds_order();
+    }
     u32x4 kw, vw;
     if constexpr (KB == 0) {
       kw = st.k;
       vw = st.v;
       if constexpr (CV) {
-        // a bf16 value of magnitude >= 65536 (or inf / NaN) flags the unit
-        uint32_t big = 0u;
+        // a bf16 value of magnitude >= 65536 (or inf / NaN) flags the unit:
+        // the largest magnitude bits of either half, >= 0x4780
+        u16x2 big = {0, 0};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const uint32_t x = vw[k];
-          big |= ((x & 0x7FFFu) + 0x3880u) | ((((x >> 16) & 0x7FFFu) + 0x3880u));  // bit 15: >= 0x4780
+          const uint32_t x = vw[k], mag = x & 0x7FFF7FFFu;
+          big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2, mag));
           vw[k] = cvt_pk<0>(__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u));
         }
-        const bool any = __builtin_amdgcn_ballot_w64((big & 0x8000u) != 0u) != 0;
-        if (lane == 0) s_flag[r & 3][wave] = any ? 1 : 0;
+        const bool any =
+            __builtin_amdgcn_ballot_w64(((__builtin_bit_cast(uint32_t, big) + 0x38803880u) & 0x80008000u) != 0u) != 0;
+        if (lane == 0) s_flag[r & 7][wave] = any ? 1 : 0;
       }
     } else {
       using QC = QCode<KB>;
@@ -238,10 +260,6 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
         if constexpr (KB == 4) return nib_to_f16(w[0]);
         else return byte_to_f16(w[0], w[1]);
       };
-      // the unit's scale / bias entries through this wave's own LDS rows
-      // (a wave's LDS accesses complete in order)
-      s_ent[wave][lane & 31] = st.e;
-      wave_lds_order();
       const uint32_t* ent = (const uint32_t*)s_ent[wave];
       {
         // row m of QK key tile t is token 8 (m / 4) + 4 t + m % 4 of the unit
@@ -266,7 +284,6 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
         }
         vw = deq(codes(st.v), sp, bp);
       }
-      wave_lds_order();
     }
     if constexpr (decltype(mask_tag)::value) {
       // V of tokens past the sequence end (stale page data) is zeroed
@@ -277,8 +294,9 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
         vw[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
       }
     }
-    s_k[r & 1][wave * 64 + lane] = kw;
-    s_v[r & 3][wave * 64 + lane] = vw;
+    s_k[r & 3][wave * 64 + lane] = kw;
+    s_v[r & 7][wave * 64 + lane] = vw;
+    if constexpr (KB != 0) wave_lds_order();
   };
 
   // --- this wave's columns
@@ -292,7 +310,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   const int kl = ((col >> 3) & 1) * 256 + 8 * (col >> 4) + 4 * ((col >> 2) & 1) + (col & 3) + 16 * hh;
   const int vl = (col >> 4) * 64 + (col & 15) + 16 * hh;
   auto scores = [&](int r) __attribute__((always_inline)) {  // S^T of unit ua + r
-    const u32x4* kp = s_k[r & 1] + kl;
+    const u32x4* kp = s_k[r & 3] + kl;
     f32x16 a;
 #pragma unroll
     for (int i = 0; i < 16; ++i) a[i] = 0.f;
@@ -307,15 +325,18 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
 #pragma unroll
       for (int i = 0; i < 16; ++i) a[i] = 16 * (i >> 3) + (i & 7) <= lim ? a[i] : -INFINITY;
     }
-    float x = fmaxf(a[0], a[1]);
-#pragma unroll
-    for (int i = 2; i < 16; i += 2) x = fmaxf(x, fmaxf(a[i], a[i + 1]));
-    return x;
+    float x = fmaxf(fmaxf(a[0], a[1]), a[2]), y = fmaxf(fmaxf(a[3], a[4]), a[5]);
+    x = fmaxf(fmaxf(x, a[6]), a[7]);
+    y = fmaxf(fmaxf(y, a[8]), a[9]);
+    x = fmaxf(fmaxf(x, a[10]), a[11]);
+    y = fmaxf(fmaxf(y, a[12]), a[13]);
+    x = fmaxf(fmaxf(x, a[14]), a[15]);
+    return fmaxf(x, y);
   };
   // step r: `cur` holds S of unit r, `nxt` takes that of unit r + 1.  BIG: the
   // unit's V holds a value fp16 cannot take
   int flag = 0;  // CV: whether the next step's unit does
-  auto step = [&](int r, f32x16& cur, f32x16& nxt, Staged<KB>& st, auto act, auto mask_tag, auto big_tag)
+  auto step = [&](int r, f32x16& cur, f32x16& nxt, Staged<KB>& st, auto act, auto mask_tag, auto big_tag, bool sync)
       __attribute__((always_inline)) {
     constexpr bool ACT = decltype(act)::value;
     [[maybe_unused]] int fnext = 0;
@@ -335,18 +356,17 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       }
-      if constexpr (CV) fnext = s_flag[(r + 1) & 3][lane & 7];
+      if constexpr (CV) fnext = s_flag[(r + 1) & 7][lane & 7];
     }
-    stage(r + 2, st, mask_tag);
-    load(ua + r + 4, st);
+    stage(r + 3, st, mask_tag);
+    load(ua + r + 5, st);
     if constexpr (ACT) {
       nxt = scores(r + 1);
-      float ps = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        cur[i] = __builtin_amdgcn_exp2f(fmaf(cur[i], sc, -m));
-        ps += cur[i];
-      }
+      for (int i = 0; i < 16; ++i) cur[i] = __builtin_amdgcn_exp2f(fmaf(cur[i], sc, -m));
+      float ps = cur[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) ps += cur[i];
       l += ps;  // this lane's tokens; the column's halves are summed at the end
       if constexpr (decltype(big_tag)::value) {
         // bf16 P as hi + lo against the cache's own V fragments
@@ -377,7 +397,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
           }
         }
       } else {
-        const u32x4* vp = s_v[r & 3] + vl;
+        const u32x4* vp = s_v[r & 7] + vl;
         u32x4 pf[2];
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk)
@@ -391,7 +411,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
       lm = lane_max(nxt, r + 1, mask_tag);
       if constexpr (CV) flag = __builtin_amdgcn_ballot_w64(fnext != 0) != 0 ? 1 : 0;
     }
-    unit_barrier();
+    if (sync) unit_barrier();
   };
 
   Staged<KB> st0, st1;
@@ -401,7 +421,9 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   stage(0, st0, std::true_type{});
   load(ua + 2, st0);
   stage(1, st1, std::true_type{});
-  load(ua + 3, st1);
+  load(ua + 4, st1);
+  stage(2, st0, std::true_type{});
+  load(ua + 3, st0);
   unit_barrier();
   if (active) {
     sa = scores(0);
@@ -410,11 +432,11 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   }
   unit_barrier();
   // every wave takes ub - ua steps (one barrier each); a wave past the last
-  // query token only loads and stages.  The steps whose units (up to r + 2)
+  // query token only loads and stages.  The steps whose units (up to r + 3)
   // are whole and visible to every column go in pairs (fixed registers for
   // both score tiles and both staged units), the others one by one.
   auto run = [&](auto act) __attribute__((always_inline)) {
-    const int n = ub - ua, plain = nfull - ua - 3;  // pairs r, r + 1 with r + 3 < nfull - ua
+    const int n = ub - ua, plain = nfull - ua - 4;  // pairs r, r + 1 with r + 4 < nfull - ua
     int r = 0;
     auto flip = [&]() __attribute__((always_inline)) {
       const f32x16 sx = sa;
@@ -428,24 +450,26 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
     while (r < n) {
       if constexpr (CV && decltype(act)::value) {
         if (flag) {
-          step(r++, sa, sb2, st0, act, std::true_type{}, std::true_type{});
+          step(r, sa, sb2, st0, act, std::true_type{}, std::true_type{}, (r & 1) != 0);
+          ++r;
           flip();
           continue;
         }
       }
-      if (r < plain) {
+      if (r < plain && (r & 1) == 0) {
 #pragma unroll 1
         do {
-          step(r++, sa, sb2, st0, act, std::false_type{}, std::false_type{});
+          step(r++, sa, sb2, st0, act, std::false_type{}, std::false_type{}, false);
           if (CV && flag) {
             flip();
             break;
           }
-          step(r++, sb2, sa, st1, act, std::false_type{}, std::false_type{});
+          step(r++, sb2, sa, st1, act, std::false_type{}, std::false_type{}, true);
         } while (r < plain && !(CV && flag));
         continue;
       }
-      step(r++, sa, sb2, st0, act, std::true_type{}, std::false_type{});
+      step(r, sa, sb2, st0, act, std::true_type{}, std::false_type{}, (r & 1) != 0);
+      ++r;
       flip();
     }
   };

@@ -9,7 +9,7 @@ import pytest
 
 from common import log, make_workload, new_cache, to_dev
 import oracle as O
-from test_gpu_prefill import _check, _run, test_prefill_quantized_cache as check_quantized
+from test_gpu_prefill import TOL, _check, _run, ulp, test_prefill_quantized_cache as check_quantized
 
 pytestmark = pytest.mark.gpu
 
@@ -35,6 +35,35 @@ def test_prefill_tile_edges(gpu, dtype, Hq, Hkv, Tb, lens, L):
 ])
 def test_prefill_tile_edges_quantized(gpu, bits, Hq, Hkv, Tb, lens, L):
     check_quantized(gpu, bits, Hq, Hkv, Tb, lens, L)
+
+
+@pytest.mark.parametrize("dtype,units,big", [
+    ("f16", 1, ()), ("bf16", 2, ()), ("f16", 3, ()), ("bf16", 4, (3,)), ("bf16", 5, (1, 2)),
+    ("bf16", 11, (2, 3, 7)), ("f16", 12, ()),
+])
+def test_prefill_unit_counts(gpu, dtype, units, big):
+    """Prefills of a few 32-token units (the waves meet after every second
+    one), odd and even; `big` units hold bf16 values that fp16 cannot, so
+    that the steps leave their pairs at odd and even units."""
+    log(f"[prefill units] {dtype} {units} {big}")
+    L, T = 20, 32 * units - 3
+    w = make_workload(8300 + units, B=1, Hq=32, Hkv=8, T=T, Tb=32, dtype=dtype, top_k=4)
+    v = O.to_f32(w.values[0], dtype)
+    for u in big:
+        v[:, 32 * u + 5, :] *= 2.0 ** 17
+    w.values[0] = O.from_f32(v, dtype)
+    got, qm, _ = _run(w, gpu, L)
+    # the error of sum_i p_i v_i scales with sum_i p_i |v_i| (each product and
+    # weight is rounded on its own), which the oracle's dense attention over
+    # |V| gives: TOL of that, and of 1 where it is smaller
+    for i in (0, 1, L // 2, L - 1):
+        for h in range(w.Hkv):
+            qh, kh, vh = qm[0, h * w.G:(h + 1) * w.G, i], w.keys[0][h][:T - L + i + 1], w.values[0][h][:T - L + i + 1]
+            ref = O.dense(qh, kh, vh, w.scale, dtype)
+            mag = O.dense(qh, kh, vh & np.uint16(0x7FFF), w.scale, dtype)
+            a = O.to_f32(got[0, h * w.G:(h + 1) * w.G, i], dtype).astype(np.float64)
+            err = float(np.max((np.abs(a - ref) - 0.5 * ulp(ref, dtype)) / np.maximum(1.0, mag)))
+            assert err <= TOL, f"query {i} head {h}: relative error {err:.3g}"
 
 
 def test_split_prefill_in_a_graph(gpu):
