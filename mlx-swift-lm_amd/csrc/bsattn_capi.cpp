@@ -24,6 +24,9 @@ using namespace bsattn;
 
 namespace {
 
+// words of the device metadata to set: index and value
+using Patches = std::vector<std::pair<int32_t, int32_t>>;
+
 thread_local std::string g_err;
 
 int fail(int code, const char* fmt, ...) noexcept {
@@ -87,6 +90,9 @@ struct bsattn_cache {
   bool stale = false;
   std::vector<std::vector<int32_t>> pages;
   std::vector<int32_t> free_pages;  // stack; back() is handed out next
+  // metadata words that a failed launch may have left unset (or set ahead of
+  // the host): sent before the next call's own (send_unsent)
+  Patches unsent;
   // opt-in per-kernel timing (bsattn_profile_*)
   bool profiling = false;
   std::vector<hipEvent_t> event_pool;
@@ -171,22 +177,67 @@ PatchBatch patch_batch(const std::pair<int32_t, int32_t>* p, size_t n) {
   return pb;
 }
 
-int flush_patches(bsattn_cache* c, std::vector<std::pair<int32_t, int32_t>>& p, hipStream_t s) {
+int send_patches(const bsattn_cache* c, const Patches& p, hipStream_t s) {
   for (size_t i = 0; i < p.size(); i += kMaxPatch) {
     const PatchBatch pb = patch_batch(p.data() + i, std::min<size_t>(kMaxPatch, p.size() - i));
     HIP_TRY(launch_patch(c->geo, pb, s), "patch launch");
   }
-  p.clear();
   return BSATTN_OK;
 }
 
+// What an earlier call could not send; every call that changes the metadata,
+// or launches work that reads it, starts here.  (The exports read block-table
+// entries of tokens already held, which have been sent.)
+int send_unsent(bsattn_cache* c, hipStream_t s) {
+  if (c->unsent.empty()) return BSATTN_OK;
+  if (int rc = send_patches(c, c->unsent, s)) return rc;
+  c->unsent.clear();
+  return BSATTN_OK;
+}
+
+// (after send_unsent)
+int flush_patches(bsattn_cache* c, Patches& p, hipStream_t s) {
+  const int rc = send_patches(c, p, s);
+  if (rc) c->unsent.swap(p);
+  return rc;
+}
+
+// The patches of an append, from the reservation of its pages (host state
+// already) to the last launch: unless sent() is called they are kept for the
+// next call, with the lengths the sequences still have, so that the device's
+// tables follow the host's whether or not a failed launch applied them.
+class AppendPatches {
+ public:
+  AppendPatches(bsattn_cache* c, const std::vector<int32_t>& seqs) : c_(c), seqs_(seqs) {}
+  ~AppendPatches() {
+    if (sent_) return;
+    for (size_t i = 0; i < seqs_.size() && lens_ + i < list.size(); ++i) list[lens_ + i].second = c_->len[seqs_[i]];
+    c_->unsent.swap(list);
+  }
+  AppendPatches(const AppendPatches&) = delete;
+  AppendPatches& operator=(const AppendPatches&) = delete;
+  // the lengths after n_tokens more (room for them is reserve_pages')
+  void lengths(int n_tokens) {
+    lens_ = list.size();
+    for (int s : seqs_) list.emplace_back(s, c_->len[s] + n_tokens);
+  }
+  void sent() { sent_ = true; }
+  Patches list;
+
+ private:
+  bsattn_cache* c_;
+  const std::vector<int32_t>& seqs_;
+  size_t lens_ = SIZE_MAX / 2;
+  bool sent_ = false;
+};
+
 // device-side capacity of a sequence: tokens its pages hold
-void cap_patch(const bsattn_cache* c, int seq, std::vector<std::pair<int32_t, int32_t>>& patches) {
+void cap_patch(const bsattn_cache* c, int seq, Patches& patches) {
   patches.emplace_back(c->geo.cap_off + seq, (int32_t)c->pages[seq].size() * c->d.block_size);
 }
 
 int release_pages(bsattn_cache* c, int seq, int keep_blocks,
-                  std::vector<std::pair<int32_t, int32_t>>& patches) {
+                  Patches& patches) {
   auto& pg = c->pages[seq];
   while ((int)pg.size() > keep_blocks) {
     c->free_pages.push_back(pg.back());
@@ -196,11 +247,12 @@ int release_pages(bsattn_cache* c, int seq, int keep_blocks,
   return BSATTN_OK;
 }
 
-// Reserve pages for new lengths; on failure nothing changes.  A sequence may
+// Reserve pages for new lengths, with room in patches for the lengths too; on
+// failure nothing changes.  A sequence may
 // already hold more pages than its new length needs (bsattn_reserve took them
 // ahead): it needs none, and its surplus is not counted against the others.
 int reserve_pages(bsattn_cache* c, const std::vector<int32_t>& seqs, int L,
-                  std::vector<std::pair<int32_t, int32_t>>& patches) {
+                  Patches& patches) {
   const int tb = c->d.block_size;
   int64_t need = 0;
   for (int s : seqs) {
@@ -214,7 +266,7 @@ int reserve_pages(bsattn_cache* c, const std::vector<int32_t>& seqs, int L,
     return fail(BSATTN_ERR_NO_PAGES, "page pool exhausted: need %lld pages, %zu free", (long long)need,
                 c->free_pages.size());
   // every allocation first (may throw), then the bookkeeping (cannot)
-  patches.reserve(patches.size() + (size_t)need + seqs.size());
+  patches.reserve(patches.size() + (size_t)need + 2 * seqs.size());
   for (int s : seqs) c->pages[s].reserve((c->len[s] + L + tb - 1) / tb);
   for (int s : seqs) {
     const int newlen = c->len[s] + L;
@@ -493,7 +545,9 @@ int bsattn_reserve(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int3
   if (rc) return rc;
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
-  std::vector<std::pair<int32_t, int32_t>> patches;
+  rc = send_unsent(c, (hipStream_t)stream);
+  if (rc) return rc;
+  Patches patches;
   rc = reserve_pages(c, seqs, n_tokens, patches);
   if (rc) return rc;
   return flush_patches(c, patches, (hipStream_t)stream);
@@ -512,6 +566,8 @@ int bsattn_append_step(bsattn_cache* c, const void* k, const void* v, const int3
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
   hipStream_t s = (hipStream_t)stream;
+  rc = send_unsent(c, s);
+  if (rc) return rc;
   const size_t row = (size_t)c->geo.hkv * kHeadDim;  // elements per sequence
   for (int i0 = 0; i0 < n_seqs; i0 += kMaxBatch) {
     AppendBatch ab{};
@@ -535,6 +591,7 @@ int bsattn_sync(bsattn_cache* c, void* stream) try {
   if (!c) return fail(BSATTN_ERR_INVALID, "null argument");
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
+  if (int rs = send_unsent(c, (hipStream_t)stream)) return rs;
   HIP_TRY(hipStreamSynchronize((hipStream_t)stream), "hipStreamSynchronize");
   std::vector<int32_t> dev(c->d.max_seqs);
   HIP_TRY(hipMemcpy(dev.data(), c->geo.meta, dev.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy(lengths)");
@@ -561,11 +618,14 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   if (rc) return rc;
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
-  std::vector<std::pair<int32_t, int32_t>> patches;
-  rc = reserve_pages(c, seqs, n_tokens, patches);
+  rc = send_unsent(c, s);
+  if (rc) return rc;
+  AppendPatches ap(c, seqs);
+  rc = reserve_pages(c, seqs, n_tokens, ap.list);
   if (rc) return rc;
   const int tb = c->d.block_size;
-  for (int s_ : seqs) patches.emplace_back(s_, c->len[s_] + n_tokens);
+  ap.lengths(n_tokens);
+  const Patches& patches = ap.list;
   // first block that a sequence's append touches, and the one past the last
   auto touched = [&](int sq) {
     return std::make_pair(c->len[sq] / tb, (int)(((int64_t)c->len[sq] + n_tokens + tb - 1) / tb));
@@ -584,7 +644,7 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
       for (int b = b0; b < b1; ++b) pg.page[at++] = c->pages[seqs[i]][b];
     }
   } else {
-    rc = flush_patches(c, patches, s);
+    rc = send_patches(c, patches, s);
     if (rc) return rc;
   }
   for (int i0 = 0; i0 < n_seqs; i0 += kMaxBatch) {
@@ -604,6 +664,7 @@ int append_impl(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
     prof_collect(c, prof);
     if (e != hipSuccess) return hip_fail(e, "append launch");
   }
+  ap.sent();
   for (int s_ : seqs) c->len[s_] += n_tokens;
   return BSATTN_OK;
 }
@@ -732,6 +793,7 @@ enum class Op { Select, Attend, Decode };
 static int run_entries(bsattn_cache* c, Op op, const void* q, const Entry* es, int n, int nseq, int qhs,
                        const int32_t* idx_in, int32_t* idx_out, float scale, void* out, hipStream_t s,
                        const Workspace& ws, bool profile = true) {
+  if (int rs = send_unsent(c, s)) return rs;
   const Geometry& g = c->geo;
   const size_t idx_row = (size_t)g.hkv * g.nsel_max;
   const int waves = attend_waves(g, nseq);
@@ -896,18 +958,17 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
   hipStream_t s = (hipStream_t)stream;
-  std::vector<std::pair<int32_t, int32_t>> patches;
-  rc = reserve_pages(c, seqs, 1, patches);
+  rc = send_unsent(c, s);
   if (rc) return rc;
-  for (int sq : seqs) patches.emplace_back(sq, c->len[sq] + 1);
-  if (patches.size() > (size_t)kMaxPatch) {  // applied by a launch of their own
-    rc = flush_patches(c, patches, s);
-    if (rc) return rc;
-  }
+  AppendPatches patches(c, seqs);
+  rc = reserve_pages(c, seqs, 1, patches.list);
+  if (rc) return rc;
+  patches.lengths(1);
+  static_assert(3 * kMaxBatch <= kMaxPatch, "a step's page, capacity and length of every sequence fit its launch");
   StepAppend ap{};
   ap.k = (const uint16_t*)k;
   ap.v = (const uint16_t*)v;
-  ap.pb = patch_batch(patches.data(), patches.size());
+  ap.pb = patch_batch(patches.list.data(), patches.list.size());
   SeqBatch b{};
   b.n = n_seqs;
   b.qhs = kHeadDim;
@@ -924,6 +985,7 @@ int bsattn_append_decode(bsattn_cache* c, const void* k, const void* v, const vo
                                      attend_waves(g, n_seqs), scale, out, c->partials, c->arrive, s, prof);
   prof_collect(c, prof);
   if (e != hipSuccess) return hip_fail(e, "append-decode launch");
+  patches.sent();
   for (int sq : seqs) c->len[sq] += 1;
   return BSATTN_OK;
 } catch (...) {
@@ -985,6 +1047,8 @@ int bsattn_prefill(bsattn_cache* c, const void* q, const int32_t* seq_ids, int32
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
   hipStream_t s = (hipStream_t)stream;
+  rc = send_unsent(c, s);
+  if (rc) return rc;
   // q / out [n, Hq, L, D]: a launch takes whole sequences whose row offsets fit int32
   const int64_t per_seq = (int64_t)c->geo.hq * n_query * kHeadDim;
   const int step = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxBatch, INT32_MAX / per_seq));
@@ -1025,7 +1089,9 @@ int bsattn_trim(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, int32_t
   if (rc) return rc;
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
-  std::vector<std::pair<int32_t, int32_t>> patches;
+  rc = send_unsent(c, (hipStream_t)stream);
+  if (rc) return rc;
+  Patches patches;
   patches.reserve(2 * seqs.size());  // the loop below then cannot throw
   for (int i = 0; i < n_seqs; ++i) {
     const int sq = seqs[i];
@@ -1048,7 +1114,9 @@ int bsattn_reset(bsattn_cache* c, const int32_t* seq_ids, int32_t n_seqs, void* 
   if (rc) return rc;
   DeviceGuard dg(c->d.device);
   if (!dg.ok) return fail(BSATTN_ERR_HIP, "hipSetDevice(%d) failed", c->d.device);
-  std::vector<std::pair<int32_t, int32_t>> patches;
+  rc = send_unsent(c, (hipStream_t)stream);
+  if (rc) return rc;
+  Patches patches;
   patches.reserve(2 * seqs.size());  // the loop below then cannot throw
   for (int sq : seqs) {
     c->len[sq] = 0;
@@ -1071,6 +1139,7 @@ int bsattn_copy(const bsattn_cache* src, bsattn_cache** out, void* stream) try {
     c->len = src->len;
     c->pages = src->pages;
     c->free_pages = src->free_pages;
+    c->unsent = src->unsent;
   } catch (...) {
     bsattn_cache_destroy(c);
     throw;
