@@ -567,8 +567,12 @@ __global__ __launch_bounds__(64 * W) void k_decode(Geometry geo, SeqBatch sb,
     store_empty<G>(s_m[wave], s_l[wave], s_o[wave], lane);
   }
   __syncthreads();
-  attend_merge<DT, G, W, true>(geo, sb, bi, h, split, S, s_m, s_l, s_o, out, partials);
-  if (arrive) arrive_merge<DT, G, W>(geo, sb, bi, h, S, arrive + pair, partials, out);
+  if (arrive) {
+    attend_merge<DT, G, W, true>(geo, sb, bi, h, split, S, s_m, s_l, s_o, out, partials);
+    arrive_merge<DT, G, W>(geo, sb, bi, h, S, arrive + pair, partials, out);
+  } else {
+    attend_merge<DT, G, W>(geo, sb, bi, h, split, S, s_m, s_l, s_o, out, partials);
+  }
   if constexpr (APPEND) {
     // the completed block's summary: 16 lanes fold its keys from LDS (written
     // before the barriers of the merge) in token order
@@ -642,7 +646,15 @@ hipError_t decode_impl(const Geometry& g, const SeqBatch& b, int nseq, const voi
   const uint16_t* qq = (const uint16_t*)q;
   uint16_t* oo = (uint16_t*)out;
   const int lf = len_first ? 1 : 0;
-  const bool merge = p.S > 1 && p.S <= kArriveSplits && !prof;
+  // The launch merges its splits itself up to 1.5 workgroups per CU: there it
+  // saves the combine launch.  With more (a multi-token decode), a workgroup
+  // that stores its partials past its cache and merges holds up the next one
+  // on its CU.  Steps of L tokens, fp16, with the merge and with the combine:
+  // one sequence of 4k tokens, 9 splits, L = 4 (288 workgroups) 13.0 and 13.7
+  // us, L = 6 (432) 13.7 and 13.7, L = 16 29.1 and 27.5; 8 of 2k tokens, 4
+  // splits, L = 1 (256) 15.2 and 17.4, L = 4 (1024) 37.7 and 34.7, L = 16 140
+  // and 123.
+  const bool merge = p.S > 1 && p.S <= kArriveSplits && !prof && 2 * pairs * p.S <= 3 * g.cus;
   arrive = merge ? arrive + (p.S - 1) * kArrivePairs : nullptr;
   if (g.dtype == 0) {
     if (g.tb == 64) decode_g<0, 64, MD>(g, p, grid, b, qq, idx, sl2, oo, partials, arrive, lf, ap, s, prof);

@@ -90,3 +90,20 @@ def test_merge_in_the_launch(gpu, dtype, B, Hkv, G, K):
         torch.cuda.synchronize()
         assert torch.equal(o.view(torch.int16), ref), f"replay {n}"
         assert torch.equal(c.decode(q, w.scale).view(torch.int16), ref)
+
+
+@pytest.mark.parametrize("L", [2, 3, 4, 16])
+def test_merge_of_a_multi_token_decode(gpu, L):
+    """128 workgroups for each query token: up to 1.5 per CU the launch merges
+    its splits, with more the combine launch does, as when profiled."""
+    import torch
+    log(f"[small decode] multi L={L}")
+    w = make_workload(7350, B=2, Hq=32, Hkv=8, T=4000, Tb=64, dtype="bf16", top_k=30, lens=[4000, 3700])
+    c = new_cache(w)
+    fill(c, w, gpu)
+    q = torch.randn((2, 32, L, 128), generator=torch.Generator().manual_seed(L)).to(torch.bfloat16).to(gpu)
+    c.profile(True)
+    ref = c.decodeMulti(q, w.scale)
+    c.profile(False)
+    for n in range(4):
+        assert torch.equal(c.decodeMulti(q, w.scale).view(torch.int16), ref.view(torch.int16)), f"call {n}"
