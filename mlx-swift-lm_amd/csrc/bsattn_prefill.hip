@@ -29,6 +29,14 @@ __device__ __forceinline__ f32x16 mfma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// all bits of the 16-bit elements whose magnitude bits are `lim` or more
+__device__ __forceinline__ u32x4 at_least16(u32x4 w, uint32_t lim) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    w[k] = ((w[k] & 0x7FFFu) >= lim ? 0x0000FFFFu : 0u) | ((w[k] >> 16 & 0x7FFFu) >= lim ? 0xFFFF0000u : 0u);
+  return w;
+}
+
 // a workgroup barrier that orders LDS only: the global loads of later units
 // stay in flight across it
 __device__ __forceinline__ void unit_barrier() {
@@ -47,21 +55,21 @@ __device__ __forceinline__ float pair_sum(float x) {
   return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
-constexpr int kPfWaves = 8;           // waves per workgroup
+constexpr int kPfWaves = 8;           // waves per workgroup (half as many for few tiles: prefill_width)
 constexpr int kPfCols = 32;           // MFMA columns per wave
 constexpr int kPfSplits = 16;         // most parts a tile's tokens are split into
 constexpr float kNoMax = -3.0e38f;    // running maximum of a column that has seen nothing
 
-// one wave's share of a 32-token unit, as loaded: K fragment `wave` and V
-// fragment `wave` (16 bytes a lane), or their codes and one token's scales
-template <int KB>
+// one wave's share of a 32-token unit, as loaded: F of its 8 K and of its 8 V
+// fragments (16 bytes a lane), or their codes and one token's scales
+template <int KB, int F>
 struct Staged {
-  uint32_t k[KB / 4], v[KB / 4];
+  uint32_t k[F][KB / 4], v[F][KB / 4];
   u32x4 e;
 };
-template <>
-struct Staged<0> {
-  u32x4 k, v;
+template <int F>
+struct Staged<0, F> {
+  u32x4 k[F], v[F];
 };
 
 // ---------------------------------------------------------------------------
@@ -70,7 +78,7 @@ struct Staged<0> {
 // holding T tokens sits at position T - L + i and attends to tokens
 // [0, T - L + i] (the causal mask BaseKVCache.makeMask gives for n > 1).
 // A wave owns 32 MFMA columns, each a (query token, q head) pair (32 / G
-// tokens x the G heads of kv head h); the workgroup's 8 waves take
+// tokens x the G heads of kv head h); the workgroup's W waves take
 // consecutive tokens of one (sequence, kv head) and walk its tokens in units
 // of 32, with an online softmax per column:
 //   S^T[token][col] = K[token] . Q[col]        (A = K rows, B = Q^T)
@@ -100,8 +108,10 @@ struct Staged<0> {
 //
 // V of a bf16 cache is converted to fp16 on its way to LDS (exact for
 // |v| < 65520 down to the fp16 normal range) for an fp16 PV product without
-// the hi / lo split of P; a unit holding a value fp16 cannot take is flagged,
-// and its PV runs in bf16 with P as hi + lo from the cache's own fragments.
+// the hi / lo split of P.  A value fp16 cannot take is left out there and the
+// unit noted; the noted units are gone through once more after the last one,
+// for those values alone, in bf16 with P as hi + lo from the cache's own
+// fragments.
 // Codes of an affine cache (KB = 4 / 8 bits, fp16 q / out) are dequantized on
 // the way, as fp16 values fl16(scale * code + bias) (one packed fused
 // multiply-add per pair, so each is the correctly rounded value).
@@ -122,9 +132,9 @@ struct Staged<0> {
 // TFLOP/s), int4 2494 -> 2373 us; one sequence, split in 4, 362 -> 296 us; a
 // prompt of 8191 fp16 tokens 575 -> 581 us (16x16x32 MFMAs in 4-wave
 // workgroups, one unit ahead: 2839, 3000, 1125 and 687 us).
-// grid (ceil(L / (256 / G)) * Hkv * n * nsplit)
+// grid (ceil(L / (32 W / G)) * Hkv * n * nsplit), W = 8 or 4 waves
 // ---------------------------------------------------------------------------
-template <int DT, int KB>
+template <int DT, int KB, int W>
 __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatch sb, int L, int lg, int gx,
                                                           int nsplit, const uint16_t* __restrict__ q,
                                                           float sl2, uint16_t* __restrict__ out,
@@ -136,9 +146,20 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   // is skipped for most units; O^T / l is unchanged by the choice
   constexpr float kLazy = 8.f;
   constexpr bool CV = KB == 0 && DT == 1;
+  constexpr int F = 8 / W;  // K, and V, fragments of a unit that a wave loads: wave + W i
+  using St = Staged<KB, F>;
   __shared__ __align__(16) u32x4 s_k[4][8 * 64], s_v[8][8 * 64];
-  __shared__ __align__(16) u32x4 s_ent[KB ? kPfWaves : 1][KB ? 32 : 1];  // each wave's copy of a unit's scales / biases
-  __shared__ int s_flag[8][kPfWaves];  // CV: wave w's V fragment of the slot's unit holds a value fp16 cannot take
+  __shared__ __align__(16) u32x4 s_ent[KB ? W : 1][KB ? 32 : 1];  // each wave's copy of a unit's scales / biases
+  // CV: units whose V holds an element that is left to the end, bit x - ua
+  // (tables are at most 12288 blocks wide)
+  constexpr int ODDW = CV ? 2 * 12288 / 32 + 1 : 1;
+  __shared__ uint32_t s_odd[ODDW];
+  __shared__ int s_anyodd;
+  if constexpr (CV) {
+    for (int i = threadIdx.x; i < ODDW; i += 64 * W) s_odd[i] = 0u;
+    if (threadIdx.x == 0) s_anyodd = 0;
+    unit_barrier();
+  }
   const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 31, hh = lane >> 5;
   // XCD-grouped workgroup order (a bijection on [0, total))
@@ -148,7 +169,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   const int pair = uniform(run_of / nsplit), part = run_of - pair * nsplit;
   const int bi = uniform(pair / geo.hkv), h = pair - bi * geo.hkv;
   const int qpw = kPfCols >> lg;            // query tokens per wave
-  const int twg = tile * kPfWaves * qpw;    // the workgroup's first query token
+  const int twg = tile * W * qpw;           // the workgroup's first query token
   const bool active = uniform(twg + wave * qpw < L);
   const int seq = uniform(sb.ids[bi]);
   const int T = uniform(geo.meta[seq]);
@@ -168,13 +189,15 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
     for (int s = 0; s < 8; ++s) qf[s] = tq < L ? *(const u32x4*)(src + 16 * s) ^ qflip : u32x4{0u, 0u, 0u, 0u};
   }
   const int ksh = geo.tb == 64 ? 1 : 0;  // log2 of the units of a block
-  const int last = T - L + min(L - 1, twg + kPfWaves * qpw - 1);  // the workgroup's last position
+  const int last = T - L + min(L - 1, twg + W * qpw - 1);  // the workgroup's last position
   const int nunit = last / 32 + 1;
-  // (at most 2^26 units in at most 16 parts; kept in scalar registers, so that
-  // the loop's counters, page lookups and addresses are scalar too)
+  // (at most 24576 units, of 12288 blocks, in at most 16 parts; kept in scalar
+  // registers, so that the loop's counters, page lookups and addresses are
+  // scalar too)
   const int ua = uniform((int)((uint32_t)nunit * part / nsplit)), ub = uniform((int)((uint32_t)nunit * (part + 1) / nsplit));
   // units below nfull are whole and visible to every column of the workgroup
   const int nfull = uniform(min((T - L + twg + 1) / 32, ub));
+  constexpr uint32_t ODD = 0x4780u;  // magnitude bits of 65536 in bf16
 
   // --- units from memory: this wave's fragments, in the slab's own order
   const int32_t* bt = block_table(geo, seq);
@@ -182,120 +205,142 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   int pbase = ua >> ksh;  // lane i of pagev: page of block pbase + i
   int pagev = bt[min(pbase + lane, lastblk)];
   const uint32_t lane16 = 16 * (threadIdx.x & 63);
-  auto load = [&](int x, Staged<KB>& st) __attribute__((always_inline)) {
+  auto load = [&](int x, St& st) __attribute__((always_inline)) {
     x = max(min(x, ub - 1), ua);
     const int blk = x >> ksh, sub = x & ((1 << ksh) - 1);
     if (blk >= pbase + 64) {
-      pbase += 64;
+      pbase = blk;
       pagev = bt[min(pbase + lane, lastblk)];
       __builtin_amdgcn_s_waitcnt(0x0F70);  // here, every 64 blocks, and not at each use of pagev
     }
     const int page = __builtin_amdgcn_readlane(pagev, blk - pbase);
     const uint8_t* slab = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes;
     const uint8_t *ks = slab + geo.k_off, *vs = slab + geo.v_off;
-    if constexpr (KB == 0) {
-      st.k = *(const u32x4*)(ks + (8 * sub + wave) * 1024 + lane16);
-      st.v = *(const u32x4*)(vs + ((wave << ksh) + sub) * 1024 + lane16);
-    } else {
-      if constexpr (KB == 4) {
-        st.k[0] = *(const uint32_t*)(ks + (2 * sub + (wave >> 2)) * 1024 + 4 * (wave & 3) + lane16);
-        st.v[0] = *(const uint32_t*)(vs + (((wave >> 2) << ksh) + sub) * 1024 + 4 * (wave & 3) + lane16);
+#pragma unroll
+    for (int i = 0; i < F; ++i) {
+      const int f = wave + W * i;
+      if constexpr (KB == 0) {
+        st.k[i] = *(const u32x4*)(ks + (8 * sub + f) * 1024 + lane16);
+        st.v[i] = *(const u32x4*)(vs + ((f << ksh) + sub) * 1024 + lane16);
+      } else if constexpr (KB == 4) {
+        st.k[i][0] = *(const uint32_t*)(ks + (2 * sub + (f >> 2)) * 1024 + 4 * (f & 3) + lane16);
+        st.v[i][0] = *(const uint32_t*)(vs + (((f >> 2) << ksh) + sub) * 1024 + 4 * (f & 3) + lane16);
       } else {
-        const uint2 a = *(const uint2*)(ks + (4 * sub + (wave >> 1)) * 1024 + 8 * (wave & 1) + lane16);
-        const uint2 b = *(const uint2*)(vs + (((wave >> 1) << ksh) + sub) * 1024 + 8 * (wave & 1) + lane16);
-        st.k[0] = a.x;
-        st.k[1] = a.y;
-        st.v[0] = b.x;
-        st.v[1] = b.y;
+        const uint2 a = *(const uint2*)(ks + (4 * sub + (f >> 1)) * 1024 + 8 * (f & 1) + lane16);
+        const uint2 b = *(const uint2*)(vs + (((f >> 1) << ksh) + sub) * 1024 + 8 * (f & 1) + lane16);
+        st.k[i][0] = a.x;
+        st.k[i][1] = a.y;
+        st.v[i][0] = b.x;
+        st.v[i][1] = b.y;
       }
+    }
+    if constexpr (KB != 0) {
       const int x32 = lane & 31;
       st.e = *(const u32x4*)(slab + geo.sb_off + (((x32 >> 3) * (geo.tb >> 2)) + 8 * sub + (x32 & 7)) * 16);
     }
   };
+  // f16 pairs (s * c + b): c from the f16 values OFF + c / INV_UNIT exactly
+  [[maybe_unused]] auto deq = [&](u32x4 hv, const uint32_t* sp, const uint32_t* bp) __attribute__((always_inline)) {
+    using QC = QCode<KB ? KB : 4>;
+    const f16x2 unit2 = {(_Float16)QC::INV_UNIT, (_Float16)QC::INV_UNIT};
+    const f16x2 off2 = {(_Float16)(-QC::OFF * QC::INV_UNIT), (_Float16)(-QC::OFF * QC::INV_UNIT)};
+    u32x4 o4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      // (a vector element is copied out first: __builtin_bit_cast of
+      // hv[k] itself reads element 0 with this compiler)
+      const uint32_t w = hv[k];
+      const f16x2 c = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, w), unit2, off2);
+      o4[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, sp[k]), c,
+                                                                    __builtin_bit_cast(f16x2, bp[k])));
+    }
+    return o4;
+  };
+  [[maybe_unused]] auto codes = [&](const uint32_t* w) __attribute__((always_inline)) {
+    if constexpr (KB == 4) return nib_to_f16(w[0]);
+    else return byte_to_f16(w[0], w[1]);
+  };
+  // w without the elements that are left to the end, with the unit noted when
+  // there are any
+  [[maybe_unused]] auto drop = [&](int r, u32x4 w) __attribute__((always_inline)) {
+    u16x2 big = {0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t mag = w[k] & 0x7FFF7FFFu;
+      big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2, mag));
+    }
+    constexpr uint32_t UP = 0x10001u * (0x8000u - ODD);  // carries ODD and more into the sign bits
+    if (__builtin_amdgcn_ballot_w64(((__builtin_bit_cast(uint32_t, big) + UP) & 0x80008000u) != 0u) != 0) {
+      w &= ~at_least16(w, ODD);
+      if (lane == 0) {
+        atomicOr(&s_odd[min(r >> 5, ODDW - 1)], 1u << (r & 31));
+        s_anyodd = 1;
+      }
+    }
+    return w;
+  };
   // --- and into LDS, as 16-bit fragments; r: the unit's index from ua
-  auto stage = [&](int r, const Staged<KB>& st, auto mask_tag) __attribute__((always_inline)) {
+  auto stage = [&](int r, const St& st, auto mask_tag, auto raw_tag) __attribute__((always_inline)) {
+    constexpr bool RAW = decltype(raw_tag)::value;
     if constexpr (KB != 0) {
       // the unit's scale / bias entries through this wave's own LDS rows
       // (a wave's LDS accesses complete in order)
       s_ent[wave][lane & 31] = st.e;
       wave_lds_order();
     }
-    u32x4 kw, vw;
-    if constexpr (KB == 0) {
-      kw = st.k;
-      vw = st.v;
-      if constexpr (CV) {
-        // a bf16 value of magnitude >= 65536 (or inf / NaN) flags the unit:
-        // the largest magnitude bits of either half, >= 0x4780
-        u16x2 big = {0, 0};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t x = vw[k], mag = x & 0x7FFF7FFFu;
-          big = __builtin_elementwise_max(big, __builtin_bit_cast(u16x2, mag));
-          vw[k] = cvt_pk<0>(__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u));
-        }
-        const bool any =
-            __builtin_amdgcn_ballot_w64(((__builtin_bit_cast(uint32_t, big) + 0x38803880u) & 0x80008000u) != 0u) != 0;
-        if (lane == 0) s_flag[r & 7][wave] = any ? 1 : 0;
-      }
-    } else {
-      using QC = QCode<KB>;
-      // f16 pairs (s * c + b): c from the f16 values OFF + c / INV_UNIT exactly
-      auto deq = [&](u32x4 hv, const uint32_t* sp, const uint32_t* bp) __attribute__((always_inline)) {
-        const f16x2 unit2 = {(_Float16)QC::INV_UNIT, (_Float16)QC::INV_UNIT};
-        const f16x2 off2 = {(_Float16)(-QC::OFF * QC::INV_UNIT), (_Float16)(-QC::OFF * QC::INV_UNIT)};
-        u32x4 o4;
+    for (int i = 0; i < F; ++i) {
+      const int f = wave + W * i;
+      u32x4 kw, vw;
+      if constexpr (KB == 0) {
+        kw = st.k[i];
+        vw = st.v[i];
+        if constexpr (CV) {
+          if constexpr (!RAW) vw = drop(r, vw);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          // (a vector element is copied out first: __builtin_bit_cast of
-          // hv[k] itself reads element 0 with this compiler)
-          const uint32_t w = hv[k];
-          const f16x2 c = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, w), unit2, off2);
-          o4[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, sp[k]), c,
-                                                                        __builtin_bit_cast(f16x2, bp[k])));
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t x = vw[k];
+            vw[k] = cvt_pk<0>(__uint_as_float(x << 16), __uint_as_float(x & 0xFFFF0000u));
+          }
         }
-        return o4;
-      };
-      auto codes = [&](const uint32_t* w) __attribute__((always_inline)) {
-        if constexpr (KB == 4) return nib_to_f16(w[0]);
-        else return byte_to_f16(w[0], w[1]);
-      };
-      const uint32_t* ent = (const uint32_t*)s_ent[wave];
-      {
-        // row m of QK key tile t is token 8 (m / 4) + 4 t + m % 4 of the unit
-        const int t = wave >> 2, m = lane & 15;
-        const int x = 8 * (m >> 2) + 4 * t + (m & 3);
-        const uint32_t sel = (wave & 2) ? 0x03020302u : 0x01000100u;  // dim group of k-step wave & 3
-        const uint32_t s2 = __builtin_amdgcn_perm(ent[4 * x], ent[4 * x], sel);
-        const uint32_t b2 = __builtin_amdgcn_perm(ent[4 * x + 1], ent[4 * x + 1], sel);
-        const uint32_t sp[4] = {s2, s2, s2, s2}, bp[4] = {b2, b2, b2, b2};
-        kw = deq(codes(st.k), sp, bp);
-      }
-      {
-        // (v scale, v bias) of tokens 8 g + 2 k, 8 g + 2 k + 1 as f16 pairs
-        const int g = lane >> 4;
-        uint32_t sp[4], bp[4];
-        const uint32_t sel = (wave >> 2) ? 0x07060302u : 0x05040100u;
+      } else {
+        const uint32_t* ent = (const uint32_t*)s_ent[wave];
+        {
+          // row m of QK key tile t is token 8 (m / 4) + 4 t + m % 4 of the unit
+          const int t = f >> 2, m = lane & 15;
+          const int x = 8 * (m >> 2) + 4 * t + (m & 3);
+          const uint32_t sel = (f & 2) ? 0x03020302u : 0x01000100u;  // dim group of k-step f & 3
+          const uint32_t s2 = __builtin_amdgcn_perm(ent[4 * x], ent[4 * x], sel);
+          const uint32_t b2 = __builtin_amdgcn_perm(ent[4 * x + 1], ent[4 * x + 1], sel);
+          const uint32_t sp[4] = {s2, s2, s2, s2}, bp[4] = {b2, b2, b2, b2};
+          kw = deq(codes(st.k[i]), sp, bp);
+        }
+        {
+          // (v scale, v bias) of tokens 8 g + 2 k, 8 g + 2 k + 1 as f16 pairs
+          const int g = lane >> 4;
+          uint32_t sp[4], bp[4];
+          const uint32_t sel = (f >> 2) ? 0x07060302u : 0x05040100u;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint2 e0 = *(const uint2*)(ent + 4 * (8 * g + 2 * k) + 2), e1 = *(const uint2*)(ent + 4 * (8 * g + 2 * k + 1) + 2);
-          sp[k] = __builtin_amdgcn_perm(e1.x, e0.x, sel);
-          bp[k] = __builtin_amdgcn_perm(e1.y, e0.y, sel);
+          for (int k = 0; k < 4; ++k) {
+            const uint2 e0 = *(const uint2*)(ent + 4 * (8 * g + 2 * k) + 2), e1 = *(const uint2*)(ent + 4 * (8 * g + 2 * k + 1) + 2);
+            sp[k] = __builtin_amdgcn_perm(e1.x, e0.x, sel);
+            bp[k] = __builtin_amdgcn_perm(e1.y, e0.y, sel);
+          }
+          vw = deq(codes(st.v[i]), sp, bp);
         }
-        vw = deq(codes(st.v), sp, bp);
       }
+      if constexpr (decltype(mask_tag)::value) {
+        // V of tokens past the sequence end (stale page data) is zeroed
+        const int valid = T - 32 * (ua + r), g = lane >> 4;
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const int tk = 8 * g + 2 * jj;
+          vw[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
+        }
+      }
+      s_k[r & 3][f * 64 + lane] = kw;
+      s_v[r & 7][f * 64 + lane] = vw;
     }
-    if constexpr (decltype(mask_tag)::value) {
-      // V of tokens past the sequence end (stale page data) is zeroed
-      const int valid = T - 32 * (ua + r), g = lane >> 4;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int tk = 8 * g + 2 * jj;
-        vw[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
-      }
-    }
-    s_k[r & 3][wave * 64 + lane] = kw;
-    s_v[r & 7][wave * 64 + lane] = vw;
     if constexpr (KB != 0) wave_lds_order();
   };
 
@@ -333,13 +378,14 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
     x = fmaxf(fmaxf(x, a[14]), a[15]);
     return fmaxf(x, y);
   };
-  // step r: `cur` holds S of unit r, `nxt` takes that of unit r + 1.  BIG: the
-  // unit's V holds a value fp16 cannot take
-  int flag = 0;  // CV: whether the next step's unit does
-  auto step = [&](int r, f32x16& cur, f32x16& nxt, Staged<KB>& st, auto act, auto mask_tag, auto big_tag, bool sync)
+  // step r: `cur` holds S of unit r, `nxt` takes that of unit r + 1.  MASK:
+  // the units up to r + 4 may be partial, or not visible to every column.
+  // (The two score tiles and the two staged units stay in their registers: the
+  // steps come in pairs that name them the other way round.  Swapping them
+  // instead made the masked steps spill, and wait for the loads in flight.)
+  auto step = [&](int r, f32x16& cur, f32x16& nxt, St& st, auto act, auto mask_tag, bool sync)
       __attribute__((always_inline)) {
     constexpr bool ACT = decltype(act)::value;
-    [[maybe_unused]] int fnext = 0;
     if constexpr (ACT) {
       // the column's maximum is needed only when some lane's scores pass the
       // raising threshold thr = (m + kLazy) / sc
@@ -356,9 +402,8 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
 #pragma unroll
           for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       }
-      if constexpr (CV) fnext = s_flag[(r + 1) & 7][lane & 7];
     }
-    stage(r + 3, st, mask_tag);
+    stage(r + 3, st, mask_tag, std::false_type{});
     load(ua + r + 5, st);
     if constexpr (ACT) {
       nxt = scores(r + 1);
@@ -368,25 +413,93 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
 #pragma unroll
       for (int i = 1; i < 16; ++i) ps += cur[i];
       l += ps;  // this lane's tokens; the column's halves are summed at the end
-      if constexpr (decltype(big_tag)::value) {
-        // bf16 P as hi + lo against the cache's own V fragments
-        const int x = ua + r, sub = x & ((1 << ksh) - 1);
-        const uint8_t* vs = geo.pool + ((size_t)uniform(bt[x >> ksh]) * geo.hkv + h) * geo.slab_bytes + geo.v_off;
+      const u32x4* vp = s_v[r & 7] + vl;
+      u32x4 pf[2];
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) pf[kk][jj] = cvt_pk<0>(cur[8 * kk + 2 * jj], cur[8 * kk + 2 * jj + 1]);
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) o[dt] = mfma32x32x16<0>(vp[dt * 128 + kk * 32], pf[kk], o[dt]);
+      lm = lane_max(nxt, r + 1, mask_tag);
+    }
+    if (sync) unit_barrier();
+  };
+
+  St st0, st1;
+  f32x16 sa, sb2;
+  load(ua, st0);
+  load(ua + 1, st1);
+  stage(0, st0, std::true_type{}, std::false_type{});
+  load(ua + 2, st0);
+  stage(1, st1, std::true_type{}, std::false_type{});
+  load(ua + 4, st1);
+  stage(2, st0, std::true_type{}, std::false_type{});
+  load(ua + 3, st0);
+  unit_barrier();
+  if (active) {
+    sa = scores(0);
+    lm = lane_max(sa, 0, std::true_type{});
+  }
+  unit_barrier();
+  // every wave takes ub - ua steps (a barrier after every second one); a wave
+  // past the last query token only loads and stages.  The steps whose units
+  // (up to r + 4) are whole and visible to every column come first, in pairs.
+  auto run = [&](auto act) __attribute__((always_inline)) {
+    const int n = ub - ua, plain = nfull - ua - 4;  // pairs r, r + 1 with r + 4 < nfull - ua
+    int r = 0;
+#pragma unroll 1
+    for (; r < plain; r += 2) {
+      step(r, sa, sb2, st0, act, std::false_type{}, false);
+      step(r + 1, sb2, sa, st1, act, std::false_type{}, true);
+    }
+#pragma unroll 1
+    for (; r < n; r += 2) {
+      step(r, sa, sb2, st0, act, std::true_type{}, false);
+      if (r + 1 == n) break;
+      step(r + 1, sb2, sa, st1, act, std::true_type{}, true);
+    }
+  };
+  if (active) run(std::true_type{});
+  else run(std::false_type{});
+  if constexpr (CV) {
+    unit_barrier();
+    if (uniform(s_anyodd) != 0) {
+#pragma unroll 1
+      for (int r = 0; r < ub - ua; ++r) {
+        if ((uniform((int)s_odd[r >> 5]) >> (r & 31) & 1) == 0) continue;
+        const int x = ua + r, blk = x >> ksh;
+        pbase = blk;
+        pagev = bt[min(pbase + lane, lastblk)];
+        load(x, st0);
+        unit_barrier();
+        stage(r, st0, std::true_type{}, std::true_type{});
+        unit_barrier();
+        if (!active) continue;
+        sa = scores(r);
+        lane_max(sa, r, std::true_type{});
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sa[i] = __builtin_amdgcn_exp2f(fmaf(sa[i], sc, -m));
+        const uint8_t* vs = geo.pool + ((size_t)uniform(bt[blk]) * geo.hkv + h) * geo.slab_bytes + geo.v_off +
+                            (x & ((1 << ksh) - 1)) * 1024;
+        const int tile16 = 1024 << ksh;  // bytes from one 16-dim tile to the next
         const int valid = T - 32 * x;
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
           u32x4 ph, pl;
 #pragma unroll
           for (int jj = 0; jj < 4; ++jj) {
-            const float p0 = cur[8 * kk + 2 * jj], p1 = cur[8 * kk + 2 * jj + 1];
+            const float p0 = sa[8 * kk + 2 * jj], p1 = sa[8 * kk + 2 * jj + 1];
             const uint32_t w = cvt_pk<1>(p0, p1);
             ph[jj] = w;
             pl[jj] = cvt_pk<1>(p0 - __uint_as_float(w << 16), p1 - __uint_as_float(w & 0xFFFF0000u));
           }
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt) {
-            u32x4 vf = *(const u32x4*)(vs + (((2 * dt + (col >> 4)) << ksh) + sub) * 1024 +
-                                       ((col & 15) + 16 * (2 * kk + hh)) * 16);
+            u32x4 vf = *(const u32x4*)(vs + (2 * dt + (col >> 4)) * tile16 + ((col & 15) + 16 * (2 * kk + hh)) * 16);
+            vf &= at_least16(vf, ODD);
 #pragma unroll
             for (int jj = 0; jj < 4; ++jj) {
               const int tk = 8 * (2 * kk + hh) + 2 * jj;
@@ -396,85 +509,9 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
             o[dt] = mfma32x32x16<1>(vf, pl, o[dt]);
           }
         }
-      } else {
-        const u32x4* vp = s_v[r & 7] + vl;
-        u32x4 pf[2];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) pf[kk][jj] = cvt_pk<0>(cur[8 * kk + 2 * jj], cur[8 * kk + 2 * jj + 1]);
-#pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int kk = 0; kk < 2; ++kk) o[dt] = mfma32x32x16<0>(vp[dt * 128 + kk * 32], pf[kk], o[dt]);
       }
-      lm = lane_max(nxt, r + 1, mask_tag);
-      if constexpr (CV) flag = __builtin_amdgcn_ballot_w64(fnext != 0) != 0 ? 1 : 0;
     }
-    if (sync) unit_barrier();
-  };
-
-  Staged<KB> st0, st1;
-  f32x16 sa, sb2;
-  load(ua, st0);
-  load(ua + 1, st1);
-  stage(0, st0, std::true_type{});
-  load(ua + 2, st0);
-  stage(1, st1, std::true_type{});
-  load(ua + 4, st1);
-  stage(2, st0, std::true_type{});
-  load(ua + 3, st0);
-  unit_barrier();
-  if (active) {
-    sa = scores(0);
-    lm = lane_max(sa, 0, std::true_type{});
-    if constexpr (CV) flag = __builtin_amdgcn_ballot_w64(s_flag[0][lane & 7] != 0) != 0 ? 1 : 0;
   }
-  unit_barrier();
-  // every wave takes ub - ua steps (one barrier each); a wave past the last
-  // query token only loads and stages.  The steps whose units (up to r + 3)
-  // are whole and visible to every column go in pairs (fixed registers for
-  // both score tiles and both staged units), the others one by one.
-  auto run = [&](auto act) __attribute__((always_inline)) {
-    const int n = ub - ua, plain = nfull - ua - 4;  // pairs r, r + 1 with r + 4 < nfull - ua
-    int r = 0;
-    auto flip = [&]() __attribute__((always_inline)) {
-      const f32x16 sx = sa;
-      sa = sb2;
-      sb2 = sx;
-      const Staged<KB> tx = st0;
-      st0 = st1;
-      st1 = tx;
-    };
-#pragma unroll 1
-    while (r < n) {
-      if constexpr (CV && decltype(act)::value) {
-        if (flag) {
-          step(r, sa, sb2, st0, act, std::true_type{}, std::true_type{}, (r & 1) != 0);
-          ++r;
-          flip();
-          continue;
-        }
-      }
-      if (r < plain && (r & 1) == 0) {
-#pragma unroll 1
-        do {
-          step(r++, sa, sb2, st0, act, std::false_type{}, std::false_type{}, false);
-          if (CV && flag) {
-            flip();
-            break;
-          }
-          step(r++, sb2, sa, st1, act, std::false_type{}, std::false_type{}, true);
-        } while (r < plain && !(CV && flag));
-        continue;
-      }
-      step(r, sa, sb2, st0, act, std::true_type{}, std::false_type{}, (r & 1) != 0);
-      ++r;
-      flip();
-    }
-  };
-  if (active) run(std::true_type{});
-  else run(std::false_type{});
   if (!active) return;
   // O^T: entry i of a lane is dim 32 dt + 8 (i / 4) + 4 hh + i % 4 of its column
   const float lt = pair_sum(l);
@@ -526,15 +563,20 @@ __global__ __launch_bounds__(256) void k_prefill_combine(int rows, int nsplit, c
       make_uint2(pack2<DT>(a[0] * inv, a[1] * inv), pack2<DT>(a[2] * inv, a[3] * inv));
 }
 
+// tiles of whole workgroups (kPfWaves waves)
+static int64_t prefill_tiles(const Geometry& g, int n, int L) {
+  return (int64_t)((L * g.group + kPfWaves * kPfCols - 1) / (kPfWaves * kPfCols)) * g.hkv * n;
+}
+
 // Parts for n sequences of at most `tokens` tokens: the number with the least
 // rounds of workgroups (one per CU at a time) times the units a round takes,
 // where a split adds the merge.  A chunk whose tiles fill the CUs once or a
 // whole number of times is not split (8 sequences of 512 tokens: 512 tiles);
-// one sequence's 64 tiles are split in 4 (370 us; unsplit they take 4 times
-// the units of a round).
+// one sequence's 64 tiles are split in 4 (1109 us with one workgroup of 128
+// columns a tile, unsplit; 294 us).
 int prefill_splits(const Geometry& g, int n, int L, int tokens) {
   if (g.cus <= 0) return 1;
-  const int64_t tiles = (int64_t)((L * g.group + kPfWaves * kPfCols - 1) / (kPfWaves * kPfCols)) * g.hkv * n;
+  const int64_t tiles = prefill_tiles(g, n, L);
   const int64_t rows = (int64_t)n * g.hq * L;
   const int units = (tokens + 31) / 32;
   int best = 1;
@@ -552,15 +594,15 @@ int prefill_splits(const Geometry& g, int n, int L, int tokens) {
   return best;
 }
 
-template <int DT, int KB>
+template <int DT, int KB, int W>
 static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, int nsplit, const uint16_t* q, float sl2,
                                    uint16_t* out, float* ws, hipStream_t s, Timing* prof) {
   const int lg = __builtin_ctz((unsigned)g.group);
-  const int per_wg = (kPfWaves * kPfCols) >> lg;
+  const int per_wg = (W * kPfCols) >> lg;
   const int gx = (L + per_wg - 1) / per_wg;
   const int rows = b.n * g.hq * L;
   float* pml = ws ? ws + (size_t)nsplit * rows * kHeadDim : nullptr;
-  launch(k_prefill<DT, KB>, dim3((unsigned)gx * g.hkv * b.n * nsplit), dim3(64 * kPfWaves), 0, s, prof, kProfPrefill, g,
+  launch(k_prefill<DT, KB, W>, dim3((unsigned)gx * g.hkv * b.n * nsplit), dim3(64 * W), 0, s, prof, kProfPrefill, g,
          b, L, lg, gx, nsplit, q, sl2, out, ws, pml);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
@@ -568,15 +610,29 @@ static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, 
   return hipGetLastError();
 }
 
+// Workgroups of 4 waves (half a tile) where those of all tiles and parts still
+// fit the CUs at once: a wave then has a SIMD to itself, and a unit takes it
+// little more than half as long.  One fp16 prompt of 200 tokens, Hq 32, Hkv 8:
+// 17.0 us with 8 waves (32 workgroups), 12.7 with 4 (56); of 600 26.1 and
+// 20.5, of 1000 (256 workgroups of 4) 35.3 and 28.9.  With more, the second
+// round costs more than that: 1500 tokens take 47 us with 8 waves.
+template <int DT, int KB>
+static hipError_t prefill_width(const Geometry& g, const SeqBatch& b, int L, int nsplit, const uint16_t* q, float sl2,
+                                uint16_t* out, float* ws, hipStream_t s, Timing* prof) {
+  if (2 * prefill_tiles(g, b.n, L) * nsplit <= g.cus)
+    return prefill_dispatch<DT, KB, kPfWaves / 2>(g, b, L, nsplit, q, sl2, out, ws, s, prof);
+  return prefill_dispatch<DT, KB, kPfWaves>(g, b, L, nsplit, q, sl2, out, ws, s, prof);
+}
+
 hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, int nsplit, const void* q, float scale,
                           void* out, float* ws, hipStream_t s, Timing* prof) {
   const float sl2 = scale * 1.4426950408889634f;
   const uint16_t* qq = (const uint16_t*)q;
   uint16_t* oo = (uint16_t*)out;
-  if (g.kv_bits == 4) return prefill_dispatch<0, 4>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  if (g.kv_bits == 8) return prefill_dispatch<0, 8>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  if (g.dtype == 0) return prefill_dispatch<0, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  return prefill_dispatch<1, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.kv_bits == 4) return prefill_width<0, 4>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.kv_bits == 8) return prefill_width<0, 8>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.dtype == 0) return prefill_width<0, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  return prefill_width<1, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
 }
 
 }  // namespace bsattn

@@ -20,6 +20,11 @@ pytestmark = pytest.mark.gpu
     ("f16", 64, 4, 64, [4500, 4230, 4353, 4416], 256),  # 256 tiles: not split; 71 blocks
     ("bf16", 8, 8, 64, [255], 255),           # one token less than a tile, from an empty cache
     ("f16", 16, 2, 32, [33], 32),             # one token before the chunk
+    ("bf16", 32, 8, 64, [97, 33], 33),        # half tiles of 32 tokens: one token more
+    ("f16", 64, 4, 64, [200], 71),            # half tiles of 8 tokens: one token less
+    # split with a sequence of fewer units than parts, in whole tiles and in half ones
+    ("bf16", 32, 8, 64, [4700, 40, 65], 33),
+    ("f16", 8, 2, 32, [20, 2000], 20),
 ])
 def test_prefill_tile_edges(gpu, dtype, Hq, Hkv, Tb, lens, L):
     log(f"[prefill tiles] {dtype} Hq={Hq} Hkv={Hkv} Tb={Tb} lens={lens} L={L}")
@@ -64,6 +69,31 @@ def test_prefill_unit_counts(gpu, dtype, units, big):
             a = O.to_f32(got[0, h * w.G:(h + 1) * w.G, i], dtype).astype(np.float64)
             err = float(np.max((np.abs(a - ref) - 0.5 * ulp(ref, dtype)) / np.maximum(1.0, mag)))
             assert err <= TOL, f"query {i} head {h}: relative error {err:.3g}"
+
+
+@pytest.mark.parametrize("dtype,bits,Hq,Hkv,Tb", [
+    ("f16", 0, 32, 8, 64), ("bf16", 0, 32, 8, 32), ("f16", 4, 32, 8, 64), ("f16", 8, 64, 4, 32), ("bf16", 0, 8, 8, 64),
+])
+def test_prefill_widths(gpu, dtype, bits, Hq, Hkv, Tb):
+    """Many sequences in a call take workgroups of 8 waves, one alone those of
+    4 (neither is split): the same bits, at every count of units up to 13."""
+    import torch
+    log(f"[prefill widths] {dtype} int{bits} Hq={Hq} Hkv={Hkv} Tb={Tb}")
+    L, B = 40, 40
+    lens = [L + 9 * b for b in range(B)]
+    w = make_workload(8400 + bits + Hq, B=B, Hq=Hq, Hkv=Hkv, T=max(lens), Tb=Tb, dtype=dtype, top_k=4, lens=lens)
+    c = new_cache(w, kv_bits=bits)
+    for b in range(B):
+        v = to_dev(w.values[b][None], dtype, gpu)
+        if dtype == "bf16" and b % 3 == 1:
+            v[:, :, 7::29] *= 2.0 ** 17  # (beyond fp16)
+        c.append(to_dev(w.keys[b][None], dtype, gpu), v, seq_ids=[b])
+    q = to_dev(O.fill_normal(w.seed + 1, 0, 0, (B, Hq, L, 128), dtype), dtype, gpu)
+    together = c.prefill(q, w.scale)
+    for b in range(B):
+        alone = c.prefill(q[b:b + 1].contiguous(), w.scale, seq_ids=[b])
+        assert torch.equal(together[b], alone[0]), f"{lens[b]} tokens"
+    assert torch.isfinite(together.float()).all()
 
 
 def test_split_prefill_in_a_graph(gpu):
