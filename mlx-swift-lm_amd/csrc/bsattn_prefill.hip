@@ -29,11 +29,17 @@ __device__ __forceinline__ f32x16 mfma32x32x16(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
+
 // all bits of the 16-bit elements whose magnitude bits are `lim` or more
 __device__ __forceinline__ u32x4 at_least16(u32x4 w, uint32_t lim) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-    w[k] = ((w[k] & 0x7FFFu) >= lim ? 0x0000FFFFu : 0u) | ((w[k] >> 16 & 0x7FFFu) >= lim ? 0xFFFF0000u : 0u);
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t mag = w[k] & 0x7FFF7FFFu;
+    const i16x2 l = {(int16_t)lim, (int16_t)lim};
+    const i16x2 below = (__builtin_bit_cast(i16x2, mag) - l) >> 15;  // the difference's sign
+    w[k] = ~__builtin_bit_cast(uint32_t, below);
+  }
   return w;
 }
 
@@ -111,7 +117,8 @@ struct Staged<0, F> {
 // the hi / lo split of P.  A value fp16 cannot take is left out there and the
 // unit noted; the noted units are gone through once more after the last one,
 // for those values alone, in bf16 with P as hi + lo from the cache's own
-// fragments.
+// fragments.  So are infinities and NaN of any cache's V in units that some
+// columns do not see: a later token's reach no earlier query.
 // Codes of an affine cache (KB = 4 / 8 bits, fp16 q / out) are dequantized on
 // the way, as fp16 values fl16(scale * code + bias) (one packed fused
 // multiply-add per pair, so each is the correctly rounded value).
@@ -150,16 +157,12 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   using St = Staged<KB, F>;
   __shared__ __align__(16) u32x4 s_k[4][8 * 64], s_v[8][8 * 64];
   __shared__ __align__(16) u32x4 s_ent[KB ? W : 1][KB ? 32 : 1];  // each wave's copy of a unit's scales / biases
-  // CV: units whose V holds an element that is left to the end, bit x - ua
-  // (tables are at most 12288 blocks wide)
-  constexpr int ODDW = CV ? 2 * 12288 / 32 + 1 : 1;
+  // units whose V holds an element that is left to the end, bit x - odd0.  A
+  // bf16 cache: any unit (tables are at most 12288 blocks wide).  Otherwise
+  // those that only some columns see, at most 9: a word per wave, its own
+  constexpr int ODDW = CV ? 2 * 12288 / 32 + 1 : W;
   __shared__ uint32_t s_odd[ODDW];
-  __shared__ int s_anyodd;
-  if constexpr (CV) {
-    for (int i = threadIdx.x; i < ODDW; i += 64 * W) s_odd[i] = 0u;
-    if (threadIdx.x == 0) s_anyodd = 0;
-    unit_barrier();
-  }
+  __shared__ int s_anyodd;  // (CV) whether there are any
   const int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int col = lane & 31, hh = lane >> 5;
   // XCD-grouped workgroup order (a bijection on [0, total))
@@ -197,7 +200,9 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   const int ua = uniform((int)((uint32_t)nunit * part / nsplit)), ub = uniform((int)((uint32_t)nunit * (part + 1) / nsplit));
   // units below nfull are whole and visible to every column of the workgroup
   const int nfull = uniform(min((T - L + twg + 1) / 32, ub));
-  constexpr uint32_t ODD = 0x4780u;  // magnitude bits of 65536 in bf16
+  const int odd0 = CV ? ua : nfull;
+  // magnitude bits of infinity, and of the elements left to the end (bf16: from 65536)
+  constexpr uint32_t INF = DT == 0 ? 0x7C00u : 0x7F80u, ODD = CV ? 0x4780u : INF;
 
   // --- units from memory: this wave's fragments, in the slab's own order
   const int32_t* bt = block_table(geo, seq);
@@ -262,7 +267,7 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   };
   // w without the elements that are left to the end, with the unit noted when
   // there are any
-  [[maybe_unused]] auto drop = [&](int r, u32x4 w) __attribute__((always_inline)) {
+  auto drop = [&](int r, u32x4 w) __attribute__((always_inline)) {
     u16x2 big = {0, 0};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -272,9 +277,14 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
     constexpr uint32_t UP = 0x10001u * (0x8000u - ODD);  // carries ODD and more into the sign bits
     if (__builtin_amdgcn_ballot_w64(((__builtin_bit_cast(uint32_t, big) + UP) & 0x80008000u) != 0u) != 0) {
       w &= ~at_least16(w, ODD);
+      const int at = ua + r - odd0;
       if (lane == 0) {
-        atomicOr(&s_odd[min(r >> 5, ODDW - 1)], 1u << (r & 31));
-        s_anyodd = 1;
+        if constexpr (CV) {
+          atomicOr(&s_odd[min(at >> 5, ODDW - 1)], 1u << (at & 31));
+          s_anyodd = 1;
+        } else {
+          s_odd[wave] |= 1u << (at & 31);
+        }
       }
     }
     return w;
@@ -337,6 +347,8 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
           const int tk = 8 * g + 2 * jj;
           vw[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
         }
+        if constexpr (!CV && !RAW)
+          if (ua + r >= nfull) vw = drop(r, vw);
       }
       s_k[r & 3][f * 64 + lane] = kw;
       s_v[r & 7][f * 64 + lane] = vw;
@@ -432,6 +444,13 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   f32x16 sa, sb2;
   load(ua, st0);
   load(ua + 1, st1);
+  if constexpr (CV) {
+    for (int i = threadIdx.x; i < ODDW; i += 64 * W) s_odd[i] = 0u;
+    if (threadIdx.x == 0) s_anyodd = 0;
+    unit_barrier();
+  } else {
+    if (lane == 0) s_odd[wave] = 0u;
+  }
   stage(0, st0, std::true_type{}, std::false_type{});
   load(ua + 2, st0);
   stage(1, st1, std::true_type{}, std::false_type{});
@@ -464,28 +483,84 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
   };
   if (active) run(std::true_type{});
   else run(std::false_type{});
-  if constexpr (CV) {
-    unit_barrier();
-    if (uniform(s_anyodd) != 0) {
-#pragma unroll 1
-      for (int r = 0; r < ub - ua; ++r) {
-        if ((uniform((int)s_odd[r >> 5]) >> (r & 31) & 1) == 0) continue;
-        const int x = ua + r, blk = x >> ksh;
-        pbase = blk;
-        pagev = bt[min(pbase + lane, lastblk)];
-        load(x, st0);
-        unit_barrier();
-        stage(r, st0, std::true_type{}, std::true_type{});
-        unit_barrier();
-        if (!active) continue;
-        sa = scores(r);
-        lane_max(sa, r, std::true_type{});
+  // The noted units once more, for the elements left out.  Infinities and NaN
+  // are added token by token, to the columns that see the token: a product
+  // would bring 0 * inf to the others (and, with P as hi + lo, inf - inf).
+  unit_barrier();
+  uint32_t odd_word = 0u;  // (bits of units odd0 ..)
+  if constexpr (CV) odd_word = s_anyodd;
+  else
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sa[i] = __builtin_amdgcn_exp2f(fmaf(sa[i], sc, -m));
-        const uint8_t* vs = geo.pool + ((size_t)uniform(bt[blk]) * geo.hkv + h) * geo.slab_bytes + geo.v_off +
-                            (x & ((1 << ksh) - 1)) * 1024;
-        const int tile16 = 1024 << ksh;  // bytes from one 16-dim tile to the next
-        const int valid = T - 32 * x;
+    for (int w = 0; w < W; ++w) odd_word |= s_odd[w];
+  odd_word = (uint32_t)uniform((int)odd_word);
+  if (odd_word != 0u) {
+    auto next = [&](int x) __attribute__((always_inline)) {  // the first noted unit from x on, or ub
+#pragma unroll 1
+      for (; x < ub; ++x) {
+        const int at = x - odd0;
+        if ((CV ? (uint32_t)uniform((int)s_odd[at >> 5]) : odd_word) >> (at & 31) & 1u) break;
+      }
+      return x;
+    };
+    int x = next(odd0);
+    pbase = min(x, ub - 1) >> ksh;
+    pagev = bt[min(pbase + lane, lastblk)];
+    load(x, st0);
+#pragma unroll 1
+    while (x < ub) {
+      const int r = x - ua, at = x;
+      // the unit's V as it is stored: a bf16 cache's own, or the 16-bit tile
+      const uint8_t* vs = (const uint8_t*)s_v[r & 7];
+      int tile16 = 1024;  // bytes from one 16-dim tile to the next
+      [[maybe_unused]] u32x4 vf[CV ? 2 : 1][CV ? 4 : 1];
+      if constexpr (CV) {
+        const int page = __builtin_amdgcn_readlane(pagev, (x >> ksh) - pbase);
+        vs = geo.pool + ((size_t)page * geo.hkv + h) * geo.slab_bytes + geo.v_off + (x & ((1 << ksh) - 1)) * 1024;
+        tile16 = 1024 << ksh;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt)
+            vf[kk][dt] = *(const u32x4*)(vs + (2 * dt + (col >> 4)) * tile16 + ((col & 15) + 16 * (2 * kk + hh)) * 16);
+      }
+      unit_barrier();
+      stage(r, st0, std::true_type{}, std::true_type{});
+      x = next(x + 1);
+      load(x, st0);
+      unit_barrier();
+      if (!active) continue;
+      sa = scores(r);
+      if (at >= nfull) lane_max(sa, r, std::true_type{});
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sa[i] = __builtin_amdgcn_exp2f(fmaf(sa[i], sc, -m));
+      if constexpr (CV) {
+        const int valid = T - 32 * at;
+        u16x2 top = {0, 0};
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+          for (int dt = 0; dt < 4; ++dt) {
+            u32x4& v = vf[kk][dt];
+            v &= at_least16(v, ODD);
+            if (valid < 32)  // (stale page data)
+#pragma unroll
+              for (int jj = 0; jj < 4; ++jj) {
+                const int tk = 8 * (2 * kk + hh) + 2 * jj;
+                v[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
+              }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t mag = v[k] & 0x7FFF7FFFu;
+              top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, mag));
+            }
+          }
+        const bool each =
+            __builtin_amdgcn_ballot_w64(((__builtin_bit_cast(uint32_t, top) + 0x10001u * (0x8000u - INF)) & 0x80008000u) != 0u) != 0;
+        if (each)
+#pragma unroll
+          for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) vf[kk][dt] &= ~at_least16(vf[kk][dt], INF);
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
           u32x4 ph, pl;
@@ -498,17 +573,28 @@ __global__ __launch_bounds__(64 * kPfWaves) void k_prefill(Geometry geo, SeqBatc
           }
 #pragma unroll
           for (int dt = 0; dt < 4; ++dt) {
-            u32x4 vf = *(const u32x4*)(vs + (2 * dt + (col >> 4)) * tile16 + ((col & 15) + 16 * (2 * kk + hh)) * 16);
-            vf &= at_least16(vf, ODD);
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-              const int tk = 8 * (2 * kk + hh) + 2 * jj;
-              vf[jj] &= (tk < valid ? 0x0000FFFFu : 0u) | (tk + 1 < valid ? 0xFFFF0000u : 0u);
-            }
-            o[dt] = mfma32x32x16<1>(vf, ph, o[dt]);
-            o[dt] = mfma32x32x16<1>(vf, pl, o[dt]);
+            o[dt] = mfma32x32x16<1>(vf[kk][dt], ph, o[dt]);
+            o[dt] = mfma32x32x16<1>(vf[kk][dt], pl, o[dt]);
           }
         }
+        if (!each) continue;
+      }
+      const int lim = pos - 32 * at;
+#pragma unroll 1
+      for (int t = 0; t < 32; ++t) {
+        const int own = 8 * (t >> 4) + (t & 7);  // entry of token t in the lanes of half t / 8 % 2
+        float p = sa[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) p = i == own ? sa[i] : p;
+        p = __shfl(p, col + 32 * ((t >> 3) & 1), 64);
+        const uint8_t* vt = vs + 256 * (t >> 3) + 2 * (t & 7) + 64 * hh;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const uint32_t w = *(const uint16_t*)(vt + (2 * dt + (i >> 3)) * tile16 + 128 * ((i >> 2) & 1) + 16 * (i & 3));
+            if (t <= lim && (w & 0x7FFFu) >= INF) o[dt][i] = fmaf(p, to_f32<DT>((uint16_t)w), o[dt][i]);
+          }
       }
     }
   }

@@ -120,3 +120,53 @@ def test_split_prefill_in_a_graph(gpu):
         assert torch.equal(a.prefill(q, w.scale), want)
         torch.cuda.synchronize()
     assert np.isfinite(want.float().cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("dtype,bits,Hq,Hkv,Tb,T,L", [
+    ("f16", 0, 32, 8, 64, 200, 150),    # half tiles
+    ("bf16", 0, 32, 8, 32, 130, 130),
+    ("f16", 8, 64, 4, 32, 300, 200),
+    ("f16", 4, 32, 8, 64, 900, 300),
+    ("bf16", 0, 32, 8, 64, 4500, 200),  # split
+    ("f16", 0, 8, 8, 64, 2100, 2000),   # whole tiles of 256 tokens
+    ("bf16", 0, 8, 8, 64, 2100, 2000),
+])
+def test_prefill_values_that_are_not_finite(gpu, dtype, bits, Hq, Hkv, Tb, T, L):
+    """An infinity or NaN in a token's V reaches the queries that see the token,
+    in its dim and head, and no other output: those are the bits of a cache
+    with a finite value there."""
+    import torch
+    log(f"[prefill not finite] {dtype} int{bits} Hq={Hq} Hkv={Hkv} Tb={Tb} T={T} L={L}")
+    w = make_workload(8500 + T + Hq, B=1, Hq=Hq, Hkv=Hkv, T=T, Tb=Tb, dtype=dtype, top_k=4)
+    G = Hq // Hkv
+    k, v = to_dev(w.keys[0][None], dtype, gpu), to_dev(w.values[0][None], dtype, gpu)
+    q = to_dev(O.fill_normal(w.seed + 1, 0, 0, (1, Hq, L, 128), dtype), dtype, gpu)
+    inf, nan = float("inf"), float("nan")
+    odd = [(T - L + 3, 0, 5, inf), (T - L // 2, 0, 70, nan), (T - 9, Hkv - 1, 127, -inf), (T - 1, 1, 64, inf)]
+    caches = []
+    for bad in (False, True):
+        c = new_cache(w, kv_bits=bits)
+        if bits:  # the whole 64-dim group of the token: V = scale * code + bias
+            src = new_cache(w, kv_bits=bits)
+            src.append(k, v)
+            kq, vq = src.exportQuantized([0])
+            if bad:
+                for pos, h, d, x in odd:
+                    vq[2][0, h, pos, d // 64] = x
+            c.appendQuantized(kq, vq)
+        else:
+            vb = v.clone()
+            if bad:
+                for pos, h, d, x in odd:
+                    vb[0, h, pos, d] = x
+            c.append(k, vb)
+        caches.append(c)
+    good, got = (c.prefill(q, w.scale)[0].float() for c in caches)
+    hit = torch.zeros_like(good, dtype=torch.bool)
+    for pos, h, d, x in odd:
+        dims = slice(d // 64 * 64, d // 64 * 64 + 64) if bits else slice(d, d + 1)
+        seen = got[h * G:(h + 1) * G, max(0, pos - (T - L)):, dims]
+        assert bool(torch.isnan(seen).all() if x != x else (seen == x).all()), f"token {pos}: its queries"
+        hit[h * G:(h + 1) * G, max(0, pos - (T - L)):, dims] = True
+    assert torch.isfinite(good).all()
+    assert torch.equal(got[~hit], good[~hit]), f"{int((got[~hit] != good[~hit]).sum())} outputs differ"
