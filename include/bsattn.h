@@ -72,7 +72,8 @@ typedef struct bsattn_info {
   int32_t nsel_max;        /* sink + recent + top_k: width of index outputs */
   int32_t num_splits;      /* attention partials per (sequence, q head): the most a call uses */
   int64_t page_bytes;      /* bytes of one page across all kv heads, incl. summaries */
-  int64_t pool_bytes;      /* device bytes held by the handle */
+  int64_t pool_bytes;      /* device bytes of the handle's pages, summaries and metadata
+                              (workspaces not counted) */
   int64_t free_pages;      /* pages not owned by any sequence */
 } bsattn_info;
 
@@ -204,7 +205,14 @@ int bsattn_decode_multi(bsattn_cache* cache, const void* q,
  * the causal mask (AttentionUtils.swift:46-52, BaseKVCache.makeMask,
  * KVCache.swift:160-174) computes over the whole cache (for a quantized
  * cache: quantizedScaledDotProductAttention with the causal mask,
- * KVCache.swift:1533-1621). */
+ * KVCache.swift:1533-1621).
+ * A short batch's tokens are split over the GPU and merged through a
+ * workspace of 68 MB.  The first such call allocates it; the GPU's caches
+ * share it (up to four of them when several streams prefill at once, beyond
+ * which a call waits on its stream for another's) and the last one destroyed
+ * frees it.  Under capture the cache allocates one of the call's size for
+ * itself and keeps it.  When none can be had the call runs unsplit: slower,
+ * and rounded differently. */
 int bsattn_prefill(bsattn_cache* cache, const void* q, const int32_t* seq_ids,
                    int32_t n_seqs, int32_t n_query, float scale, void* out,
                    void* stream);

@@ -12,6 +12,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <stdexcept>
 #include <string>
@@ -83,7 +84,9 @@ struct bsattn_cache {
   float* partials = nullptr;  // [rows][hq][nsplit][D + 2]
   uint32_t* arrive = nullptr; // [kArriveWords] arrival counters of split merges, 0 between launches
   float* err_ws = nullptr;    // [rows][hkv][2][mfma_err_stride]: MFMA score bounds, chunk floors
-  float* prefill_ws = nullptr;  // split prefill partials (allocated by the first call that splits)
+  // split prefill partials of captured calls (a graph holds their addresses):
+  // workspace and its rows, kept until the cache is destroyed
+  std::vector<std::pair<float*, int64_t>> graph_ws;
   std::vector<int32_t> len;
   // set by bsattn_append_step: the device-side lengths may be ahead of `len`
   // until bsattn_sync
@@ -114,6 +117,141 @@ struct DeviceGuard {
     if (prev >= 0) (void)hipSetDevice(prev);
   }
 };
+
+// Lets this thread allocate, free and query events while any thread captures
+// a graph, without invalidating the capture.
+class RelaxedCapture {
+ public:
+  RelaxedCapture() { ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+  ~RelaxedCapture() {
+    if (ok_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  RelaxedCapture(const RelaxedCapture&) = delete;
+  RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+  bool ok() const { return ok_; }
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool ok_ = false;
+};
+
+constexpr size_t kPrefillRowBytes = (kHeadDim + 2) * sizeof(float);
+
+// ---------------------------------------------------------------------------
+// Workspaces of the split prefills of one GPU (68 MB each), shared by its
+// caches: a model has one cache per layer, and its layers' prefills follow
+// each other on a stream.  A call takes the one that its stream used last, or
+// one whose last user has finished; failing that another is allocated, up to
+// kMost, and beyond that the call waits, on its stream, for another stream's.
+// In each case the stream waits for the event of the last use (nothing to
+// wait for on the same stream), so a handle that names another stream by now
+// is no matter.  The lock is held from the choice until the event is
+// recorded.  All are freed with the GPU's last cache.
+// The event belongs to the merge's dispatch and has no system fence (only
+// streams of the GPU wait for it): a call takes no longer with it than without
+// (64 bf16 tokens behind 960, 19.9 and 19.7 us; recorded by itself, or with
+// the fence, 20.9-22.6).
+// ---------------------------------------------------------------------------
+class PrefillSpaces {
+ public:
+  static PrefillSpaces* of(int device) {
+    static PrefillSpaces all[kMaxDevices];
+    return device >= 0 && device < kMaxDevices ? &all[device] : nullptr;
+  }
+  void add_cache() {
+    std::lock_guard<std::mutex> lock(mu_);
+    ++caches_;
+  }
+  void drop_cache() {  // (the device is current and idle)
+    std::lock_guard<std::mutex> lock(mu_);
+    if (--caches_ > 0) return;
+    RelaxedCapture relaxed;
+    for (int i = 0; i < count_; ++i) {
+      (void)hipFree(spaces_[i].p);
+      (void)hipEventDestroy(spaces_[i].done);
+    }
+    count_ = 0;
+  }
+  // launch(workspace, event that its last kernel must record), or launch(null,
+  // null) when there is no workspace to be had
+  template <typename F>
+  hipError_t with(hipStream_t s, F launch) {
+    std::unique_lock<std::mutex> lock(mu_);
+    Space* sp = pick(s);
+    if (sp && hipStreamWaitEvent(s, sp->done, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      sp = nullptr;
+    }
+    if (!sp) {
+      lock.unlock();
+      return launch(nullptr, nullptr);
+    }
+    sp->stream = s;
+    const hipError_t e = launch(sp->p, sp->done);
+    // (part of the work may be under way without the event)
+    if (e != hipSuccess && hipEventRecord(sp->done, s) != hipSuccess) (void)hipDeviceSynchronize();
+    return e;
+  }
+
+ private:
+  static constexpr int kMaxDevices = 64, kMost = 4;
+  struct Space {
+    float* p;
+    hipEvent_t done;  // recorded by the last use
+    hipStream_t stream;
+  };
+  Space* pick(hipStream_t s) {
+    RelaxedCapture relaxed;
+    if (!relaxed.ok()) return nullptr;
+    for (int i = 0; i < count_; ++i)
+      if (spaces_[i].stream == s) return &spaces_[i];
+    for (int i = 0; i < count_; ++i) {
+      if (hipEventQuery(spaces_[i].done) == hipSuccess) return &spaces_[i];
+      (void)hipGetLastError();  // (not ready is no error of this call)
+    }
+    if (count_ < kMost) {
+      Space n{nullptr, nullptr, s};
+      if (hipMalloc((void**)&n.p, (size_t)kPrefillRows * kPrefillRowBytes) == hipSuccess) {
+        if (hipEventCreateWithFlags(&n.done, hipEventDisableTiming | hipEventDisableSystemFence) == hipSuccess) {
+          spaces_[count_] = n;
+          return &spaces_[count_++];
+        }
+        (void)hipFree(n.p);
+      }
+      (void)hipGetLastError();
+    }
+    return count_ > 0 ? &spaces_[next_++ % count_] : nullptr;
+  }
+  std::mutex mu_;
+  int caches_ = 0, count_ = 0;
+  unsigned next_ = 0;
+  Space spaces_[kMost] = {};
+};
+
+// whether work on s is recorded into a graph (also when that cannot be told)
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// the cache's own workspace of at least `rows` rows for a captured call, or
+// null
+float* graph_workspace(bsattn_cache* c, int64_t rows) {
+  for (const auto& w : c->graph_ws)
+    if (w.second >= rows) return w.first;
+  RelaxedCapture relaxed;
+  if (!relaxed.ok()) return nullptr;
+  c->graph_ws.reserve(c->graph_ws.size() + 1);
+  float* p = nullptr;
+  if (hipMalloc((void**)&p, (size_t)rows * kPrefillRowBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  c->graph_ws.emplace_back(p, rows);
+  return p;
+}
 
 int validate_desc(const bsattn_desc& d) {
   if (d.max_seqs < 1) return fail(BSATTN_ERR_INVALID, "max_seqs must be >= 1 (got %d)", d.max_seqs);
@@ -442,6 +580,7 @@ int bsattn_cache_create(const bsattn_desc* desc, bsattn_cache** out) try {
   if ((e = hipMemset(c->arrive, 0, kArriveWords * 4)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(counters)"));
   if ((e = hipMemset(g.meta, 0, c->meta_words * 4)) != hipSuccess) return cleanup(hip_fail(e, "hipMemset(meta)"));
   if ((e = hipDeviceSynchronize()) != hipSuccess) return cleanup(hip_fail(e, "hipDeviceSynchronize"));
+  if (PrefillSpaces* ps = PrefillSpaces::of(d.device)) ps->add_cache();
   *out = c;
   return BSATTN_OK;
 } catch (...) {
@@ -461,7 +600,8 @@ int bsattn_cache_destroy(bsattn_cache* c) try {
   (void)hipFree(c->partials);
   (void)hipFree(c->err_ws);
   (void)hipFree(c->arrive);
-  (void)hipFree(c->prefill_ws);
+  for (const auto& w : c->graph_ws) (void)hipFree(w.first);
+  if (PrefillSpaces* ps = PrefillSpaces::of(c->d.device)) ps->drop_cache();
   delete c;
   return BSATTN_OK;
 } catch (...) {
@@ -1014,24 +1154,6 @@ int bsattn_decode_multi(bsattn_cache* c, const void* q, const int32_t* seq_ids, 
   return on_exception();
 }
 
-// The split prefill's workspace, or null when it cannot be had (the call then
-// runs unsplit).  Allocated once per cache and kept until it is destroyed (a
-// captured graph may hold its address); the relaxed capture mode keeps the
-// allocation from invalidating a capture that is under way on any thread.
-static float* prefill_workspace(bsattn_cache* c) {
-  if (c->prefill_ws) return c->prefill_ws;
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
-  float* p = nullptr;
-  const hipError_t e = hipMalloc((void**)&p, (size_t)kPrefillRows * (kHeadDim + 2) * sizeof(float));
-  (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  return c->prefill_ws = p;
-}
-
 int bsattn_prefill(bsattn_cache* c, const void* q, const int32_t* seq_ids, int32_t n_seqs,
                    int32_t n_query, float scale, void* out, void* stream) try {
   if (!c || !q || !out) return fail(BSATTN_ERR_INVALID, "null argument");
@@ -1064,13 +1186,18 @@ int bsattn_prefill(bsattn_cache* c, const void* q, const int32_t* seq_ids, int32
       b.qoff[i] = (int32_t)(i * per_seq);
       tokens = std::max(tokens, c->len[seqs[i0 + i]]);
     }
-    int nsplit = prefill_splits(c->geo, b.n, n_query, tokens);
-    float* ws = nsplit > 1 ? prefill_workspace(c) : nullptr;
-    if (!ws) nsplit = 1;
+    const int nsplit = prefill_splits(c->geo, b.n, n_query, tokens);
     Timing tm[kProfKinds];
     Timing* prof = prof_slots(c, s, tm);
-    hipError_t e = launch_prefill(c->geo, b, n_query, nsplit, (const uint16_t*)q + i0 * per_seq, scale,
-                                  (uint16_t*)out + i0 * per_seq, ws, s, prof);
+    auto run = [&](float* ws, hipEvent_t done) {  // (without a workspace: unsplit)
+      return launch_prefill(c->geo, b, n_query, ws ? nsplit : 1, (const uint16_t*)q + i0 * per_seq, scale,
+                            (uint16_t*)out + i0 * per_seq, ws, done, s, prof);
+    };
+    PrefillSpaces* spaces = PrefillSpaces::of(c->d.device);
+    hipError_t e;
+    if (nsplit == 1) e = run(nullptr, nullptr);
+    else if (capturing(s)) e = run(graph_workspace(c, (int64_t)nsplit * b.n * c->geo.hq * n_query), nullptr);
+    else e = spaces ? spaces->with(s, run) : run(nullptr, nullptr);
     prof_collect(c, prof);
     if (e != hipSuccess) return hip_fail(e, "prefill launch");
   }

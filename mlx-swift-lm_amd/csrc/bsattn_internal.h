@@ -30,7 +30,7 @@ constexpr int kArrivePairs = kMaxBatch * 16;
 constexpr int kArriveWords = kArriveSplits * kArrivePairs;
 // device scratch of the no-allocation decode (bsattn_noalloc.hip), per GPU
 constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
-// rows of prefill partials (query rows times parts) a cache's workspace holds
+// rows of prefill partials (query rows times parts) a workspace holds
 constexpr int64_t kPrefillRows = 131072;
 // floats after the last block-score row: the workgroup selection reads a
 // thread's candidates as whole vectors, up to 12 x 1024 entries from a row
@@ -234,9 +234,9 @@ hipError_t launch_fused_append_decode(const Geometry& g, const SeqBatch& b, cons
 // dense causal attention of the last L tokens of each sequence.  nsplit > 1:
 // every query's tokens are split into that many parts, whose partials (ws:
 // nsplit * n * hq * L rows of kHeadDim + 2 floats, at most kPrefillRows rows)
-// a second launch merges.
+// a second launch merges; it records `done` (may be null).
 hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, int nsplit, const void* q, float scale,
-                          void* out, float* ws, hipStream_t s, Timing* prof);
+                          void* out, float* ws, hipEvent_t done, hipStream_t s, Timing* prof);
 // parts for a launch of n sequences of up to `tokens` tokens
 int prefill_splits(const Geometry& g, int n, int L, int tokens);
 hipError_t launch_export(const Geometry& g, const SeqBatch& b, int T, void* k_out,

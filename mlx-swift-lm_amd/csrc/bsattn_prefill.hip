@@ -4,6 +4,7 @@
 // Built with -fno-honor-nans -mno-amdgpu-ieee: the scores are MFMA results
 // (never signalling NaNs), so max trees compile to v_max3_f32 without the
 // operand quieting IEEE mode asks for.
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -682,7 +683,7 @@ int prefill_splits(const Geometry& g, int n, int L, int tokens) {
 
 template <int DT, int KB, int W>
 static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, int nsplit, const uint16_t* q, float sl2,
-                                   uint16_t* out, float* ws, hipStream_t s, Timing* prof) {
+                                   uint16_t* out, float* ws, hipEvent_t done, hipStream_t s, Timing* prof) {
   const int lg = __builtin_ctz((unsigned)g.group);
   const int per_wg = (W * kPfCols) >> lg;
   const int gx = (L + per_wg - 1) / per_wg;
@@ -692,7 +693,12 @@ static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, 
          b, L, lg, gx, nsplit, q, sl2, out, ws, pml);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
-  hipLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0, s, rows, nsplit, ws, pml, out);
+  // (the event is the dispatch's own: no packet of its own behind it)
+  if (done)
+    hipExtLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0u, s, nullptr, done, 0u, rows, nsplit,
+                          (const float*)ws, (const float*)pml, out);
+  else
+    hipLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0, s, rows, nsplit, ws, pml, out);
   return hipGetLastError();
 }
 
@@ -704,21 +710,21 @@ static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, 
 // round costs more than that: 1500 tokens take 47 us with 8 waves.
 template <int DT, int KB>
 static hipError_t prefill_width(const Geometry& g, const SeqBatch& b, int L, int nsplit, const uint16_t* q, float sl2,
-                                uint16_t* out, float* ws, hipStream_t s, Timing* prof) {
+                                uint16_t* out, float* ws, hipEvent_t done, hipStream_t s, Timing* prof) {
   if (2 * prefill_tiles(g, b.n, L) * nsplit <= g.cus)
-    return prefill_dispatch<DT, KB, kPfWaves / 2>(g, b, L, nsplit, q, sl2, out, ws, s, prof);
-  return prefill_dispatch<DT, KB, kPfWaves>(g, b, L, nsplit, q, sl2, out, ws, s, prof);
+    return prefill_dispatch<DT, KB, kPfWaves / 2>(g, b, L, nsplit, q, sl2, out, ws, done, s, prof);
+  return prefill_dispatch<DT, KB, kPfWaves>(g, b, L, nsplit, q, sl2, out, ws, done, s, prof);
 }
 
 hipError_t launch_prefill(const Geometry& g, const SeqBatch& b, int L, int nsplit, const void* q, float scale,
-                          void* out, float* ws, hipStream_t s, Timing* prof) {
+                          void* out, float* ws, hipEvent_t done, hipStream_t s, Timing* prof) {
   const float sl2 = scale * 1.4426950408889634f;
   const uint16_t* qq = (const uint16_t*)q;
   uint16_t* oo = (uint16_t*)out;
-  if (g.kv_bits == 4) return prefill_width<0, 4>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  if (g.kv_bits == 8) return prefill_width<0, 8>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  if (g.dtype == 0) return prefill_width<0, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
-  return prefill_width<1, 0>(g, b, L, nsplit, qq, sl2, oo, ws, s, prof);
+  if (g.kv_bits == 4) return prefill_width<0, 4>(g, b, L, nsplit, qq, sl2, oo, ws, done, s, prof);
+  if (g.kv_bits == 8) return prefill_width<0, 8>(g, b, L, nsplit, qq, sl2, oo, ws, done, s, prof);
+  if (g.dtype == 0) return prefill_width<0, 0>(g, b, L, nsplit, qq, sl2, oo, ws, done, s, prof);
+  return prefill_width<1, 0>(g, b, L, nsplit, qq, sl2, oo, ws, done, s, prof);
 }
 
 }  // namespace bsattn

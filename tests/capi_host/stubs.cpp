@@ -6,8 +6,15 @@
 using namespace bsattn;
 
 extern "C" {
-hipError_t hipMalloc(void** p, size_t n) { return (*p = std::calloc(1, n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipMalloc(void** p, size_t n) {
+  if (n > stub::memory_limit || !(*p = std::calloc(1, n))) return hipErrorOutOfMemory;
+  std::lock_guard<std::mutex> lock(stub::mu);
+  stub::memory[*p] = n;
+  return hipSuccess;
+}
 hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lock(stub::mu);
+  CHECK(!p || stub::memory.erase(p) == 1);
   std::free(p);
   return hipSuccess;
 }
@@ -33,12 +40,24 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
   *v = 256;
   return hipSuccess;
 }
-hipError_t hipEventCreate(hipEvent_t* e) {
-  *e = (hipEvent_t)std::malloc(1);
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = (hipEvent_t)new stub::Event;
   return hipSuccess;
 }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) {
-  std::free(e);
+  delete (stub::Event*)e;
+  return hipSuccess;
+}
+hipError_t hipEventQuery(hipEvent_t e) { return ((stub::Event*)e)->done ? hipSuccess : hipErrorNotReady; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  ((stub::Event*)e)->done = false;
+  ++((stub::Event*)e)->records;
+  return hipSuccess;
+}
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  std::lock_guard<std::mutex> lock(stub::mu);
+  if (!((stub::Event*)e)->done) stub::waits.emplace_back(s, (stub::Event*)e);
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
@@ -47,7 +66,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
   return hipSuccess;
 }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) {
-  *st = hipStreamCaptureStatusNone;
+  *st = stub::capture;
   return hipSuccess;
 }
 hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode*) { return hipSuccess; }
@@ -109,10 +128,16 @@ hipError_t launch_fused_attend(const Geometry& g, const SeqBatch&, int, const vo
                                float*, uint32_t*, hipStream_t, Timing*) {
   return run(g, nullptr);
 }
-int prefill_splits(const Geometry&, int, int, int) { return 1; }
-hipError_t launch_prefill(const Geometry& g, const SeqBatch&, int, int, const void*, float, void*, float*, hipStream_t,
-                          Timing*) {
-  return run(g, nullptr);
+int prefill_splits(const Geometry&, int, int, int) { return stub::splits; }
+hipError_t launch_prefill(const Geometry& g, const SeqBatch&, int, int nsplit, const void*, float, void*, float* ws,
+                          hipEvent_t done, hipStream_t s, Timing*) {
+  {
+    std::lock_guard<std::mutex> lock(stub::mu);
+    stub::prefills.push_back({ws, (stub::Event*)done, nsplit});
+  }
+  const hipError_t e = run(g, nullptr);
+  if (e == hipSuccess && done) (void)hipEventRecord(done, s);
+  return e;
 }
 hipError_t launch_export(const Geometry& g, const SeqBatch&, int, void*, void*, hipStream_t) { return run(g, nullptr); }
 hipError_t launch_export_quantized(const Geometry& g, const SeqBatch&, int, uint32_t*, void*, void*, uint32_t*, void*,

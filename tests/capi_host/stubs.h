@@ -11,6 +11,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <vector>
 
 #include "../../include/bsattn.h"
@@ -20,6 +22,24 @@ namespace stub {
 inline int launches_left = -1;  // launches that succeed before the next one fails (-1: all)
 inline bool applies = false;    // whether the failing launch still writes the metadata
 inline bsattn::Geometry last{};     // geometry of the last launch
+
+// events: `done` says whether the work before the last record has finished
+struct Event {
+  bool done = true;
+  int records = 0;
+};
+inline std::vector<std::pair<hipStream_t, Event*>> waits;  // hipStreamWaitEvent on unfinished work
+inline hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+inline std::map<void*, size_t> memory;                     // device allocations
+inline size_t memory_limit = SIZE_MAX;                     // largest allocation that succeeds
+struct Prefill {
+  float* ws;
+  Event* done;
+  int nsplit;
+};
+inline std::vector<Prefill> prefills;
+inline int splits = 1;  // what prefill_splits answers
+inline std::mutex mu;
 
 // one launch: its patches, and whether it fails
 inline hipError_t run(const bsattn::Geometry& g, const bsattn::PatchBatch* pb) {

@@ -24,7 +24,7 @@ def objects(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("program", ["failed_launch"])
+@pytest.mark.parametrize("program", ["failed_launch", "prefill_workspace"])
 def test_capi_host(objects, tmp_path, program):
     exe = str(tmp_path / program)
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include",
