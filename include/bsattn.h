@@ -281,7 +281,7 @@ int bsattn_export_summaries(const bsattn_cache* cache, int32_t seq, void* out,
 #define BSATTN_KERNEL_SCORE 0   /* block scoring */
 #define BSATTN_KERNEL_TOPK 1    /* top-K selection (bsattn_select) */
 #define BSATTN_KERNEL_ATTEND 2  /* gather + attention (selection fused in bsattn_decode) */
-#define BSATTN_KERNEL_COMBINE 3 /* split combine */
+#define BSATTN_KERNEL_COMBINE 3 /* split combine (decode or prefill) */
 #define BSATTN_KERNEL_APPEND 4  /* token append */
 #define BSATTN_KERNEL_SUMMARY 5 /* block summary refresh */
 #define BSATTN_KERNEL_PREFILL 6 /* dense causal prefill attention */

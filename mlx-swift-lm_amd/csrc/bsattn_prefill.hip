@@ -693,13 +693,15 @@ static hipError_t prefill_dispatch(const Geometry& g, const SeqBatch& b, int L, 
          b, L, lg, gx, nsplit, q, sl2, out, ws, pml);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit == 1) return e;
-  // (the event is the dispatch's own: no packet of its own behind it)
-  if (done)
-    hipExtLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0u, s, nullptr, done, 0u, rows, nsplit,
-                          (const float*)ws, (const float*)pml, out);
+  const dim3 grid((rows + 7) / 8), blk(256);
+  const float *po = ws, *ml = pml;
+  if (done && !prof)  // (the event is the dispatch's own: no packet of its own behind it)
+    hipExtLaunchKernelGGL(k_prefill_combine<DT>, grid, blk, 0u, s, nullptr, done, 0u, rows, nsplit, po, ml, out);
   else
-    hipLaunchKernelGGL(k_prefill_combine<DT>, dim3((rows + 7) / 8), dim3(256), 0, s, rows, nsplit, ws, pml, out);
-  return hipGetLastError();
+    launch(k_prefill_combine<DT>, grid, blk, 0, s, prof, kProfCombine, rows, nsplit, po, ml, out);
+  e = hipGetLastError();
+  if (e == hipSuccess && done && prof) e = hipEventRecord(done, s);
+  return e;
 }
 
 // Workgroups of 4 waves (half a tile) where those of all tiles and parts still

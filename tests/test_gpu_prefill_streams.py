@@ -91,3 +91,20 @@ def test_layers_share_a_workspace(gpu):
     held = free - torch.cuda.mem_get_info()[0]
     assert held <= 100 << 20, f"{held >> 20} MiB for 8 caches"
     assert all(np.isfinite(o.float().cpu().numpy()).all() for o in outs)
+
+
+def test_the_merge_is_timed(gpu):
+    """A profiled split prefill: its merge is a combine launch of its own."""
+    import torch
+    from bsattn import _lib
+    log("[prefill streams] profile")
+    (c, q, scale), = _caches(gpu, 1, 1500)
+    want = c.prefill(q, scale)
+    c.profile(True)
+    for _ in range(3):
+        assert torch.equal(c.prefill(q, scale), want)
+    for kind in (_lib.KERNEL_PREFILL, _lib.KERNEL_COMBINE):
+        ms, n = c.profileRead(kind)
+        assert n == 3 and ms > 0.0
+    c.profile(False)
+    assert torch.equal(c.prefill(q, scale), want)
