@@ -228,14 +228,6 @@ class PrefillSpaces {
   Space spaces_[kMost] = {};
 };
 
-// whether work on s is recorded into a graph (also when that cannot be told)
-bool capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
-}
-
 // the cache's own workspace of at least `rows` rows for a captured call, or
 // null
 float* graph_workspace(bsattn_cache* c, int64_t rows) {
@@ -323,11 +315,22 @@ int send_patches(const bsattn_cache* c, const Patches& p, hipStream_t s) {
   return BSATTN_OK;
 }
 
+// whether work on s is recorded into a graph (also when that cannot be told)
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // What an earlier call could not send; every call that changes the metadata,
 // or launches work that reads it, starts here.  (The exports read block-table
-// entries of tokens already held, which have been sent.)
+// entries of tokens already held, which have been sent.)  Not into a graph,
+// whose every replay would set the words back.
 int send_unsent(bsattn_cache* c, hipStream_t s) {
   if (c->unsent.empty()) return BSATTN_OK;
+  if (capturing(s))
+    return fail(BSATTN_ERR_INVALID, "an earlier launch of this cache failed: make one call outside the capture first");
   if (int rc = send_patches(c, c->unsent, s)) return rc;
   c->unsent.clear();
   return BSATTN_OK;

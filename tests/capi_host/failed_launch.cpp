@@ -55,6 +55,24 @@ int main() {
     append_fails(100, 30, 40, 3, applies, false);  // the second batch's append
     append_fails(70, 31, 1, 2, applies, true);     // a step of two calls
   }
+  // not into a graph: its replays would set the words back
+  {
+    bsattn_cache* g = filled(2, 16, 31);
+    stub::launches_left = 0;
+    stub::applies = false;
+    CHECK(bsattn_append(g, kv, kv, nullptr, 2, 5, nullptr) == BSATTN_ERR_HIP);
+    stub::launches_left = -1;
+    stub::capture = hipStreamCaptureStatusActive;
+    CHECK(decode(g, 2) == BSATTN_ERR_INVALID && append_decode(g, 2) == BSATTN_ERR_INVALID);
+    CHECK(stub::last.meta[stub::last.cap_off] == 32);  // (nothing was sent)
+    stub::capture = hipStreamCaptureStatusNone;
+    CHECK(decode(g, 2) == BSATTN_OK);
+    check_meta(g, 0, 31);
+    stub::capture = hipStreamCaptureStatusActive;
+    CHECK(decode(g, 2) == BSATTN_OK);
+    stub::capture = hipStreamCaptureStatusNone;
+    bsattn_cache_destroy(g);
+  }
   // patches that a reserve, a trim and a reset could not send
   bsattn_cache* c = filled(2, 16, 40);
   stub::launches_left = 0;
