@@ -889,8 +889,7 @@ def bench_loop(args, light: bool = False):
     torch.cuda.synchronize()
     kern = {}
     total = 0.0
-    names = {"append": bsattn._lib.KERNEL_APPEND, "summary": bsattn._lib.KERNEL_SUMMARY,
-             "append+score": bsattn._lib.KERNEL_SCORE, "topk": bsattn._lib.KERNEL_TOPK,
+    names = {"append": bsattn._lib.KERNEL_APPEND, "append+score": bsattn._lib.KERNEL_SCORE, "topk": bsattn._lib.KERNEL_TOPK,
              "attend": bsattn._lib.KERNEL_ATTEND, "combine": bsattn._lib.KERNEL_COMBINE}
     for name, kind in names.items():
         ms, n = cache.profileRead(kind)

@@ -278,12 +278,12 @@ int bsattn_export_summaries(const bsattn_cache* cache, int32_t seq, void* out,
  * (A small batch's decode merges its splits inside the attention launch; a
  * timed one launches the combine by itself, so that its time is seen.  The
  * results are the same bits.) */
-#define BSATTN_KERNEL_SCORE 0   /* block scoring */
+#define BSATTN_KERNEL_SCORE 0   /* block scoring (with the step's append in bsattn_append_decode) */
 #define BSATTN_KERNEL_TOPK 1    /* top-K selection (bsattn_select) */
 #define BSATTN_KERNEL_ATTEND 2  /* gather + attention (selection fused in bsattn_decode) */
 #define BSATTN_KERNEL_COMBINE 3 /* split combine (decode or prefill) */
 #define BSATTN_KERNEL_APPEND 4  /* token append */
-#define BSATTN_KERNEL_SUMMARY 5 /* block summary refresh */
+#define BSATTN_KERNEL_SUMMARY 5 /* retired, always 0: summaries are written by the launch that stores the keys */
 #define BSATTN_KERNEL_PREFILL 6 /* dense causal prefill attention */
 int bsattn_profile_enable(bsattn_cache* cache, int32_t enable);
 int bsattn_profile_read(bsattn_cache* cache, int32_t kernel, double* total_ms,

@@ -175,11 +175,11 @@ def run_case(gpu, case, wseed, dtype, Tb, Hq, Hkv, K, ns, nr, bits, lens0, steps
     if one_launch:
         # one fused decode launch per step (followed by the split combine
         # when a (sequence, kv head) has several splits), and no append,
-        # scoring, summary or selection launch
+        # scoring or selection launch
         n_att = a.profileRead(_lib.KERNEL_ATTEND)[1]
         n_comb = a.profileRead(_lib.KERNEL_COMBINE)[1]
         others = {k: a.profileRead(getattr(_lib, k))[1] for k in
-                  ("KERNEL_APPEND", "KERNEL_SCORE", "KERNEL_SUMMARY", "KERNEL_TOPK")}
+                  ("KERNEL_APPEND", "KERNEL_SCORE", "KERNEL_TOPK")}
         a.profile(False)
         assert n_att == steps and n_comb in (0, steps) and not any(others.values()), \
             f"not one decode launch per step: attend {n_att}, combine {n_comb}, others {others}"
