@@ -674,10 +674,12 @@ bool fused_decode_ok(const Geometry& g, int nseq, int max_nc) {
   if (g.kv_bits != 0 || g.group > 4 || max_nc > kFusedMaxCand || g.top_k > kSelMaxK) return false;
   const FusedPlan p = fused_plan(g, nseq);
   // every split of a pair scores all of the pair's candidates: worth it with
-  // one split (no redundancy, and no combine), or with few candidates.  (A CU
-  // pulls ~20 GB/s while every CU loads: the 128 KiB of summaries of a
-  // 510-candidate pair take it ~6 us, against ~5 us for a scoring kernel that
-  // spreads them over every CU.)
+  // one split (no redundancy), or with few candidates.  The line is an
+  // estimate, of when the splits still had a combine launch and a selection
+  // of seven barriers behind them: a CU pulls ~20 GB/s while every CU loads,
+  // so the 128 KiB of summaries of a 510-candidate pair take it ~6 us, against
+  // ~5 us for a scoring kernel that spreads them over every CU.  Not measured
+  // since the merge and the selection per wave (which holds as many).
   if (p.S > 1 && max_nc > 256) return false;
   if (p.R > kMaxRounds) return false;
   // every candidate fits the workgroup selection's keys

@@ -159,7 +159,7 @@ __device__ __forceinline__ void put_token(const Geometry& g, int page, int h, in
 
 // dims 8c .. 8c+7 of a full block's summary: the mean of its tb keys (held in
 // LDS as blk[token][c]), summed in token order, each add and the final scale
-// rounded once in fp32 (the order summary16 follows)
+// rounded once in fp32 (the order k_append_blocks' fold follows)
 template <int DT>
 __device__ __forceinline__ u32x4 fold_block(const u32x4 (*blk)[16], int tb, int c) {
   float acc[8];
@@ -1351,7 +1351,8 @@ __device__ __forceinline__ void attend_merge(const Geometry& geo, const SeqBatch
 // It takes the launch 0.5-1.2 us where the combine kernel takes 3.9: per step
 // of the fused decode, fp16, 32 query and 8 kv heads (kernel times): one
 // sequence of 4k tokens 14.6 -> 12.0 us, 4 of 8k 18.1 -> 14.8, 8 of 16k
-// 24.2 -> 20.5, 16 of 16k (256 workgroups) 35.5 -> 32.2.
+// 24.2 -> 20.5, 16 of 16k (256 workgroups) 35.5 -> 32.2.  (With several
+// rounds of workgroups it loses: decode_impl.)
 // No workgroup waits for another.  Each thread's partials have reached device
 // scope (THROUGH stores, waited for) before its workgroup counts itself in;
 // the last one's loads are issued after its count returns and are
