@@ -111,7 +111,7 @@ struct Staged<0, F> {
 // (16 KiB a wave and unit) and the VALU work of a wave's softmax between its
 // MFMAs (16 x 32 cycles a wave and unit, two waves per SIMD): ~70 VALU a unit
 // and 16 exp2, 20 more for bf16 V.  Four waves of 64 columns, which halve the
-// LDS reads and leave one wave per SIMD, take 2575 us where this takes 2198.
+// LDS reads and leave one wave per SIMD, took 2575 us where this took 2198.
 //
 // V of a bf16 cache is converted to fp16 on its way to LDS (exact for
 // |v| < 65520 down to the fp16 normal range) for an fp16 PV product without
@@ -136,10 +136,12 @@ struct Staged<0, F> {
 // or the compiler keeps them in vector registers and 64-bit vector products
 // at every unit.
 // Measured, 512-token chunks at 32k tokens, Hq 32, Hkv 8, with vector counters
-// and a barrier at every unit -> now: 8 sequences, bf16 2388 -> 2198 us (993
-// TFLOP/s), int4 2494 -> 2373 us; one sequence, split in 4, 362 -> 296 us; a
-// prompt of 8191 fp16 tokens 575 -> 581 us (16x16x32 MFMAs in 4-wave
-// workgroups, one unit ahead: 2839, 3000, 1125 and 687 us).
+// and a barrier at every unit -> with scalar ones and a barrier at every
+// second unit -> now (no flags in the loop, nothing spilled): 8 sequences,
+// bf16 2388 -> 2215 -> 2133 us (1022 TFLOP/s), int4 2494 -> 2391 -> 2373 us;
+// one sequence, split in 4, 362 -> 297 -> 283 us; a prompt of 8191 fp16 tokens
+// 575 -> 585 -> 562 us (16x16x32 MFMAs in 4-wave workgroups, one unit ahead:
+// 2838, 2985, 1124 and 685 us).
 // grid (ceil(L / (32 W / G)) * Hkv * n * nsplit), W = 8 or 4 waves
 // ---------------------------------------------------------------------------
 template <int DT, int KB, int W>
